@@ -105,7 +105,38 @@ struct LeafDesc {
 struct EpiDesc {
   uint64_t root;   // device address of the root scalar, 0: empty slice
   int32_t rbits;   // r as the dtype's bit pattern
-  int32_t pad_;
+  int32_t res;     // index of the result
+};
+
+// A fused subtree ("unit"): every step of a maximal subtree whose tensors all
+// fit in LDS, contracted by one workgroup; only the subtree's root goes to
+// memory.  Inside a unit every tensor holds its labels in one global order
+// (elimination time, latest first), so a step's union index -- the output's
+// bits, then the reduced labels' -- maps to an operand's by keeping the
+// operand's bits (mA / mB), and a step is 16 bytes.
+constexpr int kUnitWaves = 4;      // waves of a unit's workgroup
+constexpr int kUnitLds = 8192;     // LDS elements of a unit
+constexpr int kUnitBits = 15;      // union labels of a unit's step
+constexpr int kUnitRank = 14;      // output labels of a unit's step
+constexpr int kUnitReduce = 6;     // reduced labels of a unit's step
+// One wave's share of one step: chunks c0 .. c0+nc-1 of 64 outputs.
+struct UnitItem {
+  uint16_t mA, mB;      // union bits held by A / B
+  uint16_t oA, oB, oC;  // LDS element offsets
+  uint16_t c0, nc;      // nc = 0: nothing to do
+  uint16_t f;           // output bits | reduced bits << 4 | flags
+};
+constexpr int kItemBarrier = 1 << 8;  // the last item of a level (in every wave)
+constexpr int kItemRoot = 1 << 9;     // the unit's output: to memory
+struct UnitDesc {
+  uint64_t c;        // device address of the output, 0: the slice's root scalar
+  uint32_t item0;    // first item; wave w's are item0 + w rounds + 0 .. rounds-1
+  uint32_t w0;       // first vertex weight
+  int32_t rounds;    // items per wave; 0: a leaf tensor (nvert 1: vertex, 0: edge)
+  int32_t nvert;     // vertex leaves, [0, w] at LDS 4 + 2 i (the edge tensor is at 0)
+  int32_t res;       // c == 0: index of the slice's result
+  int32_t rbits;     // ... and its r
+  uint64_t pos;      // nibble k: the C position of output bit k
 };
 
 }  // namespace tbh

@@ -15,12 +15,14 @@
 //                         are staged HBM -> LDS by DMA.
 //      tbh_ew_direct_kernel  the same for small steps without LDS (wave tiles
 //                         reading straight from memory).
-//   K3 tbh_leaf_kernel    leaf tensors of the MIS network from weights.
+//   K3 tbh_leaf_kernel    leaf tensors of the MIS network from weights (PLAIN;
+//                         BATCHED leaves and small subtrees: tbh_unit.hip).
 //   K5 tbh_epi_kernel     per-slice root + r.
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
 
+#include "tbh_device.hpp"
 #include "tbh_internal.hpp"
 
 // minimum waves per SIMD the EW kernels are register-limited to
@@ -80,11 +82,6 @@ struct KAcc<KEwS> {
   using type = KI8S;
 };
 #define TBH_KF(d, f) (typename KAcc<decltype(d)>::type{(d), (uint32_t)offsetof(EwDesc, f)})
-// Tensors are addressed in the global address space: their loads are
-// global_load (counted by vmcnt only), not flat loads, which also count in
-// lgkmcnt and so would make every wait for an LDS or scalar access wait for
-// the data loads in flight too.
-#define TBH_GLOBAL __attribute__((address_space(1)))
 #define TBH_LDS __attribute__((address_space(3)))
 // Sub-tensors are staged with global_load_lds_dword (HBM -> LDS without a
 // register round trip, so every load of a sub-tensor is in flight at once);
@@ -106,50 +103,6 @@ struct KAcc<KEwS> {
 #if TBH_LDS_DMA && TBH_LDS_PAD_SHIFT && TBH_LDS_PAD_SHIFT < 6
 #error "LDS DMA writes 64 consecutive entries per wave: pad at most once per 64"
 #endif
-
-template <typename T>
-struct Trop;
-template <>
-struct Trop<float> {
-  static __device__ __forceinline__ float zero() { return -__builtin_inff(); }
-  static __device__ __forceinline__ float one() { return 0.0f; }
-  static __device__ __forceinline__ float mul(float a, float b) { return a + b; }
-  static __device__ __forceinline__ float add(float a, float b) { return __builtin_fmaxf(a, b); }
-  static __device__ __forceinline__ float canon(float x) { return x; }
-};
-template <>
-struct Trop<int32_t> {
-  // accumulator start; sums of canonical values are >= -2^31
-  static __device__ __forceinline__ int32_t zero() { return INT32_MIN; }
-  static __device__ __forceinline__ int32_t one() { return 0; }
-  static __device__ __forceinline__ int32_t mul(int32_t a, int32_t b) {
-    return (int32_t)((uint32_t)a + (uint32_t)b);
-  }
-  static __device__ __forceinline__ int32_t add(int32_t a, int32_t b) { return a > b ? a : b; }
-  static __device__ __forceinline__ int32_t canon(int32_t x) {
-    return x < kI32NegThresh ? kI32NegInf : x;
-  }
-};
-// max(a, b, c) as one v_max3 (the compiler forms it for only part of the
-// GEMM's reductions).  Register operands only; inputs are never NaN.
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-__device__ __forceinline__ int32_t max3(int32_t a, int32_t b, int32_t c) {
-  int32_t r;
-  asm("v_max3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-
-// zero used to pad GEMM operands (adds without overflow for Int32)
-template <typename T>
-__device__ __forceinline__ T pad_zero();
-template <>
-__device__ __forceinline__ float pad_zero<float>() { return -__builtin_inff(); }
-template <>
-__device__ __forceinline__ int32_t pad_zero<int32_t>() { return kI32NegInf; }
 
 // ---------------------------------------------------------------- K2 -----
 // The 4 high bits (8..11) of a per-thread index: strides of those bits, and
@@ -1505,11 +1458,11 @@ __global__ void tbh_epi_kernel(const EpiDesc* __restrict__ e, int64_t n, T* __re
   T r;
   __builtin_memcpy(&r, &E.rbits, sizeof(T));
   if (!E.root) {
-    out[i] = r;
+    out[E.res] = r;
     return;
   }
   const T v = *reinterpret_cast<const T*>(E.root);
-  out[i] = Trop<T>::canon(Trop<T>::mul(v, r));
+  out[E.res] = Trop<T>::canon(Trop<T>::mul(v, r));
 }
 
 // -------------------------------------------------------- launchers -----

@@ -67,10 +67,13 @@ int validate(const SliceIn& s, std::string* err) {
   return 0;
 }
 
-// labels of leaves then internal nodes, each in first-appearance order
-void compute_labels(const SliceIn& s, std::vector<std::vector<int32_t>>& lab) {
+// labels of leaves then internal nodes, each in first-appearance order;
+// uni[j]: labels of internal node j's two children together
+void compute_labels(const SliceIn& s, std::vector<std::vector<int32_t>>& lab,
+                    std::vector<int32_t>* uni = nullptr) {
   int32_t nl = s.nleaves, nn = std::max(0, nl - 1);
   lab.assign(nl + nn, {});
+  if (uni) uni->assign(nn, 0);
   std::vector<std::vector<int32_t>> cnt(nl + nn);
   std::vector<int32_t> total(std::max(1, s.nv), 0), acc(std::max(1, s.nv), 0);
   for (int32_t i = 0; i < nl; i++)
@@ -87,6 +90,7 @@ void compute_labels(const SliceIn& s, std::vector<std::vector<int32_t>>& lab) {
       for (size_t k = 0; k < lab[c].size(); k++) {
         int32_t l = lab[c][k];
         if (acc[l] > 0) {
+          if (uni) (*uni)[j]++;
           if (acc[l] < total[l]) {
             lab[o].push_back(l);
             cnt[o].push_back(acc[l]);
@@ -469,9 +473,13 @@ int64_t assign_offsets(std::vector<PTensor>& T) {
   int64_t top = 0;
   size_t di = 0;
   for (int t : idx) {
+    if (T[t].bytes == 0) {  // lives in LDS
+      T[t].off = 0;
+      continue;
+    }
     while (di < by_death.size() && T[by_death[di]].death < T[t].birth) {
       const PTensor& d = T[by_death[di]];
-      if (d.off >= 0) freel[std::max<int64_t>(d.bytes, 16)].push_back(d.off);
+      if (d.off >= 0 && d.bytes > 0) freel[std::max<int64_t>(d.bytes, 16)].push_back(d.off);
       di++;
     }
     int64_t cls = std::max<int64_t>(T[t].bytes, 16);
@@ -725,6 +733,279 @@ void reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree,
   tree.swap(out);
 }
 
+// ---- units: subtrees contracted in LDS (UnitDesc) -----------------------
+// A node joins a unit when its children do (or are leaves) and its step, the
+// unit's work and its LDS tensors stay within the limits; the unit is the
+// largest such subtree.  About 93% of the nodes of the sliced 3-regular and
+// King's-subgraph trees are in one of a slice's 15-40 units.
+struct UnitBuilder {
+  const SliceIn& s;
+  const std::vector<std::vector<int32_t>>& lab;
+  const std::vector<int32_t>& uni;
+  const std::vector<int32_t>& prio;  // label -> place in the order of all labels
+  SlicePlan& P;
+  int32_t nl;
+  // log2 of a unit's MACs at most: 4 waves take about 5 us for 2^17
+  static constexpr double kUnitMacs = 131072.0;
+  std::vector<char> in_unit;         // tree node (leaf or internal) inside a unit
+  std::vector<char> fit;             // internal node may be inside a unit
+  std::vector<int32_t> parent, level, node_at, vert;
+  std::vector<int32_t> off;          // LDS offset of a unit's tensor
+  std::vector<std::vector<int32_t>> sorted;  // labels of a unit's tensors, by prio
+
+  UnitBuilder(const SliceIn& s_, const std::vector<std::vector<int32_t>>& lab_,
+              const std::vector<int32_t>& uni_, const std::vector<int32_t>& prio_, SlicePlan& P_)
+      : s(s_), lab(lab_), uni(uni_), prio(prio_), P(P_), nl(s_.nleaves) {}
+
+  int rank(int32_t x) const { return (int)lab[x].size(); }
+
+  // which internal nodes may be inside a unit
+  void mark() {
+    const int32_t nn = nl - 1, tot = nl + nn;
+    in_unit.assign(tot, 0);
+    fit.assign(tot, 0);
+    parent.assign(tot, -1);
+    level.assign(tot, 0);
+    off.assign(tot, 0);
+    vert.assign(nl, -1);
+    sorted.resize(tot);
+    std::vector<int64_t> peak(tot, 0);
+    std::vector<double> macs(tot, 0.0);
+    for (int32_t i = 0; i < nl; i++) fit[i] = 1;
+    for (int32_t j = 0; j < nn; j++) {
+      const int32_t o = nl + j, x = s.tree[2 * j], y = s.tree[2 * j + 1];
+      parent[x] = parent[y] = o;
+      // live LDS elements, the child with the larger peak first (leaves are
+      // outside this count)
+      const int64_t sx = x < nl ? 0 : (int64_t)1 << std::min(rank(x), 30);
+      const int64_t sy = y < nl ? 0 : (int64_t)1 << std::min(rank(y), 30);
+      const int64_t so = (int64_t)1 << std::min(rank(o), 30);
+      const int64_t first = std::max(peak[x], peak[y]);
+      const int64_t second = peak[x] >= peak[y] ? sx + peak[y] : sy + peak[x];
+      peak[o] = std::max(std::max(first, second), sx + sy + so);
+      macs[o] = macs[x] + macs[y] + std::ldexp(1.0, uni[j]);
+      fit[o] = fit[x] && fit[y] && uni[j] <= kUnitBits && rank(o) <= kUnitRank && uni[j] - rank(o) <= kUnitReduce &&
+               macs[o] <= kUnitMacs && std::max(first, second) <= kUnitLds;
+    }
+  }
+
+  // Plans the unit of root `root`, or returns false when its tensors do not
+  // fit the LDS (levels keep more tensors alive than the estimate of mark()).
+  bool build(int32_t root) {
+    // nodes of the subtree, parents before children; a level is the distance
+    // from the deepest node (children run one level before their parent)
+    node_at.clear();
+    node_at.push_back(root);
+    level[root] = 0;
+    int depth = 0, nvert = 0;
+    std::vector<int32_t> verts;
+    for (size_t k = 0; k < node_at.size(); k++) {
+      const int32_t o = node_at[k], j = o - nl;
+      for (int q = 0; q < 2; q++) {
+        const int32_t c = s.tree[2 * j + q];
+        if (c < nl) {
+          if (rank(c) == 1) {
+            vert[c] = nvert++;
+            verts.push_back(c);
+          }
+          continue;
+        }
+        level[c] = level[o] + 1;
+        depth = std::max(depth, level[c]);
+        node_at.push_back(c);
+      }
+    }
+    // breadth first: node_at is in descending level order from the back
+    // LDS: the edge tensor, the vertex tensors, then the internal tensors,
+    // blocks of a level's dead operands reused one level later
+    int top = 4 + 2 * nvert;
+    std::vector<int32_t> freeb[kUnitBits + 1];
+    size_t dead = node_at.size();  // node_at[dead..]: tensors already released
+    for (size_t k = node_at.size(); k-- > 1;) {
+      const int32_t o = node_at[k];
+      // tensors of levels >= level[o] + 2 were read a level before o's
+      while (dead > 0 && level[node_at[dead - 1]] >= level[o] + 2) {
+        dead--;
+        freeb[rank(node_at[dead])].push_back(off[node_at[dead]]);
+      }
+      const int r = rank(o);
+      int c = r;
+      while (c <= kUnitBits && freeb[c].empty()) c++;
+      if (c <= kUnitBits) {
+        const int32_t at = freeb[c].back();
+        freeb[c].pop_back();
+        for (int b = r; b < c; b++) freeb[b].push_back(at + (1 << b));  // the rest of the block
+        off[o] = at;
+      } else {
+        off[o] = top;
+        top += 1 << r;
+        if (top > kUnitLds) return false;
+      }
+    }
+    // steps, deepest level first: the union's labels by merging the
+    // operands' (each in prio order); the output keeps its first ones
+    PUnit u;
+    u.tensor = root;
+    u.nvert = nvert;
+    u.item0 = (uint32_t)P.items.size();
+    u.w0 = (uint32_t)P.unit_w.size();
+    for (int32_t c : verts) {
+      const int32_t v = lab[c][0];
+      P.unit_w.push_back(s.wbits ? s.wbits[v] : s.unit_wbits);
+    }
+    std::vector<UnitItem> wave[kUnitWaves];
+    int next = 0;
+    size_t k = node_at.size();
+    while (k > 0) {
+      const int lv = level[node_at[k - 1]];
+      for (; k > 0 && level[node_at[k - 1]] == lv; k--) {
+        const int32_t o = node_at[k - 1], j = o - nl;
+        const int32_t x = s.tree[2 * j], y = s.tree[2 * j + 1];
+        for (int32_t c : {x, y})
+          if (c < nl) {
+            sorted[c] = lab[c];
+            if (sorted[c].size() == 2 && prio[sorted[c][0]] > prio[sorted[c][1]])
+              std::swap(sorted[c][0], sorted[c][1]);
+          }
+        const auto &LX = sorted[x], &LY = sorted[y];
+        auto& LO = sorted[o];
+        LO.clear();
+        UnitItem it{};
+        int n = 0;
+        for (size_t a = 0, b = 0; a < LX.size() || b < LY.size(); n++) {
+          const int pa = a < LX.size() ? prio[LX[a]] : INT32_MAX;
+          const int pb = b < LY.size() ? prio[LY[b]] : INT32_MAX;
+          LO.push_back(pa <= pb ? LX[a] : LY[b]);
+          if (pa <= pb) it.mA |= (uint16_t)(1u << n), a++;
+          if (pb <= pa) it.mB |= (uint16_t)(1u << n), b++;
+        }
+        const int nP = rank(o), nR = n - nP;
+        LO.resize(nP);
+        auto lds_of = [&](int32_t c) {
+          return c >= nl ? off[c] : vert[c] >= 0 && rank(c) == 1 ? 4 + 2 * vert[c] : 0;
+        };
+        it.oA = (uint16_t)lds_of(x);
+        it.oB = (uint16_t)lds_of(y);
+        it.oC = (uint16_t)(o == root ? 0 : off[o]);
+        it.f = (uint16_t)(nP | nR << 4 | (o == root ? kItemRoot : 0));
+        // the step's chunks in up to kUnitWaves equal runs
+        const int chunks = nP > 6 ? 1 << (nP - 6) : 1;
+        const int runs = std::min(chunks, kUnitWaves);
+        for (int q = 0; q < runs; q++) {
+          it.c0 = (uint16_t)(chunks / runs * q);
+          it.nc = (uint16_t)(chunks / runs);
+          wave[next].push_back(it);
+          next = (next + 1) % kUnitWaves;
+        }
+        P.unit_steps.push_back({(int8_t)rank(x), (int8_t)rank(y), (int8_t)nP, (int8_t)nR});
+        P.exec_macs += std::ldexp(1.0, n);
+      }
+      // every wave ends the level in the same round
+      size_t rounds = 0;
+      for (auto& w : wave) rounds = std::max(rounds, w.size());
+      for (auto& w : wave) {
+        w.resize(rounds, UnitItem{});
+        w.back().f |= kItemBarrier;
+      }
+    }
+    u.rounds = (int)wave[0].size();
+    for (auto& w : wave) P.items.insert(P.items.end(), w.begin(), w.end());
+    P.units.push_back(u);
+    P.unit_levels = std::max(P.unit_levels, depth + 1);
+    for (int32_t o : node_at) {
+      in_unit[o] = 1;
+      for (int q = 0; q < 2; q++) in_unit[s.tree[2 * (o - nl) + q]] = 1;
+    }
+    return true;
+  }
+
+  // Units of the whole tree, then a leaf unit for every leaf outside them.
+  // in_unit afterwards: 1 inside a unit, 2 a unit's (or leaf's) output.
+  void run() {
+    const int32_t nn = nl - 1;
+    mark();
+    std::vector<int32_t> roots;
+    for (int32_t o = nl + nn - 1; o >= nl; o--)
+      if (fit[o] && (parent[o] < 0 || !fit[parent[o]])) roots.push_back(o);
+    while (!roots.empty()) {
+      const int32_t o = roots.back();
+      roots.pop_back();
+      if (build(o)) {
+        in_unit[o] = 2;
+        continue;
+      }
+      for (int q = 0; q < 2; q++) {
+        const int32_t c = s.tree[2 * (o - nl) + q];
+        if (c >= nl) roots.push_back(c);
+      }
+    }
+    for (int32_t i = 0; i < nl; i++) {
+      if (in_unit[i]) continue;
+      PUnit u;
+      u.tensor = i;
+      u.nvert = rank(i) == 1 ? 1 : 0;
+      u.item0 = (uint32_t)P.items.size();
+      u.w0 = (uint32_t)P.unit_w.size();
+      if (u.nvert) P.unit_w.push_back(s.wbits ? s.wbits[lab[i][0]] : s.unit_wbits);
+      P.units.push_back(u);
+      in_unit[i] = 2;
+    }
+  }
+
+  // output bit -> position in the layout its consumer reads
+  void set_layout(PUnit* u, const std::vector<int32_t>& lay) {
+    if (u->rounds == 0) return;  // a leaf: its content is symmetric
+    const auto& L = sorted[u->tensor];
+    for (size_t k = 0; k < L.size(); k++) u->pos |= (uint64_t)(pos_in(lay, L[k]) & 15) << (4 * k);
+  }
+};
+
+// Every LDS and memory address a unit forms is in range, and its items cover
+// every output of every step.
+int verify_units(const SlicePlan& P, std::string* err) {
+  auto bad = [&](const std::string& m) { return fail(err, "plan check: unit " + m); };
+  for (const PUnit& u : P.units) {
+    if (u.tensor < 0 || u.tensor >= (int)P.tensors.size()) return bad("output");
+    if (u.w0 + (size_t)u.nvert > P.unit_w.size() || 4 + 2 * u.nvert > kUnitLds)
+      return bad("weights");
+    const int rank = P.tensors[u.tensor].rank;
+    if (u.rounds == 0) {
+      if (rank != (u.nvert ? 1 : 2)) return bad("leaf");
+      continue;
+    }
+    if (u.item0 + (size_t)u.rounds * kUnitWaves > P.items.size()) return bad("items");
+    uint32_t used = 0;
+    for (int k = 0; k < rank; k++) {
+      const int p = (int)(u.pos >> (4 * k)) & 15;
+      if (p >= rank || ((used >> p) & 1)) return bad("layout");
+      used |= 1u << p;
+    }
+    int64_t root_chunks = 0;
+    for (int r = 0; r < u.rounds; r++)
+      for (int w = 0; w < kUnitWaves; w++) {
+        const UnitItem& it = P.items[u.item0 + (size_t)w * u.rounds + r];
+        if ((it.f ^ P.items[u.item0 + r].f) & kItemBarrier) return bad("levels");
+        if (r == u.rounds - 1 && !(it.f & kItemBarrier)) return bad("last level");
+        if (!it.nc) continue;
+        const int nP = it.f & 15, nR = (it.f >> 4) & 15, n = nP + nR;
+        const int chunks = nP > 6 ? 1 << (nP - 6) : 1;
+        if (n > kUnitBits || nR > kUnitReduce || it.c0 + it.nc > chunks || it.nc > 64 ||
+            (uint32_t)(it.mA | it.mB) != (1u << n) - 1 ||
+            it.oA + (1 << __builtin_popcount(it.mA)) > kUnitLds ||
+            it.oB + (1 << __builtin_popcount(it.mB)) > kUnitLds)
+          return bad("step");
+        if (it.f & kItemRoot) {
+          if (nP != rank) return bad("root");
+          root_chunks += it.nc;
+        } else if (it.oC < 4 + 2 * u.nvert || it.oC + (1 << nP) > kUnitLds) {
+          return bad("tensor");
+        }
+      }
+    if (root_chunks != (rank > 6 ? 1 << (rank - 6) : 1)) return bad("root cover");
+  }
+  return 0;
+}
+
 }  // namespace
 
 int slice_labels(const SliceIn& s, std::vector<std::vector<int32_t>>* labels, std::string* err) {
@@ -807,22 +1088,18 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   P.empty = false;
   SliceIn s = s_in;
   const int32_t nl = s.nleaves, nn = nl - 1;
+  P.n_leaves = nl;
   std::vector<std::vector<int32_t>> lab;
-  compute_labels(s, lab);
+  std::vector<int32_t> uni;
+  compute_labels(s, lab, &uni);
   // tree-node contraction count of the given tree (the reference's tc)
-  for (int32_t j = 0; j < nn; j++) {
-    const auto &A = lab[s.tree[2 * j]], &Bv = lab[s.tree[2 * j + 1]];
-    int u = (int)A.size();
-    for (int32_t l : Bv)
-      if (pos_in(A, l) < 0) u++;
-    P.node_macs += std::ldexp(1.0, u);
-  }
+  for (int32_t j = 0; j < nn; j++) P.node_macs += std::ldexp(1.0, uni[j]);
   std::vector<int32_t> tree2;
   if (opt.batched && opt.reassociate && nn >= 3 && !std::getenv("TBH_NO_REASSOCIATE")) {
     tree2.assign(s.tree, s.tree + 2 * (size_t)nn);
     reassociate(nl, s.nv, tree2, lab, opt);
     s.tree = tree2.data();
-    compute_labels(s, lab);
+    compute_labels(s, lab, &uni);
   }
 
   // elimination step of each label (node index where it disappears)
@@ -848,9 +1125,28 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   P.ops.reserve(3 * (size_t)nn + 4);
   P.tensors.reserve(3 * (size_t)(nl + nn) + 4);
   B.layout.reserve(3 * (size_t)(nl + nn) + 4);
+  // batched: the subtrees that run as units; a single leaf, and every leaf
+  // and step outside them, as below
+  std::vector<int32_t> prio;
+  const bool units = opt.batched && opt.units;
+  if (units) {
+    std::vector<int32_t> all(s.nv);
+    std::iota(all.begin(), all.end(), 0);
+    all = sorted_key(all);
+    prio.resize(s.nv);
+    for (int32_t k = 0; k < s.nv; k++) prio[all[k]] = k;
+  }
+  UnitBuilder U(s, lab, uni, prio, P);
+  if (units) U.run();
+  auto inside = [&](int32_t x) { return units && U.in_unit[x] == 1; };
   // leaves are tensors 0..nl-1 (content is symmetric, so any layout works)
   for (int32_t i = 0; i < nl; i++) {
+    if (inside(i)) {
+      B.add_tensor({});
+      continue;
+    }
     B.add_tensor(opt.batched ? sorted_key(lab[i]) : lab[i]);
+    if (units) continue;
     PLeaf L;
     L.tensor = i;
     L.kind = (int)lab[i].size();
@@ -862,7 +1158,8 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     P.leaves.push_back(L);
   }
   // internal node output tensors nl..nl+nn-1 (layouts fixed below)
-  for (int32_t j = 0; j < nn; j++) B.add_tensor(lab[nl + j]);
+  for (int32_t j = 0; j < nn; j++)
+    B.add_tensor(inside(nl + j) ? std::vector<int32_t>() : lab[nl + j]);
 
   // classify labels of node j
   struct Cls {
@@ -925,9 +1222,14 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     std::vector<std::vector<int32_t>> gemm_out(nn);
     std::vector<int> split(nn, 0);
     for (int32_t j = nn - 1; j >= 0; j--) {
+      const int o = nl + j;
+      if (inside(o)) continue;
+      if (units && U.in_unit[o]) {
+        B.layout[o] = has_req[o] ? req[o] : sorted_key(lab[o]);
+        continue;
+      }
       cls[j] = classify(j);
       Cls& c = cls[j];
-      const int o = nl + j;
       int na = (int)c.a.size(), nb = (int)c.b.size(), nk = (int)c.k.size();
       bool g = !c.priv && gemm_shaped(opt, na, nb, nk);
       is_gemm[j] = g;
@@ -964,8 +1266,10 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     for (int32_t i = 0; i < nl; i++)
       if (has_req[i]) B.layout[i] = req[i];
     // emit steps in post-order
+    for (PUnit& u : P.units) U.set_layout(&u, B.layout[u.tensor]);
     for (int32_t j = 0; j < nn; j++) {
       const int o = nl + j;
+      if (units && U.in_unit[o]) continue;
       Cls& c = cls[j];
       if (is_gemm[j]) {
         int dst = o;
@@ -1049,6 +1353,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   }
   if (P.tensors[P.root].rank != 0) return fail(err, "root tensor is not a scalar");
 
+  P.unit_root = units && nn > 0 && U.in_unit[P.root] != 0;
   // producers and levels
   const int nt = (int)P.tensors.size();
   std::vector<int> producer(nt, -1), consumer(nt, -1);
@@ -1087,8 +1392,20 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     }
   }
   for (auto& t : P.tensors) t.off = -1;
+  if (units) {
+    // the arena holds no tensor from inside a unit, and no root a unit
+    // writes as the slice's result
+    for (int32_t x = 0; x < nl + nn; x++)
+      if (U.in_unit[x] == 1 || (P.unit_root && x == P.root)) P.tensors[x].bytes = 0;
+  }
   P.arena_bytes = assign_offsets(P.tensors);
-  if (verify_plan(P, err)) return -1;
+  // never below the largest tensor of the tree, in LDS or not: callers size
+  // pools by it (at most 2^(kUnitBits + 2) bytes more)
+  for (int32_t j = 0; units && j < nn; j++)
+    if (U.in_unit[nl + j])
+      P.arena_bytes = std::max<int64_t>(P.arena_bytes, (int64_t)4 << lab[nl + j].size());
+  P.arena_bytes = (P.arena_bytes + 255) / 256 * 256;
+  if (verify_plan(P, err) || verify_units(P, err)) return -1;
   for (const auto& op : P.ops) {
     P.exec_macs += op.macs;
     P.exec_bytes += op.bytes;

@@ -58,11 +58,32 @@ struct PLeaf {
   uint32_t wbits;
 };
 
+// A fused subtree (UnitDesc without addresses).
+struct PUnit {
+  int tensor = -1;        // output; kind and weight of a leaf as in UnitDesc
+  uint32_t item0 = 0, w0 = 0;  // into SlicePlan::items / unit_w
+  int rounds = 0, nvert = 0;
+  uint64_t pos = 0;
+};
+
+// A step inside a unit (plan_steps, work accounting).
+struct PUnitStep {
+  int8_t rank_a, rank_b, rank_c, n_reduced;
+};
+
 struct SlicePlan {
   bool empty = true;     // no leaves: the contraction is the tropical one
   std::vector<PTensor> tensors;
   std::vector<POp> ops;  // in dependency order
-  std::vector<PLeaf> leaves;
+  std::vector<PLeaf> leaves;  // plain plans only; batched: leaf units
+  // batched: the subtrees contracted in LDS, before level 1
+  std::vector<PUnit> units;
+  std::vector<UnitItem> items;
+  std::vector<uint32_t> unit_w;  // vertex weights of the units
+  std::vector<PUnitStep> unit_steps;
+  int n_leaves = 0;
+  bool unit_root = false;  // the root is a unit: the unit writes the result
+  int unit_levels = 0;     // deepest unit
   int root = -1;         // tensor holding the scalar result
   int nlevels = 0;       // ops use levels 1..nlevels
   int64_t arena_bytes = 0;
@@ -104,6 +125,8 @@ struct PlanOptions {
   // GEMM tile rule (gemm_shape): 0 128 x 128 only, 1 tall-skinny tiles for
   // N <= 64, 2 also 256 x 64 up to N = 128
   int gemm_tiles = 1;
+  // subtrees whose tensors fit in LDS run as units (batched only)
+  bool units = true;
   // tiled EW steps: outer labels absent from the larger sub-tensor first,
   // so that consecutive tiles reuse it from LDS; false: C's label order
   bool reuse_order = true;

@@ -627,17 +627,23 @@ int stat_kind(int kind) { return kind < 2 ? kind : 2; }  // tbh_stats: direct, t
 
 }  // namespace
 
+// algorithmic bytes of a step inside a unit: |A| + |B| + |C| entries x 4
+double unit_step_bytes(const PUnitStep& s) {
+  return 4.0 * (std::ldexp(1.0, s.rank_a) + std::ldexp(1.0, s.rank_b) + std::ldexp(1.0, s.rank_c));
+}
+
 size_t desc_bytes(const SlicePlan& P) {
   if (P.empty) return sizeof(EpiDesc) + 4;
   // a step: its descriptor, its prefix entry and (per-step profiling) its
   // one-step prefix pair
   return P.ops.size() * (std::max(sizeof(EwDesc), sizeof(GemmDesc)) + 3 * sizeof(int64_t)) +
-         P.leaves.size() * sizeof(LeafDesc) + sizeof(EpiDesc) + 4;
+         P.units.size() * sizeof(UnitDesc) + P.items.size() * sizeof(UnitItem) +
+         P.unit_w.size() * sizeof(uint32_t) + sizeof(EpiDesc) + 4;
 }
 
 size_t desc_batch_overhead(int levels) {
   const size_t slots = (size_t)kKinds * (size_t)(levels + 1);
-  return 256 * (3 + 3 * slots) + sizeof(int64_t) * slots;
+  return 256 * (5 + 3 * slots) + sizeof(int64_t) * slots;
 }
 
 namespace {
@@ -768,8 +774,9 @@ struct IssueJob {
   bool prof = false, per_step = false;
   int bidx = 0, H = 0;
   size_t nb = 0;
-  int64_t nleaves = 0;
-  size_t o_leaves = 0, o_epi = 0, o_res = 0;
+  int64_t nunits = 0, nepi = 0;
+  int unit_levels = 0;   // deepest unit
+  size_t o_units = 0, o_items = 0, o_w = 0, o_epi = 0, o_res = 0;
   char* dbase = nullptr;     // the batch's descriptors on the device
   const char* hb = nullptr;  // ... and in the pinned staging buffer (step tags)
   hipEvent_t up = nullptr, done = nullptr;
@@ -793,17 +800,25 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
   char* dbase = j.dbase;
   // a launch failure forced from the host (error-path tests), checked
   // before every launch of the batch; nothing is launched in its place
-  auto injected = [ctx] {
+  // (the units' launch counts as many as the levels it runs)
+  auto injected = [ctx](int64_t n = 1) {
     int64_t v = ctx->inject_launch_failure.load();
     while (v >= 0)
-      if (ctx->inject_launch_failure.compare_exchange_weak(v, v - 1)) return v == 0;
+      if (ctx->inject_launch_failure.compare_exchange_weak(v, std::max<int64_t>(-1, v - n)))
+        return v < n;
     return false;
   };
   if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, j.up, 0);
-  if (e == hipSuccess && j.nleaves && injected()) e = hipErrorLaunchFailure;
-  if (e == hipSuccess)
-    e = launch_leaves(dtype, (const LeafDesc*)(dbase + j.o_leaves), j.nleaves, ctx->stream);
-  ctx->stats.launches += j.nleaves ? 1 : 0;
+  if (e == hipSuccess && j.nunits && injected(std::max(1, j.unit_levels)))
+    e = hipErrorLaunchFailure;
+  if (e == hipSuccess && j.nunits) {
+    hipEvent_t ev = prof ? ctx->prof.begin(ctx->stream) : nullptr;
+    e = launch_units(dtype, (const UnitDesc*)(dbase + j.o_units),
+                     (const UnitItem*)(dbase + j.o_items), (const uint32_t*)(dbase + j.o_w),
+                     j.nunits, dbase + j.o_res, ctx->stream);
+    if (prof) ctx->prof.end(ctx->stream, ev, 0, 0, (int)j.nunits, 0, 0, "units");
+    ctx->stats.launches++;
+  }
   hipEvent_t ev = nullptr;
   // one launch per kernel kind and level (direct EW, tiled EW, GEMM); in
   // the per-step profiling mode every step alone, tagged with its shape
@@ -817,7 +832,7 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
   auto& evpool = ctx->lvl_events[j.bidx & 1];
   size_t evn = 0;
   // dirty[s]: stream s launched work the other stream has not waited for
-  // (the upload wait and the leaves are stream-0 work)
+  // (the upload wait and the units are stream-0 work)
   bool dirty[2] = {true, false};
   auto sync_to = [&](int s) {  // stream s waits for the other stream's work so far
     const int o = 1 - s;
@@ -895,10 +910,11 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
     ctx->stats.waves++;
   }
   if (e == hipSuccess && conc) e = sync_to(0);  // the last GEMMs before the epilogue
-  if (e == hipSuccess && injected()) e = hipErrorLaunchFailure;
-  if (e == hipSuccess) {
-    e = launch_epilogue(dtype, (const EpiDesc*)(dbase + j.o_epi), (int64_t)j.nb, dbase + j.o_res,
-                        ctx->stream);
+  if (e == hipSuccess && j.nepi) {
+    if (injected()) e = hipErrorLaunchFailure;
+    if (e == hipSuccess)
+      e = launch_epilogue(dtype, (const EpiDesc*)(dbase + j.o_epi), j.nepi, dbase + j.o_res,
+                          ctx->stream);
     ctx->stats.launches++;
   }
   if (e == hipSuccess)
@@ -1014,12 +1030,24 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   std::vector<std::vector<int64_t>> pfx(W, std::vector<int64_t>(1, 0));
   std::vector<double> lvl_bytes(W, 0.0), lvl_macs(W, 0.0);
   std::vector<std::vector<std::pair<double, double>>> step_work(per_step ? W : 0);
-  std::vector<int64_t> leaf_start(nb + 1, 0);
+  // per slice: its first unit, item, vertex weight and epilogue entry
+  struct Start {
+    int64_t unit = 0, item = 0, w = 0, epi = 0;
+  };
+  std::vector<Start> first(nb + 1);
+  int unit_levels = 0;
   for (size_t i = 0; i < nb; i++) {
     const SlicePlan& P = *plans[i];
     std::memcpy(&start[i * W], cnt.data(), W * sizeof(int32_t));
-    leaf_start[i + 1] = leaf_start[i] + (P.empty ? 0 : (int64_t)P.leaves.size());
+    first[i + 1] = first[i];
+    first[i + 1].epi += P.empty || !P.unit_root;
     if (P.empty) continue;
+    first[i + 1].unit += (int64_t)P.units.size();
+    first[i + 1].item += (int64_t)P.items.size();
+    first[i + 1].w += (int64_t)P.unit_w.size();
+    unit_levels = std::max(unit_levels, P.unit_levels);
+    ctx->stats.ew_ops += P.unit_steps.size();
+    for (const PUnitStep& st : P.unit_steps) ctx->stats.ew_ops_algo_bytes += unit_step_bytes(st);
     for (const POp& op : P.ops) {
       const int w = slot(op_kind(op), op.level);
       cnt[w]++;
@@ -1036,9 +1064,8 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
       }
     }
     ctx->stats.total_algo_ops += 2 * P.node_macs;
-    ctx->stats.leaf_tensors += P.leaves.size();
+    ctx->stats.leaf_tensors += P.n_leaves;
   }
-  const int64_t nleaves = leaf_start[nb];
   // layout of the upload (256-byte aligned arrays)
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -1046,8 +1073,10 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
     off = o + bytes;
     return o;
   };
-  const size_t o_leaves = take((size_t)nleaves * sizeof(LeafDesc));
-  const size_t o_epi = take(nb * sizeof(EpiDesc));
+  const size_t o_units = take((size_t)first[nb].unit * sizeof(UnitDesc));
+  const size_t o_items = take((size_t)first[nb].item * sizeof(UnitItem));
+  const size_t o_w = take((size_t)first[nb].w * sizeof(uint32_t));
+  const size_t o_epi = take((size_t)first[nb].epi * sizeof(EpiDesc));
   const size_t o_res = take(4 * nb);
   std::vector<size_t> o_desc(W), o_pfx(W), o_one(W);
   for (int w = 0; w < W; w++) {
@@ -1079,19 +1108,34 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   parallel_for(nb, ctx->workers, ctx->plan_threads, [&](size_t i, int t) {
     const SlicePlan& P = *plans[i];
     const uint64_t b = sbase[i];
-    EpiDesc e;
-    std::memset(&e, 0, sizeof e);
-    e.rbits = add_r ? slices[i]->rbits : zero_bits;
-    e.root = P.empty ? 0 : b + (uint64_t)P.tensors[P.root].off;
-    std::memcpy(hb + o_epi + i * sizeof(EpiDesc), &e, sizeof e);
-    if (P.empty) return;
-    LeafDesc* ld = reinterpret_cast<LeafDesc*>(hb + o_leaves) + leaf_start[i];
-    for (const PLeaf& L : P.leaves) {
-      ld->p = b + (uint64_t)P.tensors[L.tensor].off;
-      ld->kind = L.kind;
-      ld->wbits = (int32_t)L.wbits;
-      ld++;
+    const uint32_t rbits = add_r ? slices[i]->rbits : zero_bits;
+    if (P.empty || !P.unit_root) {
+      EpiDesc e;
+      e.root = P.empty ? 0 : b + (uint64_t)P.tensors[P.root].off;
+      e.rbits = (int32_t)rbits;
+      e.res = (int32_t)i;
+      std::memcpy(hb + o_epi + (size_t)first[i].epi * sizeof(EpiDesc), &e, sizeof e);
     }
+    if (P.empty) return;
+    UnitDesc* ud = reinterpret_cast<UnitDesc*>(hb + o_units) + first[i].unit;
+    for (const PUnit& u : P.units) {
+      const bool result = P.unit_root && u.tensor == P.root;
+      ud->c = result ? 0 : b + (uint64_t)P.tensors[u.tensor].off;
+      ud->item0 = (uint32_t)first[i].item + u.item0;
+      ud->w0 = (uint32_t)first[i].w + u.w0;
+      ud->rounds = u.rounds;
+      ud->nvert = u.nvert;
+      ud->res = (int32_t)i;
+      ud->rbits = (int32_t)rbits;
+      ud->pos = u.pos;
+      ud++;
+    }
+    if (!P.items.empty())
+      std::memcpy(hb + o_items + (size_t)first[i].item * sizeof(UnitItem), P.items.data(),
+                  P.items.size() * sizeof(UnitItem));
+    if (!P.unit_w.empty())
+      std::memcpy(hb + o_w + (size_t)first[i].w * sizeof(uint32_t), P.unit_w.data(),
+                  P.unit_w.size() * sizeof(uint32_t));
     std::vector<int32_t>& loc = local[t];
     std::fill(loc.begin(), loc.end(), 0);
     const int32_t* st = &start[i * W];
@@ -1144,8 +1188,12 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   job->bidx = bidx;
   job->H = H;
   job->nb = nb;
-  job->nleaves = nleaves;
-  job->o_leaves = o_leaves;
+  job->nunits = first[nb].unit;
+  job->nepi = first[nb].epi;
+  job->unit_levels = unit_levels;
+  job->o_units = o_units;
+  job->o_items = o_items;
+  job->o_w = o_w;
   job->o_epi = o_epi;
   job->o_res = o_res;
   job->dbase = dbase;
@@ -1893,13 +1941,26 @@ int tbh_plan_steps(const tbh_slice* slice, tbh_dtype dtype, tbh_mode mode, tbh_s
     set_error(err);
     return TBH_EINVAL;
   }
-  int n = (int)P.ops.size();
-  for (int i = 0; i < n && i < cap; i++) {
-    const POp& op = P.ops[i];
+  // the units' steps are wave 1, the other steps' waves follow
+  const int nu = (int)P.unit_steps.size(), n = nu + (int)P.ops.size();
+  for (int i = 0; i < nu && i < cap; i++) {
+    const PUnitStep& u = P.unit_steps[i];
+    tbh_step_info& s = out[i];
+    std::memset(&s, 0, sizeof s);
+    s.level = 1;
+    s.rank_a = u.rank_a;
+    s.rank_b = u.rank_b;
+    s.rank_c = u.rank_c;
+    s.n_reduced = u.n_reduced;
+    s.macs = std::ldexp(1.0, u.rank_c + u.n_reduced);
+    s.bytes = unit_step_bytes(u);
+  }
+  for (int i = nu; i < n && i < cap; i++) {
+    const POp& op = P.ops[i - nu];
     tbh_step_info& s = out[i];
     std::memset(&s, 0, sizeof s);
     s.kind = op.kind;
-    s.level = op.level;
+    s.level = op.level + (P.units.empty() ? 0 : 1);
     s.rank_a = P.tensors[op.a].rank;
     s.rank_b = op.b >= 0 ? P.tensors[op.b].rank : -1;
     s.rank_c = P.tensors[op.c].rank;
