@@ -22,7 +22,7 @@ HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-march=x86-64-v3", "-pthread",
               "-Wall", f"-I{INC}"]
 
 TBH_SOURCES = ["tbh_kernels.hip", "tbh_plan.cpp", "tbh_runtime.cpp", "tbh_serve.cpp",
-               "tbh_regions.hip", "tbh_unit.hip"]
+               "tbh_regions.hip", "tbh_unit.hip", "tbh_gemm.hip"]
 
 
 def _run(cmd):

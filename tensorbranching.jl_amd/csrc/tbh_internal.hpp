@@ -94,6 +94,17 @@ struct GemmDesc {
   int32_t ep_n, ep_split;
 };
 
+// One max-plus GEMM in 64 x 64 tiles (K1b, passed by value): ksplit K ranges
+// of kpart (a multiple of 32) per tile, their maxima to ws when ksplit > 1
+// (batch x ksplit x N x M).  M >= 4, K >= 4.
+struct GemmSplit {
+  uint64_t a, b, c, ws;
+  int32_t M, N, K, batch;
+  int64_t lda, ldb, ldc;
+  int64_t sA, sB, sC;
+  int32_t tiles_m, tiles_n, ksplit, kpart;
+};
+
 // Leaf tensor writes (vertex [0,w] or edge [0,0,0,-inf]).
 struct LeafDesc {
   uint64_t p;      // device address

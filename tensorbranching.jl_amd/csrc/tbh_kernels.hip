@@ -1513,62 +1513,28 @@ hipError_t launch_ew_direct(int dtype, const EwDesc* ops, const int64_t* prefix,
   return hipGetLastError();
 }
 
+// The scalar-load kernel (a standalone product of M or K below 4, or of more
+// tiles than K1b indexes) has 128 x 128 tiles only.
+template <typename T>
+static void* gemm_kernel(bool vec, int shape) {
+  if (!vec) return (void*)tbh_gemm_kernel<T, false, 0>;
+  return shape == 1   ? (void*)tbh_gemm_kernel<T, true, 1>
+         : shape == 2 ? (void*)tbh_gemm_kernel<T, true, 2>
+                      : (void*)tbh_gemm_kernel<T, true, 0>;
+}
+
 hipError_t launch_gemm(int dtype, bool vec, int shape, const GemmDesc* ops, const int64_t* prefix,
                        int nops, int64_t total, int grid, hipStream_t s) {
   if (total <= 0) return hipSuccess;
-#define TBH_GEMM_LAUNCH(T, V, S) tbh_gemm_kernel<T, V, S><<<grid, 256, 0, s>>>(ops, prefix, nops, total)
-#define TBH_GEMM_SHAPES(T, V)      \
-  if (shape == 1)                  \
-    TBH_GEMM_LAUNCH(T, V, 1);      \
-  else if (shape == 2)             \
-    TBH_GEMM_LAUNCH(T, V, 2);      \
-  else                             \
-    TBH_GEMM_LAUNCH(T, V, 0);
-  if (dtype == 0) {
-    if (vec) {
-      TBH_GEMM_SHAPES(float, true)
-    } else {
-      TBH_GEMM_SHAPES(float, false)
-    }
-  } else {
-    if (vec) {
-      TBH_GEMM_SHAPES(int32_t, true)
-    } else {
-      TBH_GEMM_SHAPES(int32_t, false)
-    }
-  }
-#undef TBH_GEMM_SHAPES
-#undef TBH_GEMM_LAUNCH
-  return hipGetLastError();
+  void* args[] = {&ops, &prefix, &nops, &total};
+  const void* k = dtype == 0 ? gemm_kernel<float>(vec, shape) : gemm_kernel<int32_t>(vec, shape);
+  return hipLaunchKernel(k, dim3(grid), dim3(256), args, 0, s);
 }
 
 int gemm_blocks_per_cu(int dtype, bool vec, int shape) {
   int n = 0;
-  hipError_t err = hipSuccess;
-#define TBH_GEMM_OCC(T, V, S) \
-  err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, tbh_gemm_kernel<T, V, S>, 256, 0)
-#define TBH_GEMM_OCC_SHAPES(T, V) \
-  if (shape == 1)                 \
-    TBH_GEMM_OCC(T, V, 1);        \
-  else if (shape == 2)            \
-    TBH_GEMM_OCC(T, V, 2);        \
-  else                            \
-    TBH_GEMM_OCC(T, V, 0);
-  if (dtype == 0) {
-    if (vec) {
-      TBH_GEMM_OCC_SHAPES(float, true)
-    } else {
-      TBH_GEMM_OCC_SHAPES(float, false)
-    }
-  } else {
-    if (vec) {
-      TBH_GEMM_OCC_SHAPES(int32_t, true)
-    } else {
-      TBH_GEMM_OCC_SHAPES(int32_t, false)
-    }
-  }
-#undef TBH_GEMM_OCC_SHAPES
-#undef TBH_GEMM_OCC
+  const void* k = dtype == 0 ? gemm_kernel<float>(vec, shape) : gemm_kernel<int32_t>(vec, shape);
+  const hipError_t err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 256, 0);
   return err == hipSuccess && n > 0 ? n : 2;
 }
 

@@ -1735,6 +1735,36 @@ int tbh_contract_max(tbh_ctx* ctx, tbh_dtype dtype, const tbh_slice* slices, siz
   return 0;
 }
 
+// Whether a standalone product runs on K1b (64 x 64 tiles), and in how many
+// K ranges.  K1 keeps the aligned products of at least 512 of its tiles and
+// K <= 256: there K1b's pass over the waves' maxima, once per 64 x 64 outputs,
+// costs more than its finer tiles give (4096 x 4096, kernel us K1 / K1b: K = 16
+// 22 / 46, 64 46 / 62, 256 136 / 151, 1024 486 / 491, 4096 1803 / 1742; 512
+// products of 128 x 128 x 64 27 / 34).  With fewer tiles K1 leaves CUs idle
+// (3072 x 2048 x 128 38 / 37; 2048^2 x 64 22 / 20; 1024^3 224 / 47; 512^3
+// 114 / 19), and unaligned extents took K1's scalar loads (three 1021 x 515 x
+// 777 Int32 238 / 92).  K1 alone takes M or K below one quad.  Products of
+// fewer than 256 tiles are split over K until 512 workgroups run, in ranges
+// of at least 128 (64^2 outputs of K = 3428: 800 / 25; 256 or 768 workgroups,
+// or ranges of 64, measured within 10% of this).
+static bool split_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec,
+                       int64_t k1_tiles, GemmSplit* g) {
+  if (M < 4 || K < 4 || (vec && k1_tiles >= 512 && K <= 256)) return false;
+  const int64_t tm = (M + 63) / 64, tn = (N + 63) / 64;
+  if (tm * tn > (int64_t)1 << 28 || tm * tn * batch > (int64_t)1 << 28) return false;
+  const int64_t tiles = tm * tn * batch;
+  const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(K / 128, 512 / tiles));
+  g->M = (int32_t)M;
+  g->N = (int32_t)N;
+  g->K = (int32_t)K;
+  g->batch = (int32_t)batch;
+  g->tiles_m = (int32_t)tm;
+  g->tiles_n = (int32_t)tn;
+  g->kpart = (int32_t)std::min<int64_t>(((K + parts - 1) / parts + 31) / 32 * 32, 1 << 30);
+  g->ksplit = (int32_t)((K + g->kpart - 1) / g->kpart);
+  return true;
+}
+
 int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_t K, int64_t batch,
                      const void* A, int64_t lda, int64_t strideA, const void* B, int64_t ldb,
                      int64_t strideB, void* C, int64_t ldc, int64_t strideC,
@@ -1796,6 +1826,54 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
     set_error("unknown ptr_kind");
     return TBH_EINVAL;
   }
+  // after the launch: the result back to a host C, then everything released
+  auto finish = [&](hipError_t e, hipEvent_t ev) {
+    if (ev)
+      ctx->prof.end(ctx->stream, ev, 2, 0, 1, 4.0 * (double)batch * (M * K + K * N + M * N),
+                    (double)M * N * K * batch);
+    ctx->stats.launches++;
+    if (e == hipSuccess && ptr_kind == TBH_HOST)
+      e = hipMemcpyAsync(C, dC, 4 * ec, hipMemcpyDeviceToHost, ctx->stream);
+    hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (ctx->profiling) ctx->prof.collect(ctx->stats);
+    release();
+    if (e != hipSuccess || es != hipSuccess) {
+      set_error(std::string("max-plus GEMM: ") + hipGetErrorString(e != hipSuccess ? e : es));
+      return (int)TBH_EDEVICE;
+    }
+    return (int)TBH_OK;
+  };
+  const bool vec = M % 4 == 0 && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
+                   strideA % 4 == 0 && strideB % 4 == 0 && strideC % 4 == 0 &&
+                   ((uint64_t)dA % 16 == 0) && ((uint64_t)dB % 16 == 0) && ((uint64_t)dC % 16 == 0);
+  const int shape = vec ? gemm_shape(M, N) : 0;
+  const int64_t k1_m = (M + gemm_bm(shape) - 1) / gemm_bm(shape),
+                k1_n = (N + gemm_bn(shape) - 1) / gemm_bn(shape);
+  GemmSplit gs;
+  if (split_gemm(M, N, K, batch, vec, k1_m * k1_n * batch, &gs)) {
+    gs.a = (uint64_t)dA;
+    gs.b = (uint64_t)dB;
+    gs.c = (uint64_t)dC;
+    gs.lda = lda;
+    gs.ldb = ldb;
+    gs.ldc = ldc;
+    gs.sA = strideA;
+    gs.sB = strideB;
+    gs.sC = strideC;
+    gs.ws = 0;
+    if (gs.ksplit > 1) {
+      const int64_t o = ctx->pool.alloc((size_t)4 * gs.ksplit * M * N * batch);
+      if (o >= 0) {
+        offs.push_back(o);
+        gs.ws = (uint64_t)(ctx->base + o);
+      } else {
+        gs.ksplit = 1;  // no room for partial maxima
+        gs.kpart = (int32_t)std::min<int64_t>(((int64_t)gs.K + 31) / 32 * 32, INT32_MAX / 32 * 32);
+      }
+    }
+    hipEvent_t ev = ctx->profiling ? ctx->prof.begin(ctx->stream) : nullptr;
+    return finish(launch_gemm_ksplit(dtype, gs, ctx->stream), ev);
+  }
   GemmDesc d;
   std::memset(&d, 0, sizeof d);
   d.a = (uint64_t)dA;
@@ -1811,14 +1889,11 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
   d.sA = strideA;
   d.sB = strideB;
   d.sC = strideC;
-  d.shape = gemm_shape(M, N);
+  d.shape = shape;
   d.scatter = 0;
-  d.tiles_m = (int32_t)((M + gemm_bm(d.shape) - 1) / gemm_bm(d.shape));
-  d.tiles_n = (int32_t)((N + gemm_bn(d.shape) - 1) / gemm_bn(d.shape));
+  d.tiles_m = (int32_t)k1_m;
+  d.tiles_n = (int32_t)k1_n;
   const int64_t total = gemm_tiles(d);
-  const bool vec = M % 4 == 0 && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
-                   strideA % 4 == 0 && strideB % 4 == 0 && strideC % 4 == 0 &&
-                   ((uint64_t)dA % 16 == 0) && ((uint64_t)dB % 16 == 0) && ((uint64_t)dC % 16 == 0);
   int64_t doff = ctx->pool.alloc(sizeof d + 64);
   if (doff < 0) {
     release();
@@ -1841,20 +1916,7 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
   if (e == hipSuccess)
     e = launch_gemm(dtype, vec, d.shape, (const GemmDesc*)dd, (const int64_t*)(dd + sizeof d), 1,
                     total, gemm_grid(ctx, total, dtype, vec, d.shape), ctx->stream);
-  if (ev)
-    ctx->prof.end(ctx->stream, ev, 2, 0, 1, 4.0 * (double)batch * (M * K + K * N + M * N),
-                  (double)M * N * K * batch);
-  ctx->stats.launches++;
-  if (e == hipSuccess && ptr_kind == TBH_HOST)
-    e = hipMemcpyAsync(C, dC, 4 * ec, hipMemcpyDeviceToHost, ctx->stream);
-  hipError_t es = hipStreamSynchronize(ctx->stream);
-  if (ctx->profiling) ctx->prof.collect(ctx->stats);
-  release();
-  if (e != hipSuccess || es != hipSuccess) {
-    set_error(std::string("maxplus_gemm: ") + hipGetErrorString(e != hipSuccess ? e : es));
-    return TBH_EDEVICE;
-  }
-  return 0;
+  return finish(e, ev);
 }
 
 static int view_slice(const tbh_slice* s, SliceIn* in) {

@@ -29,6 +29,7 @@ hipError_t launch_ew_direct(int dtype, const EwDesc* ops, const int64_t* prefix,
                             int64_t total, int grid, int chunk, hipStream_t s);
 hipError_t launch_gemm(int dtype, bool vec, int shape, const GemmDesc* ops, const int64_t* prefix,
                        int nops, int64_t total, int grid, hipStream_t s);
+hipError_t launch_gemm_ksplit(int dtype, const GemmSplit& g, hipStream_t s);  // tbh_gemm.hip
 hipError_t launch_leaves(int dtype, const LeafDesc* leaves, int64_t n, hipStream_t s);
 hipError_t launch_epilogue(int dtype, const EpiDesc* e, int64_t n, void* out, hipStream_t s);
 hipError_t launch_units(int dtype, const UnitDesc* units, const UnitItem* items,
