@@ -160,7 +160,14 @@ struct Builder {
       if (pos_in(LC, l) < 0) R.push_back(l);
     for (int32_t l : LB)
       if (pos_in(LC, l) < 0 && pos_in(LA, l) < 0) R.push_back(l);
-    if ((R.size() > 8 && op.nP < 20) || R.size() > (size_t)kMaxReduce) {
+    // (7: a tile of 2^12 outputs loops 2^R configurations in stages of about
+    // 2 us, and such steps have few tiles: 20-label operands reduced to 14
+    // labels took 140 us and more in 4 workgroups.  301 slices of 3-regular
+    // n=200 at sc 20: tiled EW 3.33 ms when only R > 8 splits, 1.99 from 7,
+    // 1.92 from 6, 1.85 from 5; n=300 at sc 25 the same within 1%.  Below
+    // 2^18 configurations a second launch costs more than the loop.)
+    if ((R.size() >= 7 && op.nP < 20 && (op.nP + R.size() >= 18 || R.size() > 8)) ||
+        R.size() > (size_t)kMaxReduce) {
       // split-K: keep the last s reduced labels in a temporary (more
       // outputs, shorter loops), then reduce them in a second step
       const int s_keep = R.size() > (size_t)kMaxReduce && op.nP >= 20

@@ -598,12 +598,21 @@ int direct_grid(tbh_ctx* ctx, int64_t total, int chunk) {
 // on launches large enough to give every workgroup of the grid such a claim:
 // smaller launches (serving rounds, small solves) were slower with 8 than
 // with 4, so a claim above 4 is halved, down to 4, until the launch fills the
-// grid with claims.
-int direct_chunk(tbh_ctx* ctx, int64_t) { return std::max(1, ctx->tune.direct_chunk); }
+// grid with claims.  A claim is halved further until the launch gives every
+// resident workgroup two claims: below that the tiles of a claim, one after
+// another, are the launch's length while CUs are idle (3-regular n=200 whole:
+// tiled EW 571 us with claims of 4, 272 so; the King's subgraph 837 -> 534;
+// one or four claims per workgroup within 5% of two).  Direct claims follow
+// the same rule on 16 waves per CU (132 -> 111 us there).
+int direct_chunk(tbh_ctx* ctx, int64_t total) {
+  return (int)std::max<int64_t>(
+      1, std::min<int64_t>(ctx->tune.direct_chunk, total / ((int64_t)ctx->num_cus * 16)));
+}
 int ew_chunk(tbh_ctx* ctx, int64_t total) {
   int c = std::max(1, ctx->tune.ew_chunk);
-  const int64_t grid_cap = (int64_t)ctx->num_cus * ctx->tune.ew_per_cu * ctx->tune.ew_grid_mult;
-  while (c > 4 && total < (int64_t)c * grid_cap) c >>= 1;
+  const int64_t slots = (int64_t)ctx->num_cus * ctx->tune.ew_per_cu;
+  while (c > 4 && total < (int64_t)c * slots * ctx->tune.ew_grid_mult) c >>= 1;
+  while (c > 1 && total < (int64_t)c * slots * 2) c >>= 1;
   return c;
 }
 
