@@ -222,9 +222,10 @@ typedef struct {
  * entry the region's best weight with its open vertices fixed to each b (the
  * tropical zero where b is not independent) -- the SizeMax contraction of
  * the region's network with its boundary open, which callers obtain from
- * tbh_contract_slices (one slice per b); on return the reduced alpha tensor
- * (mis_compactify!: an entry is set to the tropical zero when a proper
- * subset of its boundary configuration reaches at least its value).
+ * tbh_region_alpha, or from tbh_contract_slices (one slice per b); on return
+ * the reduced alpha tensor (mis_compactify!: an entry is set to the tropical
+ * zero when a proper subset of its boundary configuration reaches at least
+ * its value).
  * configs: every region configuration (bitmask over the region's vertices)
  * that is independent and whose weight equals the reduced alpha of its
  * boundary bits, i.e. the rows of the BranchingTable; region i's
@@ -235,6 +236,13 @@ typedef struct {
 int tbh_region_tables(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region* regions,
                       size_t n, void* alpha, size_t* group_ptr,
                       uint32_t* configs, size_t cap, size_t* total);
+
+/* The alpha tensors tbh_region_tables takes, of the same regions: every
+ * region configuration enumerated on the GPU.  Int32 regions need the bound of
+ * an Int32 slice for every independent boundary configuration: |sum of its
+ * weights| + sum |w| over the inner vertices it leaves < 2^28. */
+int tbh_region_alpha(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region* regions, size_t n,
+                     void* alpha);
 
 /* ---- introspection ---------------------------------------------------- */
 /* One planned step of a slice (no reference counterpart: used by tests and

@@ -114,6 +114,8 @@ TBH_SIGNATURES = {
     "tbh_serve_start_ex": (C.c_int, [C.c_void_p, C.POINTER(TbhServeConfig)]),
     "tbh_serve_stats": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64),
                                   C.POINTER(C.c_uint64)]),
+    "tbh_region_alpha": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(TbhRegion), C.c_size_t,
+                                   C.c_void_p]),
     "tbh_region_tables": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(TbhRegion), C.c_size_t,
                                     C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t,
                                     C.POINTER(C.c_size_t)]),

@@ -7,15 +7,13 @@ vertices are those with a neighbour outside it.  Its alpha tensor holds, per
 boundary configuration b (bit k = the k-th open vertex in region order),
 the best weight of an independent set of the region whose boundary part is
 b: the SizeMax contraction of the region's tensor network with its open
-labels kept.  It is computed here as one scalar contraction per b -- the
-open vertices fixed to b (those in b taken, with r = their weight, and
-their neighbours removed; the others removed), the rest of the region
-contracted -- for every region and b in ONE batched tbh_contract_slices
-submit.  tbh_region_tables then prunes each tensor as mis_compactify! does
-(an entry that a proper subset of its boundary configuration matches or
-beats becomes the tropical zero) and enumerates, for each surviving b,
-every region configuration that reaches it: the rows of the table.  Both
-steps run on the GPU.
+labels kept.  tbh_region_alpha computes it for every region in one
+launch by enumerating the region's configurations (at most 2^24), which the
+table's rows need anyway.  tbh_region_tables then prunes each tensor as
+mis_compactify! does (an entry that a proper subset of its boundary
+configuration matches or beats becomes the tropical zero) and enumerates, for
+each surviving b, every region configuration that reaches it: the rows of the
+table.  All of it runs on the GPU.
 
 Exact parity with OptimalBranchingMIS (not vendored here) is unpinned; the
 tests pin the tables against brute-force enumeration of every region
@@ -27,18 +25,15 @@ import numpy as np
 
 from . import _lib
 from ._lib import check
-from .api import MISProblem, SimpleGraph, SlicedBranch, _dtype_code, default_backend
-from .workload import initialize_code
+from .api import _dtype_code, default_backend
 
 
 def open_vertices(g, vs):
     """The vertices of vs with a neighbour outside vs, in vs order."""
-    inside = set(int(v) for v in vs)
-    nb = {}
-    for u, v in np.asarray(g.edges).reshape(-1, 2):
-        nb.setdefault(int(u), []).append(int(v))
-        nb.setdefault(int(v), []).append(int(u))
-    return [int(v) for v in vs if any(x not in inside for x in nb.get(int(v), ()))]
+    edges = np.asarray(g.edges).reshape(-1, 2)
+    inside = np.isin(edges, [int(v) for v in vs])
+    crossing = set(edges[inside & ~inside[:, ::-1]].tolist())
+    return [int(v) for v in vs if int(v) in crossing]
 
 
 def neighbor_region(g, seeds, n_max):
@@ -91,11 +86,10 @@ def _region(p, vs, npdt):
         raise ValueError("a region lists a vertex twice")
     nv = len(vs)
     adj = np.zeros(max(1, nv), np.uint32)
-    for u, v in np.asarray(p.g.edges).reshape(-1, 2):
-        u, v = int(u), int(v)
-        if u in pos and v in pos:
-            adj[pos[u]] |= np.uint32(1 << pos[v])
-            adj[pos[v]] |= np.uint32(1 << pos[u])
+    edges = np.asarray(p.g.edges).reshape(-1, 2)
+    for u, v in edges[np.isin(edges, vs).all(axis=1)].tolist():
+        adj[pos[u]] |= np.uint32(1 << pos[v])
+        adj[pos[v]] |= np.uint32(1 << pos[u])
     ov = open_vertices(p.g, vs)
     opos = [pos[v] for v in ov]
     if p.weights is None:
@@ -105,63 +99,23 @@ def _region(p, vs, npdt):
     return vs, adj[:nv] if nv else adj[:0], ov, opos, w
 
 
-def _inner_slice(adj, w, keep, r, weighted, cache, trials, seed):
-    """The slice of the region's vertices in `keep` (fixed part worth r)."""
-    key = tuple(keep)
-    if key not in cache:
-        idx = {v: i for i, v in enumerate(keep)}
-        edges = [[idx[v], idx[u]] for v in keep for u in keep
-                 if u > v and (int(adj[v]) >> u) & 1]
-        g = SimpleGraph(len(keep), np.array(edges, np.int32).reshape(-1, 2))
-        code = initialize_code(g, trials, seed) if len(keep) else None
-        cache[key] = (g, code)
-    g, code = cache[key]
-    wk = np.asarray(w)[list(keep)] if weighted and len(keep) else None
-    return SlicedBranch(MISProblem(g, wk), code, r)
-
-
 def branching_tables(items, element_type=np.float32, backend=None, order_trials=4, seed=0):
     """Branching tables of many regions at once: items = [(MISProblem,
-    region vertex list), ...] -> [BranchingTable, ...].  Every region's
-    boundary configurations are contracted in one batched submit, then
-    pruned and enumerated on the GPU (tbh_region_tables)."""
+    region vertex list), ...] -> [BranchingTable, ...].  Every region's alpha
+    tensor, its pruning and its rows come from the GPU (tbh_region_alpha,
+    tbh_region_tables).  order_trials and seed, which tune a search for
+    contraction trees, have no effect on the tables."""
     be = backend or default_backend()
     code, npdt = _dtype_code(element_type)
-    zero = -np.inf if npdt == np.float32 else _lib.TBH_I32_NEG_INF
-    regions, slices, where = [], [], []
-    for it, (p, vs) in enumerate(items):
+    regions = []
+    for p, vs in items:
         vs, adj, ov, opos, w = _region(p, vs, npdt)
         if len(vs) > 24 or len(ov) > 16:
             raise ValueError("a region needs at most 24 vertices and 16 open vertices")
-        open_mask = sum(1 << i for i in opos)
-        inner = [i for i in range(len(vs)) if not (open_mask >> i) & 1]
-        cache = {}
-        nb = 1 << len(opos)
-        for b in range(nb):
-            chosen = [opos[k] for k in range(len(opos)) if (b >> k) & 1]
-            cmask = sum(1 << c for c in chosen)
-            if any(int(adj[c]) & cmask for c in chosen):
-                continue  # not independent: alpha[b] is the tropical zero
-            removed = 0
-            for c in chosen:
-                removed |= int(adj[c])
-            keep = [i for i in inner if not (removed >> i) & 1]
-            r = sum(w[c] for c in chosen)
-            r = float(r) if npdt == np.float32 else int(r)
-            slices.append(_inner_slice(adj, w, keep, r, p.weights is not None, cache,
-                                       order_trials, seed))
-            where.append((it, b))
-        regions.append((vs, adj, ov, opos, w, open_mask, nb))
-    # one batched submit for every region's boundary configurations
-    vals = be.contract_slices(slices, npdt, "batched") if slices else np.zeros(0, npdt)
-    a0 = np.cumsum([0] + [R[6] for R in regions])
-    alpha = np.full(int(a0[-1]), zero, npdt)
-    for (it, b), v in zip(where, vals):
-        alpha[a0[it] + b] = v
-    # prune and enumerate on the GPU
+        regions.append((vs, adj, ov, opos, w))
     arr = (_lib.TbhRegion * max(1, len(regions)))()
     keep = []
-    for i, (vs, adj, ov, opos, w, open_mask, nb) in enumerate(regions):
+    for i, (vs, adj, ov, opos, w) in enumerate(regions):
         a = np.ascontiguousarray(adj, np.uint32)
         keep.append(a)
         arr[i].nv = len(vs)
@@ -172,26 +126,37 @@ def branching_tables(items, element_type=np.float32, backend=None, order_trials=
             arr[i].weights = ww.ctypes.data
         else:
             arr[i].weights = None
-        arr[i].open = open_mask
-    gptr = np.zeros(len(regions) + 1, np.uint64)
+        arr[i].open = sum(1 << k for k in opos)
+    n = len(regions)
+    a0 = np.cumsum([0] + [1 << len(R[3]) for R in regions])
+    alpha = np.empty(max(1, int(a0[-1])), npdt)
+    check(_lib.tbh().tbh_region_alpha(be.handle, code, arr, n, alpha.ctypes.data))
+    # the rows, into a buffer most calls fit; else once more with their number
+    gptr = np.zeros(n + 1, np.uint64)
     total = C.c_size_t()
-    raw = alpha.copy()
-    check(_lib.tbh().tbh_region_tables(be.handle, code, arr, len(regions), raw.ctypes.data,
-                                       gptr.ctypes.data, None, 0, C.byref(total)))
-    cfg = np.zeros(max(1, total.value), np.uint32)
     reduced = alpha.copy()
-    check(_lib.tbh().tbh_region_tables(be.handle, code, arr, len(regions), reduced.ctypes.data,
-                                       gptr.ctypes.data, cfg.ctypes.data, total.value,
-                                       C.byref(total)))
+    cap = min(sum(1 << len(R[0]) for R in regions), 1 << 20)
+    cfg = np.empty(max(1, cap), np.uint32)
+    rc = _lib.tbh().tbh_region_tables(be.handle, code, arr, n, reduced.ctypes.data,
+                                      gptr.ctypes.data, cfg.ctypes.data, cap, C.byref(total))
+    if rc == _lib.TBH_ENOMEM and total.value > cap:
+        cfg = np.empty(total.value, np.uint32)
+        reduced = alpha.copy()
+        rc = _lib.tbh().tbh_region_tables(be.handle, code, arr, n, reduced.ctypes.data,
+                                          gptr.ctypes.data, cfg.ctypes.data, total.value,
+                                          C.byref(total))
+    check(rc)
     out = []
-    for i, (vs, adj, ov, opos, w, open_mask, nb) in enumerate(regions):
+    for i, (vs, adj, ov, opos, w) in enumerate(regions):
         red = reduced[a0[i]:a0[i + 1]]
-        rows = {}
-        for x in cfg[int(gptr[i]):int(gptr[i + 1])]:
-            x = int(x)
-            b = sum(((x >> opos[k]) & 1) << k for k in range(len(opos)))
-            rows.setdefault(b, []).append(x)
-        table = [rows[b] for b in sorted(rows)]
+        x = cfg[int(gptr[i]):int(gptr[i + 1])]
+        # ordered by boundary configuration, then ascending: a row each
+        b = np.zeros(len(x), np.uint32)
+        for k, at in enumerate(opos):
+            b |= ((x >> np.uint32(at)) & np.uint32(1)) << np.uint32(k)
+        rows = x.tolist()
+        cuts = [0] + (np.flatnonzero(b[1:] != b[:-1]) + 1).tolist() + [len(rows)]
+        table = [rows[s:e] for s, e in zip(cuts, cuts[1:]) if e > s]
         out.append(BranchingTable(vs, ov, red.copy(), table))
     return out
 

@@ -7,10 +7,18 @@
 // mis_compactify!) -- and, per surviving b, every region configuration that
 // reaches it (the table rows of a BranchingTable).
 //
-// The alpha tensors themselves are tropical contractions (SizeMax of the
-// region's network with its boundary fixed, one scalar slice per b) and
-// come in through tbh_contract_slices, batched over every region and b; this
-// file prunes them and enumerates the configurations, both on the GPU:
+// The alpha tensors are the SizeMax contraction of the region's network with
+// its boundary fixed; they come in from the caller, or from tbh_region_alpha,
+// which enumerates the region's 2^nv configurations (nv <= 24) as the table
+// itself does.  A contraction per b (one scalar slice each: 2224 slices for 8
+// regions of 14 vertices) took 45 ms, nearly all of it building and planning
+// slices on the host; with the enumeration of the same regions, one launch,
+// the tables take 1.6 ms:
+//   tbh_alpha_kernel        a workgroup walks a run of a region's
+//                           configurations, weighs the independent ones and
+//                           keeps the best per boundary bits in LDS (up to
+//                           2^12 of them, else straight in memory), merged by
+//                           an integer atomic max on order-preserving keys;
 //   tbh_compactify_kernel   one thread per (region, a): a survives unless a
 //                           proper subset b of a has alpha[b] >= alpha[a];
 //   tbh_configs_kernel      one thread per (region, x in {0,1}^nv): x is kept
@@ -77,6 +85,87 @@ __device__ __forceinline__ int find_region(const int64_t* __restrict__ prefix, i
   return lo;
 }
 
+// Order-preserving integer keys of the finite values of T (and the inverse);
+// kNoKey: no configuration seen.
+constexpr int32_t kNoKey = INT32_MIN;
+__device__ __forceinline__ int32_t key_of(int32_t v) { return v; }
+__device__ __forceinline__ int32_t key_of(float v) {
+  const int32_t b = __builtin_bit_cast(int32_t, v);
+  return b < 0 ? b ^ 0x7fffffff : b;
+}
+template <typename T>
+__device__ __forceinline__ T of_key(int32_t k);
+template <>
+__device__ __forceinline__ int32_t of_key<int32_t>(int32_t k) { return k; }
+template <>
+__device__ __forceinline__ float of_key<float>(int32_t k) {
+  return __builtin_bit_cast(float, k < 0 ? k ^ 0x7fffffff : k);
+}
+
+constexpr int kAlphaLdsBits = 12;    // boundary bits kept in LDS
+constexpr int kAlphaRun = 1 << 12;   // configurations of one workgroup
+
+__global__ __launch_bounds__(256) void tbh_alpha_fill_kernel(int32_t* __restrict__ keys,
+                                                              int64_t total) {
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < total) keys[g] = kNoKey;
+}
+
+// Workgroup w: configurations run0 .. of region r (bprefix: workgroups per
+// region), in ascending vertex order of their weights' sum, as in
+// tbh_configs_kernel.
+template <typename T>
+__global__ __launch_bounds__(256) void tbh_alpha_kernel(const RegionDesc* __restrict__ R,
+                                                        const int64_t* __restrict__ bprefix,
+                                                        int n, int32_t* __restrict__ keys) {
+  __shared__ int32_t best[1 << kAlphaLdsBits];
+  __shared__ uint32_t adj[kRegionMaxNv], wb[kRegionMaxNv];
+  const int r = find_region(bprefix, n, blockIdx.x);
+  const RegionDesc& d = R[r];
+  const int tid = threadIdx.x;
+  const uint32_t open = d.open, entries = 1u << d.nopen;
+  const bool lds = d.nopen <= kAlphaLdsBits;
+  if (tid < kRegionMaxNv) {
+    adj[tid] = d.adj[tid];
+    wb[tid] = d.wbits[tid];
+  }
+  if (lds)
+    for (uint32_t k = tid; k < entries; k += 256) best[k] = kNoKey;
+  __syncthreads();
+  const uint32_t total = 1u << d.nv;
+  const uint32_t x0 = (uint32_t)(blockIdx.x - bprefix[r]) * kAlphaRun;
+  const uint32_t x1 = x0 + kAlphaRun < total ? x0 + kAlphaRun : total;
+  for (uint32_t x = x0 + tid; x < x1; x += 256) {
+    T w = (T)0;
+    bool ok = true;
+    for (uint32_t m = x; m && ok; m &= m - 1) {
+      const int v = __builtin_ctz(m);
+      ok = (adj[v] & x) == 0;
+      w += __builtin_bit_cast(T, wb[v]);
+    }
+    if (!ok) continue;
+    const uint32_t e = pext32(x, open);
+    if (lds)
+      atomicMax(&best[e], key_of(w));
+    else
+      atomicMax(&keys[d.a0 + e], key_of(w));
+  }
+  if (!lds) return;
+  __syncthreads();
+  for (uint32_t k = tid; k < entries; k += 256)
+    if (best[k] != kNoKey) atomicMax(&keys[d.a0 + k], best[k]);
+}
+
+// the keys as values, in place; no configuration: the tropical zero
+template <typename T>
+__global__ __launch_bounds__(256) void tbh_alpha_value_kernel(int32_t* __restrict__ keys,
+                                                              int64_t total) {
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= total) return;
+  const int32_t k = keys[g];
+  reinterpret_cast<T*>(keys)[g] = k == kNoKey ? tzero<T>() : of_key<T>(k);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void tbh_compactify_kernel(const RegionDesc* __restrict__ R,
                                                               const int64_t* __restrict__ aprefix,
@@ -140,22 +229,18 @@ __global__ __launch_bounds__(256) void tbh_configs_kernel(const RegionDesc* __re
 
 using namespace tbh;
 
-extern "C" int tbh_region_tables(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region* regions,
-                                 size_t n, void* alpha, size_t* group_ptr, uint32_t* configs,
-                                 size_t cap, size_t* total) {
-  if (!ctx || (n && (!regions || !alpha || !group_ptr || !total))) {
-    set_error("null argument");
-    return TBH_EINVAL;
-  }
+// Checked descriptors of the regions and the prefixes of their
+// configurations and alpha entries.
+static int build_regions(tbh_dtype dtype, const tbh_region* regions, size_t n,
+                         std::vector<RegionDesc>& desc, std::vector<int64_t>& xprefix,
+                         std::vector<int64_t>& aprefix) {
   if (dtype != TBH_F32 && dtype != TBH_I32) {
     set_error("unknown dtype");
     return TBH_EINVAL;
   }
-  *total = 0;
-  if (n == 0) return 0;
-  // descriptors and prefixes
-  std::vector<RegionDesc> desc(n);
-  std::vector<int64_t> xprefix(n + 1, 0), aprefix(n + 1, 0);
+  desc.resize(n);
+  xprefix.assign(n + 1, 0);
+  aprefix.assign(n + 1, 0);
   for (size_t i = 0; i < n; i++) {
     const tbh_region& q = regions[i];
     if (q.nv < 0 || q.nv > kRegionMaxNv || (q.nv > 0 && !q.adj)) {
@@ -221,6 +306,108 @@ extern "C" int tbh_region_tables(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region
     xprefix[i + 1] = xprefix[i] + ((int64_t)1 << q.nv);
     aprefix[i + 1] = aprefix[i] + ((int64_t)1 << d.nopen);
   }
+  return 0;
+}
+
+extern "C" int tbh_region_alpha(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region* regions,
+                                size_t n, void* alpha) {
+  if (!ctx || (n && (!regions || !alpha))) {
+    set_error("null argument");
+    return TBH_EINVAL;
+  }
+  std::vector<RegionDesc> desc;
+  std::vector<int64_t> xprefix, aprefix;
+  int rc = build_regions(dtype, regions, n, desc, xprefix, aprefix);
+  if (rc || n == 0) return rc;
+  if (dtype == TBH_I32) {
+    // the bound of an Int32 contraction, per boundary configuration: the
+    // weights of its open vertices, summed, and the absolute weights of the
+    // inner vertices it leaves stay below 2^28 together
+    for (size_t i = 0; i < n; i++) {
+      const RegionDesc& d = desc[i];
+      double all = 0;
+      for (int v = 0; v < d.nv; v++) all += std::fabs((double)(int32_t)d.wbits[v]);
+      if (all < (double)(1 << 28)) continue;
+      uint32_t b = 0;
+      do {  // subsets of the open vertices
+        double fixed = 0, inner = 0;
+        uint32_t removed = 0;
+        for (int v = 0; v < d.nv; v++)
+          if ((b >> v) & 1u) {
+            fixed += (double)(int32_t)d.wbits[v];
+            removed |= d.adj[v];
+          }
+        for (int v = 0; v < d.nv; v++)
+          if (!(((d.open | removed) >> v) & 1u)) inner += std::fabs((double)(int32_t)d.wbits[v]);
+        if (!(removed & b) && std::fabs(fixed) + inner >= (double)(1 << 28)) {
+          set_error("region " + std::to_string(i) +
+                    ": Int32 regions need sum |w| < 2^28 for every boundary configuration");
+          return TBH_EINVAL;
+        }
+        b = (b - d.open) & d.open;
+      } while (b);
+    }
+  }
+  std::vector<int64_t> bprefix(n + 1, 0);
+  for (size_t i = 0; i < n; i++)
+    bprefix[i + 1] = bprefix[i] + std::max<int64_t>(1, ((int64_t)1 << desc[i].nv) / kAlphaRun);
+  if (bprefix[n] > INT32_MAX) {
+    set_error("region tables: too many configurations in one call");
+    return TBH_EINVAL;
+  }
+  const int64_t A = aprefix[n];
+  std::lock_guard<std::mutex> g(ctx->mu);
+  const size_t o_bp = (n * sizeof(RegionDesc) + 255) / 256 * 256;
+  const size_t o_key = (o_bp + (n + 1) * 8 + 255) / 256 * 256;
+  const int64_t doff = ctx->pool.alloc(o_key + 4 * A);
+  if (doff < 0) {
+    set_error("pool exhausted (region tables)");
+    return TBH_ENOMEM;
+  }
+  char* dev = ctx->base + doff;
+  int32_t* keys = (int32_t*)(dev + o_key);
+  hipStream_t s = ctx->stream;
+  const int ga = (int)((A + 255) / 256);
+  const RegionDesc* dR = (const RegionDesc*)dev;
+  const int64_t* dbp = (const int64_t*)(dev + o_bp);
+  hipError_t e = hipSetDevice(ctx->device);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(dev, desc.data(), n * sizeof(RegionDesc), hipMemcpyHostToDevice, s);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(dev + o_bp, bprefix.data(), (n + 1) * 8, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) {
+    tbh_alpha_fill_kernel<<<ga, 256, 0, s>>>(keys, A);
+    if (dtype == TBH_F32) {
+      tbh_alpha_kernel<float><<<(int)bprefix[n], 256, 0, s>>>(dR, dbp, (int)n, keys);
+      tbh_alpha_value_kernel<float><<<ga, 256, 0, s>>>(keys, A);
+    } else {
+      tbh_alpha_kernel<int32_t><<<(int)bprefix[n], 256, 0, s>>>(dR, dbp, (int)n, keys);
+      tbh_alpha_value_kernel<int32_t><<<ga, 256, 0, s>>>(keys, A);
+    }
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(alpha, keys, 4 * A, hipMemcpyDeviceToHost, s);
+  const hipError_t es = hipStreamSynchronize(s);
+  ctx->pool.free(doff);
+  if (e != hipSuccess || es != hipSuccess) {
+    set_error(std::string("region alpha: ") + hipGetErrorString(e != hipSuccess ? e : es));
+    return TBH_EDEVICE;
+  }
+  return 0;
+}
+
+extern "C" int tbh_region_tables(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region* regions,
+                                 size_t n, void* alpha, size_t* group_ptr, uint32_t* configs,
+                                 size_t cap, size_t* total) {
+  if (!ctx || (n && (!regions || !alpha || !group_ptr || !total))) {
+    set_error("null argument");
+    return TBH_EINVAL;
+  }
+  if (total) *total = 0;
+  std::vector<RegionDesc> desc;
+  std::vector<int64_t> xprefix, aprefix;
+  int rc0 = build_regions(dtype, regions, n, desc, xprefix, aprefix);
+  if (rc0 || n == 0) return rc0;
   const int64_t X = xprefix[n], A = aprefix[n];
   std::lock_guard<std::mutex> g(ctx->mu);
   hipError_t e = hipSetDevice(ctx->device);
