@@ -10,6 +10,7 @@
 // lgkmcnt and so would make every wait for an LDS or scalar access wait for
 // the data loads in flight too.
 #define TBH_GLOBAL __attribute__((address_space(1)))
+#define TBH_LDS __attribute__((address_space(3)))
 
 namespace tbh {
 

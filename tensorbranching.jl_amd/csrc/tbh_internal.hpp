@@ -119,9 +119,9 @@ struct EpiDesc {
   int32_t res;     // index of the result
 };
 
-// A fused subtree ("unit"): every step of a maximal subtree whose tensors all
-// fit in LDS, contracted by one workgroup; only the subtree's root goes to
-// memory.  Inside a unit every tensor holds its labels in one global order
+// A fused part of the tree ("unit"): every step of a maximal connected part
+// whose tensors all fit in LDS, contracted by one workgroup.  Tensors from
+// outside it (ext) are copied to LDS first, only its root goes to memory.  Inside a unit every tensor holds its labels in one global order
 // (elimination time, latest first), so a step's union index -- the output's
 // bits, then the reduced labels' -- maps to an operand's by keeping the
 // operand's bits (mA / mB), and a step is 16 bytes.
@@ -129,6 +129,7 @@ constexpr int kUnitWaves = 4;      // waves of a unit's workgroup
 constexpr int kUnitLds = 8192;     // LDS elements of a unit
 constexpr int kUnitBits = 15;      // union labels of a unit's step
 constexpr int kUnitRank = 14;      // output labels of a unit's step
+constexpr int kUnitOperand = 12;  // labels of a tensor read from memory
 constexpr int kUnitReduce = 6;     // reduced labels of a unit's step
 // One wave's share of one step: chunks c0 .. c0+nc-1 of 64 outputs.
 struct UnitItem {
@@ -145,9 +146,16 @@ struct UnitDesc {
   uint32_t w0;       // first vertex weight
   int32_t rounds;    // items per wave; 0: a leaf tensor (nvert 1: vertex, 0: edge)
   int32_t nvert;     // vertex leaves, [0, w] at LDS 4 + 2 i (the edge tensor is at 0)
+  uint32_t ext0;     // first tensor read from memory
+  int32_t next;      // ... and their number
   int32_t res;       // c == 0: index of the slice's result
   int32_t rbits;     // ... and its r
   uint64_t pos;      // nibble k: the C position of output bit k
+};
+struct UnitExt {
+  uint64_t p;        // device address, labels in the units' order
+  uint32_t off;      // LDS element offset
+  uint32_t rank;
 };
 
 }  // namespace tbh

@@ -82,7 +82,6 @@ struct KAcc<KEwS> {
   using type = KI8S;
 };
 #define TBH_KF(d, f) (typename KAcc<decltype(d)>::type{(d), (uint32_t)offsetof(EwDesc, f)})
-#define TBH_LDS __attribute__((address_space(3)))
 // Sub-tensors are staged with global_load_lds_dword (HBM -> LDS without a
 // register round trip, so every load of a sub-tensor is in flight at once);
 // 0 stages through registers in groups of 8.

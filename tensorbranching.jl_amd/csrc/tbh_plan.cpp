@@ -515,6 +515,7 @@ int verify_plan(const SlicePlan& P, std::string* err) {
     if (t.rank < 0 || t.rank > kMaxRank) return bad("rank");
   }
   for (const auto& op : P.ops) {
+    if (op.kind == kUnit) continue;  // verify_units
     const int ra = P.tensors[op.a].rank;
     const int rb = op.b >= 0 ? P.tensors[op.b].rank : 0;
     const int rc = P.tensors[op.c].rank;
@@ -754,9 +755,14 @@ struct UnitBuilder {
   int32_t nl;
   // log2 of a unit's MACs at most: 4 waves take about 5 us for 2^17
   static constexpr double kUnitMacs = 131072.0;
-  std::vector<char> in_unit;         // tree node (leaf or internal) inside a unit
-  std::vector<char> fit;             // internal node may be inside a unit
-  std::vector<int32_t> parent, level, node_at, vert;
+  // tree node (leaf or internal): inside a unit, the output of a unit of
+  // leaves (or a leaf in memory), or the output of a unit that also reads
+  // tensors from memory
+  enum { kOutside = 0, kInside = 1, kLeafUnit = 2, kMixedUnit = 3 };
+  std::vector<char> in_unit;
+  std::vector<char> fit;             // the node's whole subtree may be one unit
+  std::vector<char> small;           // the node's step alone may be in a unit
+  std::vector<int32_t> parent, level, node_at, vert, taken;
   std::vector<int32_t> off;          // LDS offset of a unit's tensor
   std::vector<std::vector<int32_t>> sorted;  // labels of a unit's tensors, by prio
 
@@ -771,6 +777,7 @@ struct UnitBuilder {
     const int32_t nn = nl - 1, tot = nl + nn;
     in_unit.assign(tot, 0);
     fit.assign(tot, 0);
+    small.assign(tot, 0);
     parent.assign(tot, -1);
     level.assign(tot, 0);
     off.assign(tot, 0);
@@ -791,14 +798,24 @@ struct UnitBuilder {
       const int64_t second = peak[x] >= peak[y] ? sx + peak[y] : sy + peak[x];
       peak[o] = std::max(std::max(first, second), sx + sy + so);
       macs[o] = macs[x] + macs[y] + std::ldexp(1.0, uni[j]);
-      fit[o] = fit[x] && fit[y] && uni[j] <= kUnitBits && rank(o) <= kUnitRank && uni[j] - rank(o) <= kUnitReduce &&
-               macs[o] <= kUnitMacs && std::max(first, second) <= kUnitLds;
+      small[o] = uni[j] <= kUnitBits && rank(o) <= kUnitRank &&
+                 uni[j] - rank(o) <= kUnitReduce && rank(x) <= kUnitOperand &&
+                 rank(y) <= kUnitOperand;
+      fit[o] = fit[x] && fit[y] && small[o] && macs[o] <= kUnitMacs &&
+               std::max(first, second) <= kUnitLds;
     }
   }
 
   // Plans the unit of root `root`, or returns false when its tensors do not
-  // fit the LDS (levels keep more tensors alive than the estimate of mark()).
-  bool build(int32_t root) {
+  // fit the LDS (levels keep more tensors alive than the estimate of mark())
+  // or its work passes the limit.  mixed: the unit takes the small nodes
+  // below root that are in no unit yet; what they read of other units and
+  // steps is read from memory.
+  bool build(int32_t root, bool mixed) {
+    auto external = [&](int32_t c) {
+      return mixed && c >= nl && (!small[c] || in_unit[c] != kOutside);
+    };
+    double work = 0;
     // nodes of the subtree, parents before children; a level is the distance
     // from the deepest node (children run one level before their parent)
     node_at.clear();
@@ -808,6 +825,8 @@ struct UnitBuilder {
     std::vector<int32_t> verts;
     for (size_t k = 0; k < node_at.size(); k++) {
       const int32_t o = node_at[k], j = o - nl;
+      if (external(o)) continue;
+      work += std::ldexp(1.0, uni[j]);
       for (int q = 0; q < 2; q++) {
         const int32_t c = s.tree[2 * j + q];
         if (c < nl) {
@@ -818,14 +837,22 @@ struct UnitBuilder {
           continue;
         }
         level[c] = level[o] + 1;
-        depth = std::max(depth, level[c]);
+        if (!external(c)) depth = std::max(depth, level[c]);
         node_at.push_back(c);
       }
     }
+    if (work > kUnitMacs) return false;
     // breadth first: node_at is in descending level order from the back
     // LDS: the edge tensor, the vertex tensors, then the internal tensors,
     // blocks of a level's dead operands reused one level later
     int top = 4 + 2 * nvert;
+    if (mixed)  // tensors from memory are in LDS from the start
+      for (int32_t o : node_at)
+        if (external(o)) {
+          off[o] = top;
+          top += 1 << rank(o);
+          if (top > kUnitLds) return false;
+        }
     std::vector<int32_t> freeb[kUnitBits + 1];
     size_t dead = node_at.size();  // node_at[dead..]: tensors already released
     for (size_t k = node_at.size(); k-- > 1;) {
@@ -835,6 +862,7 @@ struct UnitBuilder {
         dead--;
         freeb[rank(node_at[dead])].push_back(off[node_at[dead]]);
       }
+      if (external(o)) continue;
       const int r = rank(o);
       int c = r;
       while (c <= kUnitBits && freeb[c].empty()) c++;
@@ -856,6 +884,16 @@ struct UnitBuilder {
     u.nvert = nvert;
     u.item0 = (uint32_t)P.items.size();
     u.w0 = (uint32_t)P.unit_w.size();
+    u.ext0 = (uint32_t)P.ext.size();
+    if (mixed)
+      for (int32_t o : node_at)
+        if (external(o)) {
+          P.ext.push_back({o, (uint32_t)off[o]});
+          sorted[o].assign(lab[o].begin(), lab[o].end());
+          std::sort(sorted[o].begin(), sorted[o].end(),
+                    [&](int32_t p, int32_t q) { return prio[p] < prio[q]; });
+          u.next++;
+        }
     for (int32_t c : verts) {
       const int32_t v = lab[c][0];
       P.unit_w.push_back(s.wbits ? s.wbits[v] : s.unit_wbits);
@@ -867,6 +905,7 @@ struct UnitBuilder {
       const int lv = level[node_at[k - 1]];
       for (; k > 0 && level[node_at[k - 1]] == lv; k--) {
         const int32_t o = node_at[k - 1], j = o - nl;
+        if (external(o)) continue;
         const int32_t x = s.tree[2 * j], y = s.tree[2 * j + 1];
         for (int32_t c : {x, y})
           if (c < nl) {
@@ -904,12 +943,15 @@ struct UnitBuilder {
           wave[next].push_back(it);
           next = (next + 1) % kUnitWaves;
         }
-        P.unit_steps.push_back({(int8_t)rank(x), (int8_t)rank(y), (int8_t)nP, (int8_t)nR});
-        P.exec_macs += std::ldexp(1.0, n);
+        P.unit_steps.push_back(
+            {(int8_t)rank(x), (int8_t)rank(y), (int8_t)nP, (int8_t)nR, (int32_t)P.units.size()});
+        u.macs += (double)(1u << n);
+        u.bytes += 4.0 * ((1u << rank(x)) + (1u << rank(y)) + (1u << nP));
       }
       // every wave ends the level in the same round
       size_t rounds = 0;
       for (auto& w : wave) rounds = std::max(rounds, w.size());
+      if (rounds == 0) continue;  // a level of tensors from memory only
       for (auto& w : wave) {
         w.resize(rounds, UnitItem{});
         w.back().f |= kItemBarrier;
@@ -919,15 +961,25 @@ struct UnitBuilder {
     for (auto& w : wave) P.items.insert(P.items.end(), w.begin(), w.end());
     P.units.push_back(u);
     P.unit_levels = std::max(P.unit_levels, depth + 1);
-    for (int32_t o : node_at) {
-      in_unit[o] = 1;
-      for (int q = 0; q < 2; q++) in_unit[s.tree[2 * (o - nl) + q]] = 1;
+    // (root last: external() reads in_unit of the nodes below it)
+    for (size_t q = node_at.size(); q-- > 0;) {
+      const int32_t o = node_at[q];
+      if (external(o)) continue;
+      for (int h = 0; h < 2; h++) {
+        const int32_t c = s.tree[2 * (o - nl) + h];
+        if (c < nl) in_unit[c] = kInside;
+      }
+      taken.push_back(o);
     }
+    for (int32_t o : taken) in_unit[o] = kInside;
+    taken.clear();
+    in_unit[root] = mixed ? kMixedUnit : kLeafUnit;
     return true;
   }
 
-  // Units of the whole tree, then a leaf unit for every leaf outside them.
-  // in_unit afterwards: 1 inside a unit, 2 a unit's (or leaf's) output.
+  // Units of leaves, then units over their outputs and those of the steps
+  // between (the small end of a tree past its largest tensors, above all),
+  // then a leaf unit for every leaf outside them.
   void run() {
     const int32_t nn = nl - 1;
     mark();
@@ -937,15 +989,14 @@ struct UnitBuilder {
     while (!roots.empty()) {
       const int32_t o = roots.back();
       roots.pop_back();
-      if (build(o)) {
-        in_unit[o] = 2;
-        continue;
-      }
+      if (build(o, false)) continue;
       for (int q = 0; q < 2; q++) {
         const int32_t c = s.tree[2 * (o - nl) + q];
         if (c >= nl) roots.push_back(c);
       }
     }
+    for (int32_t o = nl + nn - 1; o >= nl; o--)
+      if (small[o] && in_unit[o] == kOutside && !build(o, true)) small[o] = 0;
     for (int32_t i = 0; i < nl; i++) {
       if (in_unit[i]) continue;
       PUnit u;
@@ -955,8 +1006,15 @@ struct UnitBuilder {
       u.w0 = (uint32_t)P.unit_w.size();
       if (u.nvert) P.unit_w.push_back(s.wbits ? s.wbits[lab[i][0]] : s.unit_wbits);
       P.units.push_back(u);
-      in_unit[i] = 2;
+      in_unit[i] = kLeafUnit;
     }
+  }
+
+  // index of the unit whose output is o
+  int unit_of(int32_t o) const {
+    for (size_t k = P.units.size(); k-- > 0;)
+      if (P.units[k].tensor == o) return (int)k;
+    return -1;
   }
 
   // output bit -> position in the layout its consumer reads
@@ -976,8 +1034,17 @@ int verify_units(const SlicePlan& P, std::string* err) {
     if (u.w0 + (size_t)u.nvert > P.unit_w.size() || 4 + 2 * u.nvert > kUnitLds)
       return bad("weights");
     const int rank = P.tensors[u.tensor].rank;
+    if (u.ext0 + (size_t)u.next > P.ext.size() || (u.next > 0) != (u.level > 0))
+      return bad("memory tensors");
+    for (int k = 0; k < u.next; k++) {
+      const PExt& x = P.ext[u.ext0 + k];
+      if (x.tensor < 0 || x.tensor >= (int)P.tensors.size() || x.off < 4u + 2 * u.nvert ||
+          P.tensors[x.tensor].rank > kUnitOperand || P.tensors[x.tensor].bytes == 0 ||
+          x.off + (1u << P.tensors[x.tensor].rank) > (uint32_t)kUnitLds)
+        return bad("memory tensor");
+    }
     if (u.rounds == 0) {
-      if (rank != (u.nvert ? 1 : 2)) return bad("leaf");
+      if (rank != (u.nvert ? 1 : 2) || u.next) return bad("leaf");
       continue;
     }
     if (u.item0 + (size_t)u.rounds * kUnitWaves > P.items.size()) return bad("items");
@@ -1145,7 +1212,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   }
   UnitBuilder U(s, lab, uni, prio, P);
   if (units) U.run();
-  auto inside = [&](int32_t x) { return units && U.in_unit[x] == 1; };
+  auto inside = [&](int32_t x) { return units && U.in_unit[x] == UnitBuilder::kInside; };
   // leaves are tensors 0..nl-1 (content is symmetric, so any layout works)
   for (int32_t i = 0; i < nl; i++) {
     if (inside(i)) {
@@ -1233,6 +1300,14 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
       if (inside(o)) continue;
       if (units && U.in_unit[o]) {
         B.layout[o] = has_req[o] ? req[o] : sorted_key(lab[o]);
+        if (U.in_unit[o] == UnitBuilder::kMixedUnit) {
+          const PUnit& u = P.units[U.unit_of(o)];
+          for (int q = 0; q < u.next; q++) {  // in the units' label order
+            const int32_t x = P.ext[u.ext0 + q].tensor;
+            req[x] = U.sorted[x];
+            has_req[x] = 1;
+          }
+        }
         continue;
       }
       cls[j] = classify(j);
@@ -1276,7 +1351,15 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     for (PUnit& u : P.units) U.set_layout(&u, B.layout[u.tensor]);
     for (int32_t j = 0; j < nn; j++) {
       const int o = nl + j;
-      if (units && U.in_unit[o]) continue;
+      if (units && U.in_unit[o]) {
+        if (U.in_unit[o] != UnitBuilder::kMixedUnit) continue;
+        POp op;
+        op.kind = kUnit;
+        op.c = o;
+        op.unit = U.unit_of(o);
+        P.ops.push_back(op);
+        continue;
+      }
       Cls& c = cls[j];
       if (is_gemm[j]) {
         int dst = o;
@@ -1364,10 +1447,18 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   // producers and levels
   const int nt = (int)P.tensors.size();
   std::vector<int> producer(nt, -1), consumer(nt, -1);
+  auto inputs = [&](const POp& op, auto f) {
+    if (op.kind == kUnit) {
+      const PUnit& u = P.units[op.unit];
+      for (int q = 0; q < u.next; q++) f(P.ext[u.ext0 + q].tensor);
+      return;
+    }
+    for (int in : {op.a, op.b})
+      if (in >= 0) f(in);
+  };
   for (size_t i = 0; i < P.ops.size(); i++) {
     producer[P.ops[i].c] = (int)i;
-    for (int in : {P.ops[i].a, P.ops[i].b})
-      if (in >= 0) consumer[in] = (int)i;
+    inputs(P.ops[i], [&](int in) { consumer[in] = (int)i; });
   }
   const int nops = (int)P.ops.size();
   if (opt.batched) {
@@ -1375,8 +1466,9 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     int H = 0;
     for (int i = 0; i < nops; i++) {
       int lv = 1;
-      for (int in : {P.ops[i].a, P.ops[i].b})
-        if (in >= 0 && producer[in] >= 0) lv = std::max(lv, asap[producer[in]] + 1);
+      inputs(P.ops[i], [&](int in) {
+        if (producer[in] >= 0) lv = std::max(lv, asap[producer[in]] + 1);
+      });
       asap[i] = lv;
       H = std::max(H, lv);
     }
@@ -1384,6 +1476,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     for (int i = nops - 1; i >= 0; i--) {
       int cons = consumer[P.ops[i].c];
       P.ops[i].level = cons < 0 ? H : P.ops[cons].level - 1;
+      if (P.ops[i].kind == kUnit) P.units[P.ops[i].unit].level = P.ops[i].level;
     }
     P.nlevels = H;
     for (int t = 0; t < nt; t++) {
@@ -1403,7 +1496,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
     // the arena holds no tensor from inside a unit, and no root a unit
     // writes as the slice's result
     for (int32_t x = 0; x < nl + nn; x++)
-      if (U.in_unit[x] == 1 || (P.unit_root && x == P.root)) P.tensors[x].bytes = 0;
+      if (inside(x) || (P.unit_root && x == P.root)) P.tensors[x].bytes = 0;
   }
   P.arena_bytes = assign_offsets(P.tensors);
   // never below the largest tensor of the tree, in LDS or not: callers size
@@ -1416,6 +1509,10 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   for (const auto& op : P.ops) {
     P.exec_macs += op.macs;
     P.exec_bytes += op.bytes;
+  }
+  for (const auto& u : P.units) {
+    P.exec_macs += u.macs;
+    P.exec_bytes += u.bytes;
   }
   return 0;
 }

@@ -30,11 +30,12 @@ struct PTensor {
   int birth = 0, death = 0;
 };
 
-enum OpKind { kEw = 0, kGemm = 1 };
+enum OpKind { kEw = 0, kGemm = 1, kUnit = 2 };
 
 struct POp {
   int kind = kEw;
   int a = -1, b = -1, c = -1;  // tensor ids (b = -1: unary)
+  int unit = -1;               // kUnit: its inputs are the unit's ext tensors
   int level = 0;               // wave (batched) or sequence index (plain)
   // EW: the step's descriptor with device addresses left 0 (set at launch)
   int nP = 0, nR = 0;
@@ -58,17 +59,25 @@ struct PLeaf {
   uint32_t wbits;
 };
 
-// A fused subtree (UnitDesc without addresses).
+// A fused part of the tree (UnitDesc without addresses).
 struct PUnit {
   int tensor = -1;        // output; kind and weight of a leaf as in UnitDesc
-  uint32_t item0 = 0, w0 = 0;  // into SlicePlan::items / unit_w
-  int rounds = 0, nvert = 0;
+  uint32_t item0 = 0, w0 = 0, ext0 = 0;  // into SlicePlan::items / unit_w / ext
+  int rounds = 0, nvert = 0, next = 0;
+  int level = 0;          // wave; 0: before every step (no ext)
+  double macs = 0, bytes = 0;  // of its steps, as POp
   uint64_t pos = 0;
 };
 
 // A step inside a unit (plan_steps, work accounting).
 struct PUnitStep {
   int8_t rank_a, rank_b, rank_c, n_reduced;
+  int32_t unit;
+};
+// A tensor a unit reads from memory.
+struct PExt {
+  int tensor;
+  uint32_t off;  // LDS element offset
 };
 
 struct SlicePlan {
@@ -76,8 +85,9 @@ struct SlicePlan {
   std::vector<PTensor> tensors;
   std::vector<POp> ops;  // in dependency order
   std::vector<PLeaf> leaves;  // plain plans only; batched: leaf units
-  // batched: the subtrees contracted in LDS, before level 1
+  // batched: the parts of the tree contracted in LDS
   std::vector<PUnit> units;
+  std::vector<PExt> ext;
   std::vector<UnitItem> items;
   std::vector<uint32_t> unit_w;  // vertex weights of the units
   std::vector<PUnitStep> unit_steps;

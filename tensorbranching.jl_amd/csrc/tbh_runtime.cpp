@@ -621,18 +621,23 @@ int ew_chunk(tbh_ctx* ctx, int64_t total) {
 // ------------------------------------------------------ BATCHED ----------
 namespace {
 
-// launch kinds: 0 direct EW, 1 tiled EW, 2 + s GEMM with tile shape s
-constexpr int kKinds = 5;
+// launch kinds: 0 direct EW, 1 tiled EW, 2 + s GEMM with tile shape s, 5 units
+constexpr int kKinds = 6, kUnitKind = 5;
 int op_kind(const POp& op) {
+  if (op.kind == kUnit) return kUnitKind;
   return op.kind == kGemm ? 2 + op.shape : (op.direct ? 0 : 1);
 }
 int64_t op_tiles(const POp& op) {
+  if (op.kind == kUnit) return 1;
   if (op.kind != kGemm) return op.tiles;
   const int sh = op.shape, bm = gemm_bm(sh), bn = gemm_bn(sh);
   return (int64_t)((op.M + bm - 1) / bm) * ((op.N + bn - 1) / bn) * op.batch;
 }
-size_t desc_size(int kind) { return kind >= 2 ? sizeof(GemmDesc) : sizeof(EwDesc); }
-int stat_kind(int kind) { return kind < 2 ? kind : 2; }  // tbh_stats: direct, tiled, GEMM
+size_t desc_size(int kind) {
+  return kind == kUnitKind ? sizeof(UnitDesc) : kind >= 2 ? sizeof(GemmDesc) : sizeof(EwDesc);
+}
+// tbh_stats: direct (and units), tiled, GEMM
+int stat_kind(int kind) { return kind == kUnitKind ? 0 : kind < 2 ? kind : 2; }
 
 }  // namespace
 
@@ -647,12 +652,12 @@ size_t desc_bytes(const SlicePlan& P) {
   // one-step prefix pair
   return P.ops.size() * (std::max(sizeof(EwDesc), sizeof(GemmDesc)) + 3 * sizeof(int64_t)) +
          P.units.size() * sizeof(UnitDesc) + P.items.size() * sizeof(UnitItem) +
-         P.unit_w.size() * sizeof(uint32_t) + sizeof(EpiDesc) + 4;
+         P.unit_w.size() * sizeof(uint32_t) + P.ext.size() * sizeof(UnitExt) + sizeof(EpiDesc) + 4;
 }
 
 size_t desc_batch_overhead(int levels) {
   const size_t slots = (size_t)kKinds * (size_t)(levels + 1);
-  return 256 * (5 + 3 * slots) + sizeof(int64_t) * slots;
+  return 256 * (6 + 3 * slots) + sizeof(int64_t) * slots;
 }
 
 namespace {
@@ -783,9 +788,9 @@ struct IssueJob {
   bool prof = false, per_step = false;
   int bidx = 0, H = 0;
   size_t nb = 0;
-  int64_t nunits = 0, nepi = 0;
+  int64_t nepi = 0;
   int unit_levels = 0;   // deepest unit
-  size_t o_units = 0, o_items = 0, o_w = 0, o_epi = 0, o_res = 0;
+  size_t o_items = 0, o_w = 0, o_ext = 0, o_epi = 0, o_res = 0;
   char* dbase = nullptr;     // the batch's descriptors on the device
   const char* hb = nullptr;  // ... and in the pinned staging buffer (step tags)
   hipEvent_t up = nullptr, done = nullptr;
@@ -818,17 +823,22 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
     return false;
   };
   if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, j.up, 0);
-  if (e == hipSuccess && j.nunits && injected(std::max(1, j.unit_levels)))
-    e = hipErrorLaunchFailure;
-  if (e == hipSuccess && j.nunits) {
-    hipEvent_t ev = prof ? ctx->prof.begin(ctx->stream) : nullptr;
-    e = launch_units(dtype, (const UnitDesc*)(dbase + j.o_units),
-                     (const UnitItem*)(dbase + j.o_items), (const uint32_t*)(dbase + j.o_w),
-                     j.nunits, dbase + j.o_res, ctx->stream);
-    if (prof) ctx->prof.end(ctx->stream, ev, 0, 0, (int)j.nunits, 0, 0, "units");
-    ctx->stats.launches++;
-  }
   hipEvent_t ev = nullptr;
+  // the units of level L (0: those that read no tensor from memory)
+  auto units = [&](int L) {
+    const int w = slot(kUnitKind, L);
+    if (!cnt[w]) return hipSuccess;
+    if (injected(L ? 1 : std::max(1, j.unit_levels))) return hipErrorLaunchFailure;
+    if (prof) ev = ctx->prof.begin(ctx->stream);
+    const hipError_t r =
+        launch_units(dtype, (const UnitDesc*)(dbase + j.o_desc[w]),
+                     (const UnitItem*)(dbase + j.o_items), (const uint32_t*)(dbase + j.o_w),
+                     (const UnitExt*)(dbase + j.o_ext), cnt[w], dbase + j.o_res, ctx->stream);
+    if (prof) ctx->prof.end(ctx->stream, ev, 0, L, cnt[w], j.lvl_bytes[w], j.lvl_macs[w], "units");
+    ctx->stats.launches++;
+    return r;
+  };
+  if (e == hipSuccess) e = units(0);
   // one launch per kernel kind and level (direct EW, tiled EW, GEMM); in
   // the per-step profiling mode every step alone, tagged with its shape
   // GEMM launches on a second stream beside a level's EW launches (not
@@ -878,13 +888,14 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
       // stream's work of earlier levels (both syncs before any launch)
       bool has[2] = {false, false};
       for (int k = 0; k < kKinds; k++)
-        if (cnt[slot(k, L)]) has[k >= 2 ? 1 : 0] = true;
+        if (cnt[slot(k, L)]) has[k >= 2 && k < kUnitKind ? 1 : 0] = true;
       if (has[0] && e == hipSuccess) e = sync_to(0);
       if (has[1] && e == hipSuccess) e = sync_to(1);
       if (has[0]) dirty[0] = true;
       if (has[1]) dirty[1] = true;
     }
-    for (int k = 0; k < kKinds && e == hipSuccess; k++) {
+    if (e == hipSuccess) e = units(L);
+    for (int k = 0; k < kUnitKind && e == hipSuccess; k++) {
       const int w = slot(k, L);
       if (!cnt[w]) continue;
       const int64_t total = pfx[w].back();
@@ -1039,9 +1050,9 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   std::vector<std::vector<int64_t>> pfx(W, std::vector<int64_t>(1, 0));
   std::vector<double> lvl_bytes(W, 0.0), lvl_macs(W, 0.0);
   std::vector<std::vector<std::pair<double, double>>> step_work(per_step ? W : 0);
-  // per slice: its first unit, item, vertex weight and epilogue entry
+  // per slice: its first item, vertex weight, memory tensor and epilogue entry
   struct Start {
-    int64_t unit = 0, item = 0, w = 0, epi = 0;
+    int64_t item = 0, w = 0, ext = 0, epi = 0;
   };
   std::vector<Start> first(nb + 1);
   int unit_levels = 0;
@@ -1051,13 +1062,20 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
     first[i + 1] = first[i];
     first[i + 1].epi += P.empty || !P.unit_root;
     if (P.empty) continue;
-    first[i + 1].unit += (int64_t)P.units.size();
+    first[i + 1].ext += (int64_t)P.ext.size();
     first[i + 1].item += (int64_t)P.items.size();
     first[i + 1].w += (int64_t)P.unit_w.size();
     unit_levels = std::max(unit_levels, P.unit_levels);
     ctx->stats.ew_ops += P.unit_steps.size();
-    for (const PUnitStep& st : P.unit_steps) ctx->stats.ew_ops_algo_bytes += unit_step_bytes(st);
+    for (const PUnit& u : P.units) {
+      const int w = slot(kUnitKind, u.level);
+      cnt[w]++;
+      lvl_bytes[w] += u.bytes;
+      lvl_macs[w] += u.macs;
+      ctx->stats.ew_ops_algo_bytes += u.bytes;
+    }
     for (const POp& op : P.ops) {
+      if (op.kind == kUnit) continue;
       const int w = slot(op_kind(op), op.level);
       cnt[w]++;
       pfx[w].push_back(pfx[w].back() + op_tiles(op));
@@ -1082,15 +1100,16 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
     off = o + bytes;
     return o;
   };
-  const size_t o_units = take((size_t)first[nb].unit * sizeof(UnitDesc));
   const size_t o_items = take((size_t)first[nb].item * sizeof(UnitItem));
   const size_t o_w = take((size_t)first[nb].w * sizeof(uint32_t));
+  const size_t o_ext = take((size_t)first[nb].ext * sizeof(UnitExt));
   const size_t o_epi = take((size_t)first[nb].epi * sizeof(EpiDesc));
   const size_t o_res = take(4 * nb);
   std::vector<size_t> o_desc(W), o_pfx(W), o_one(W);
   for (int w = 0; w < W; w++) {
     if (!cnt[w]) continue;
     o_desc[w] = take((size_t)cnt[w] * desc_size(w / (H + 1)));
+    if (w / (H + 1) == kUnitKind) continue;
     o_pfx[w] = take((size_t)(cnt[w] + 1) * sizeof(int64_t));
     if (per_step) o_one[w] = take((size_t)cnt[w] * 2 * sizeof(int64_t));
   }
@@ -1101,7 +1120,7 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   if (rc) return rc;
   char* hb = static_cast<char*>(stg.host);
   for (int w = 0; w < W; w++) {
-    if (!cnt[w]) continue;
+    if (!cnt[w] || w / (H + 1) == kUnitKind) continue;
     std::memcpy(hb + o_pfx[w], pfx[w].data(), pfx[w].size() * sizeof(int64_t));
     if (per_step) {
       int64_t* one = reinterpret_cast<int64_t*>(hb + o_one[w]);
@@ -1126,8 +1145,12 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
       std::memcpy(hb + o_epi + (size_t)first[i].epi * sizeof(EpiDesc), &e, sizeof e);
     }
     if (P.empty) return;
-    UnitDesc* ud = reinterpret_cast<UnitDesc*>(hb + o_units) + first[i].unit;
+    std::vector<int32_t>& loc = local[t];
+    std::fill(loc.begin(), loc.end(), 0);
+    const int32_t* st = &start[i * W];
     for (const PUnit& u : P.units) {
+      const int w = slot(kUnitKind, u.level);
+      UnitDesc* ud = reinterpret_cast<UnitDesc*>(hb + o_desc[w]) + st[w] + loc[w]++;
       const bool result = P.unit_root && u.tensor == P.root;
       ud->c = result ? 0 : b + (uint64_t)P.tensors[u.tensor].off;
       ud->item0 = (uint32_t)first[i].item + u.item0;
@@ -1136,8 +1159,16 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
       ud->nvert = u.nvert;
       ud->res = (int32_t)i;
       ud->rbits = (int32_t)rbits;
+      ud->ext0 = (uint32_t)first[i].ext + u.ext0;
+      ud->next = u.next;
       ud->pos = u.pos;
-      ud++;
+    }
+    UnitExt* ux = reinterpret_cast<UnitExt*>(hb + o_ext) + first[i].ext;
+    for (const PExt& x : P.ext) {
+      ux->p = b + (uint64_t)P.tensors[x.tensor].off;
+      ux->off = x.off;
+      ux->rank = (uint32_t)P.tensors[x.tensor].rank;
+      ux++;
     }
     if (!P.items.empty())
       std::memcpy(hb + o_items + (size_t)first[i].item * sizeof(UnitItem), P.items.data(),
@@ -1145,10 +1176,8 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
     if (!P.unit_w.empty())
       std::memcpy(hb + o_w + (size_t)first[i].w * sizeof(uint32_t), P.unit_w.data(),
                   P.unit_w.size() * sizeof(uint32_t));
-    std::vector<int32_t>& loc = local[t];
-    std::fill(loc.begin(), loc.end(), 0);
-    const int32_t* st = &start[i * W];
     for (const POp& op : P.ops) {
+      if (op.kind == kUnit) continue;
       const int k = op_kind(op), w = slot(k, op.level);
       const int32_t idx = st[w] + loc[w]++;
       if (k >= 2)
@@ -1197,10 +1226,9 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   job->bidx = bidx;
   job->H = H;
   job->nb = nb;
-  job->nunits = first[nb].unit;
   job->nepi = first[nb].epi;
   job->unit_levels = unit_levels;
-  job->o_units = o_units;
+  job->o_ext = o_ext;
   job->o_items = o_items;
   job->o_w = o_w;
   job->o_epi = o_epi;
@@ -2012,13 +2040,15 @@ int tbh_plan_steps(const tbh_slice* slice, tbh_dtype dtype, tbh_mode mode, tbh_s
     set_error(err);
     return TBH_EINVAL;
   }
-  // the units' steps are wave 1, the other steps' waves follow
-  const int nu = (int)P.unit_steps.size(), n = nu + (int)P.ops.size();
+  // the units that read no tensor from memory are wave 1, the other steps'
+  // waves follow
+  const int nu = (int)P.unit_steps.size();
+  int n = nu;
   for (int i = 0; i < nu && i < cap; i++) {
     const PUnitStep& u = P.unit_steps[i];
     tbh_step_info& s = out[i];
     std::memset(&s, 0, sizeof s);
-    s.level = 1;
+    s.level = P.units[u.unit].level + 1;
     s.rank_a = u.rank_a;
     s.rank_b = u.rank_b;
     s.rank_c = u.rank_c;
@@ -2026,8 +2056,10 @@ int tbh_plan_steps(const tbh_slice* slice, tbh_dtype dtype, tbh_mode mode, tbh_s
     s.macs = std::ldexp(1.0, u.rank_c + u.n_reduced);
     s.bytes = unit_step_bytes(u);
   }
-  for (int i = nu; i < n && i < cap; i++) {
-    const POp& op = P.ops[i - nu];
+  for (const POp& op : P.ops) {
+    if (op.kind == kUnit) continue;
+    const int i = n++;
+    if (i >= cap) continue;
     tbh_step_info& s = out[i];
     std::memset(&s, 0, sizeof s);
     s.kind = op.kind;

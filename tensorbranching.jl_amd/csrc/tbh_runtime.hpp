@@ -33,7 +33,7 @@ hipError_t launch_gemm_ksplit(int dtype, const GemmSplit& g, hipStream_t s);  //
 hipError_t launch_leaves(int dtype, const LeafDesc* leaves, int64_t n, hipStream_t s);
 hipError_t launch_epilogue(int dtype, const EpiDesc* e, int64_t n, void* out, hipStream_t s);
 hipError_t launch_units(int dtype, const UnitDesc* units, const UnitItem* items,
-                        const uint32_t* weights, int64_t n, void* results,
+                        const uint32_t* weights, const UnitExt* ext, int64_t n, void* results,
                         hipStream_t s);  // tbh_unit.hip
 hipError_t launch_valu_probe(int dtype, void* out, int blocks, int iters, hipStream_t s);
 // resident tiled-EW workgroups per CU (LDS and registers), from the runtime

@@ -1,5 +1,5 @@
-// tbh_unit.hip -- K4 tbh_unit_kernel: a subtree of a slice's contraction tree
-// in one workgroup, every tensor but its output in LDS.
+// tbh_unit.hip -- K4 tbh_unit_kernel: a connected part of a slice's contraction
+// tree in one workgroup, every tensor but its output in LDS.
 //
 // What bounds it: the chain of a unit's levels (10-30 of them), each a few
 // LDS reads and a barrier; its arithmetic (at most 2^17 MACs) and bytes (16
@@ -48,8 +48,9 @@ __device__ __forceinline__ uint32_t lane_read(uint32_t v, uint32_t lane) {
 template <typename T>
 __global__ __launch_bounds__(64 * kUnitWaves) void tbh_unit_kernel(
     const UnitDesc* __restrict__ units, const uint4* __restrict__ items,
-    const uint32_t* __restrict__ weights, T* __restrict__ results) {
-  __shared__ T lds[kUnitLds];
+    const uint32_t* __restrict__ weights, const UnitExt* __restrict__ ext,
+    T* __restrict__ results) {
+  __shared__ __align__(16) T lds[kUnitLds];
   const UnitDesc& u = units[blockIdx.x];
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -69,11 +70,21 @@ __global__ __launch_bounds__(64 * kUnitWaves) void tbh_unit_kernel(
   // reaches scalar registers by a lane read, with no memory access
   const uint4* my = items + u.item0 + wave * rounds;
   uint4 held = (int)lane < rounds ? my[lane] : uint4{0, 0, 0, 0};
+  // tensors from memory straight to LDS, all in flight at once
+  for (int q = 0; q < u.next; q++) {
+    const UnitExt x = ext[u.ext0 + q];
+    const TBH_GLOBAL T* X = reinterpret_cast<const TBH_GLOBAL T*>(x.p);
+    const uint32_t n = 1u << x.rank;
+    for (uint32_t i = wave * 64; i < n; i += 64 * kUnitWaves)
+      if (i + lane < n)
+        __builtin_amdgcn_global_load_lds(X + i + lane, (TBH_LDS T*)lds + x.off + i, 4, 0, 0);
+  }
   if (tid < 4) lds[tid] = tid == 3 ? pad_zero<T>() : Trop<T>::one();
   for (int i = tid; i < u.nvert; i += 64 * kUnitWaves) {
     lds[4 + 2 * i] = Trop<T>::one();
     lds[5 + 2 * i] = __builtin_bit_cast(T, w[i]);
   }
+  __builtin_amdgcn_s_waitcnt(0);  // the copies to LDS (a barrier does not wait for them)
   __syncthreads();
   for (int r = 0; r < rounds; r++) {
     if (r && (r & 63) == 0) held = r + (int)lane < rounds ? my[r + lane] : uint4{0, 0, 0, 0};
@@ -145,14 +156,15 @@ __global__ __launch_bounds__(64 * kUnitWaves) void tbh_unit_kernel(
 }
 
 hipError_t launch_units(int dtype, const UnitDesc* units, const UnitItem* items,
-                        const uint32_t* weights, int64_t n, void* results, hipStream_t s) {
+                        const uint32_t* weights, const UnitExt* ext, int64_t n, void* results,
+                        hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const uint4* it = reinterpret_cast<const uint4*>(items);
   if (dtype == 0)
-    tbh_unit_kernel<float><<<(int)n, 64 * kUnitWaves, 0, s>>>(units, it, weights,
+    tbh_unit_kernel<float><<<(int)n, 64 * kUnitWaves, 0, s>>>(units, it, weights, ext,
                                                               static_cast<float*>(results));
   else
-    tbh_unit_kernel<int32_t><<<(int)n, 64 * kUnitWaves, 0, s>>>(units, it, weights,
+    tbh_unit_kernel<int32_t><<<(int)n, 64 * kUnitWaves, 0, s>>>(units, it, weights, ext,
                                                                 static_cast<int32_t*>(results));
   return hipGetLastError();
 }

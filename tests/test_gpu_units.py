@@ -2,7 +2,8 @@
 the oracle, bit for bit.  Random pairings of a graph's leaves give trees whose
 nodes reach and pass every limit of a unit: 15 union labels, 14 output labels,
 6 reduced labels, 2^17 MACs and 8192 LDS elements, so that slices come out as
-one unit, as many units below GEMM and EW steps, and as leaves read by them."""
+one unit, as many units below and above larger steps (which then read tensors from
+memory), and as leaves read by those steps."""
 import numpy as np
 import pytest
 
@@ -43,6 +44,12 @@ def test_random_trees(tb, orc, backend, nv, degree, local, dtype):
         w = rng.integers(1, 101, nv).astype(dtype)
         branches.append(tb.SlicedBranch(tb.MISProblem(g, w), _random_code(tb, g, rng, local),
                                         int(rng.integers(0, 9))))
+    if nv in (17, 19):
+        # units above larger steps: unit steps (no tile) past the first wave
+        steps = [st for b in branches for st in tb.plan_steps(b, dtype)]
+        assert any(st["kind"] == 0 and st["level"] > 1 and st["rank_c"] > 0 and
+                   st["tile_bits"] == 0 for st in steps)
+        assert any(st["tile_bits"] > 0 for st in steps)
     print(f"[units] nv={nv} sc={[int(tb.sc(b)) for b in branches if len(b.code.tree)]}",
           flush=True)
     assert np.array_equal(backend.contract_slices(branches, dtype),
