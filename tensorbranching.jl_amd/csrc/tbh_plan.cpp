@@ -67,41 +67,72 @@ int validate(const SliceIn& s, std::string* err) {
   return 0;
 }
 
+// The labels of one tensor.
+struct Labels {
+  const int32_t* p;
+  int32_t n;
+  const int32_t* begin() const { return p; }
+  const int32_t* end() const { return p + n; }
+  size_t size() const { return (size_t)n; }
+  int32_t operator[](size_t i) const { return p[i]; }
+  operator std::vector<int32_t>() const { return std::vector<int32_t>(p, p + n); }
+};
+
+// The labels of every tensor of a tree (leaves, then internal nodes), end to
+// end: one allocation where a vector per tensor took most of a slice's
+// planning time.
+struct LabelSets {
+  std::vector<int32_t> off, lab;
+  Labels operator[](int32_t x) const { return {lab.data() + off[x], off[x + 1] - off[x]}; }
+};
+
 // labels of leaves then internal nodes, each in first-appearance order;
-// uni[j]: labels of internal node j's two children together
-void compute_labels(const SliceIn& s, std::vector<std::vector<int32_t>>& lab,
-                    std::vector<int32_t>* uni = nullptr) {
-  int32_t nl = s.nleaves, nn = std::max(0, nl - 1);
-  lab.assign(nl + nn, {});
+// uni[j]: labels of internal node j's two children together; elim[l]: the
+// internal node at which label l disappears (their number: never)
+void compute_labels(const SliceIn& s, LabelSets& L, std::vector<int32_t>* uni = nullptr,
+                    std::vector<int32_t>* elim = nullptr) {
+  const int32_t nl = s.nleaves, nn = std::max(0, nl - 1);
+  L.off.resize(nl + nn + 1);
+  L.lab.resize(s.ix_ptr[nl]);
+  std::vector<int32_t> cnt(s.ix_ptr[nl], 1);  // occurrences of a label below its tensor
   if (uni) uni->assign(nn, 0);
-  std::vector<std::vector<int32_t>> cnt(nl + nn);
+  if (elim) elim->assign(std::max(1, s.nv), nn);
   std::vector<int32_t> total(std::max(1, s.nv), 0), acc(std::max(1, s.nv), 0);
-  for (int32_t i = 0; i < nl; i++)
-    for (int32_t k = s.ix_ptr[i]; k < s.ix_ptr[i + 1]; k++) {
-      lab[i].push_back(s.ix[k]);
-      cnt[i].push_back(1);
-      total[s.ix[k]]++;
-    }
+  for (int32_t k = 0; k < s.ix_ptr[nl]; k++) {
+    L.lab[k] = s.ix[k];
+    total[s.ix[k]]++;
+  }
+  for (int32_t i = 0; i <= nl; i++) L.off[i] = s.ix_ptr[i];
   for (int32_t j = 0; j < nn; j++) {
-    int32_t a = s.tree[2 * j], b = s.tree[2 * j + 1], o = nl + j;
-    for (int32_t c : {a, b})
-      for (size_t k = 0; k < lab[c].size(); k++) acc[lab[c][k]] += cnt[c][k];
-    for (int32_t c : {a, b})
-      for (size_t k = 0; k < lab[c].size(); k++) {
-        int32_t l = lab[c][k];
-        if (acc[l] > 0) {
-          if (uni) (*uni)[j]++;
-          if (acc[l] < total[l]) {
-            lab[o].push_back(l);
-            cnt[o].push_back(acc[l]);
-          }
-          acc[l] = 0;
+    const int32_t ab[2] = {s.tree[2 * j], s.tree[2 * j + 1]};
+    int32_t top = L.off[nl + j];
+    const int32_t most = top + L.off[ab[0] + 1] - L.off[ab[0]] + L.off[ab[1] + 1] - L.off[ab[1]];
+    if ((int32_t)L.lab.size() < most) {
+      const size_t grow = std::max<size_t>(most, 2 * L.lab.size());
+      L.lab.resize(grow);
+      cnt.resize(grow);
+    }
+    for (int32_t c : ab)
+      for (int32_t k = L.off[c]; k < L.off[c + 1]; k++) acc[L.lab[k]] += cnt[k];
+    for (int32_t c : ab)
+      for (int32_t k = L.off[c]; k < L.off[c + 1]; k++) {
+        const int32_t l = L.lab[k], n = acc[l];
+        if (n == 0) continue;
+        if (uni) (*uni)[j]++;
+        if (n < total[l]) {
+          L.lab[top] = l;
+          cnt[top++] = n;
+        } else if (elim) {
+          (*elim)[l] = j;
         }
+        acc[l] = 0;
       }
+    L.off[nl + j + 1] = top;
   }
 }
 
-int pos_in(const std::vector<int32_t>& v, int32_t x) {
+template <class V>
+int pos_in(const V& v, int32_t x) {
   for (size_t i = 0; i < v.size(); i++)
     if (v[i] == x) return (int)i;
   return -1;
@@ -470,8 +501,14 @@ int gemm_split(const PlanOptions& opt, int na, int nb, int nk, int nt) {
 // Interval reuse of arena blocks: blocks freed by tensors that died at a level
 // strictly below a tensor's birth may be reused by it (exact size classes).
 int64_t assign_offsets(std::vector<PTensor>& T) {
-  std::vector<int> idx(T.size());
-  std::iota(idx.begin(), idx.end(), 0);
+  std::vector<int> idx;  // tensors in memory (bytes 0: inside a unit)
+  idx.reserve(T.size());
+  for (size_t t = 0; t < T.size(); t++) {
+    if (T[t].bytes == 0)
+      T[t].off = 0;
+    else
+      idx.push_back((int)t);
+  }
   std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) { return T[x].birth < T[y].birth; });
   std::vector<int> by_death(idx);
   std::stable_sort(by_death.begin(), by_death.end(),
@@ -480,13 +517,9 @@ int64_t assign_offsets(std::vector<PTensor>& T) {
   int64_t top = 0;
   size_t di = 0;
   for (int t : idx) {
-    if (T[t].bytes == 0) {  // lives in LDS
-      T[t].off = 0;
-      continue;
-    }
     while (di < by_death.size() && T[by_death[di]].death < T[t].birth) {
       const PTensor& d = T[by_death[di]];
-      if (d.off >= 0 && d.bytes > 0) freel[std::max<int64_t>(d.bytes, 16)].push_back(d.off);
+      if (d.off >= 0) freel[std::max<int64_t>(d.bytes, 16)].push_back(d.off);
       di++;
     }
     int64_t cls = std::max<int64_t>(T[t].bytes, 16);
@@ -510,6 +543,7 @@ int64_t assign_offsets(std::vector<PTensor>& T) {
 int verify_plan(const SlicePlan& P, std::string* err) {
   auto bad = [&](const std::string& m) { return fail(err, "plan check: " + m); };
   for (const auto& t : P.tensors) {
+    if (t.bytes == 0) continue;  // inside a unit
     if (t.off < 0 || t.off % 16 || t.off + std::max<int64_t>(t.bytes, 16) > P.arena_bytes)
       return bad("tensor outside the arena");
     if (t.rank < 0 || t.rank > kMaxRank) return bad("rank");
@@ -647,28 +681,36 @@ int verify_plan(const SlicePlan& P, std::string* err) {
 // the contraction is order-invariant), which the tests check against the
 // unmodified tree; non-integer Float32 sums regrouped this way may differ by
 // a rounding step.
-void reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree,
-                 const std::vector<std::vector<int32_t>>& lab0, const PlanOptions& opt) {
+// Returns whether it changed the tree.
+bool reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree, const LabelSets& lab0,
+                 const PlanOptions& opt) {
   const int32_t nn = nl - 1;
-  if (nn < 3) return;
+  if (nn < 3) return false;
+  // a rotation needs two spine tensors of chain_big labels, one above the other
+  bool any = false;
+  for (int32_t j = 0; j < nn && !any; j++)
+    any = (int)lab0[nl + j].size() >= opt.chain_big;
+  if (!any) return false;
   const int W = (nv + 63) / 64;
   const int tot = nl + nn;
-  std::vector<uint64_t> L((size_t)tot * W, 0);
-  auto Lp = [&](int x) { return &L[(size_t)x * W]; };
-  for (int x = 0; x < tot; x++)
+  // label sets as bits, filled for the few nodes a rotation looks at
+  std::vector<int32_t> row(tot, -1);
+  std::vector<uint64_t> bits;
+  auto Lp = [&](int x) { return &bits[(size_t)row[x] * W]; };
+  auto fill = [&](int x) {
+    if (row[x] >= 0) return;
+    row[x] = (int32_t)(bits.size() / W);
+    bits.resize(bits.size() + W, 0);
     for (int32_t l : lab0[x]) Lp(x)[l >> 6] |= 1ull << (l & 63);
-  auto rank = [&](int x) {
-    int c = 0;
-    for (int i = 0; i < W; i++) c += __builtin_popcountll(Lp(x)[i]);
-    return c;
   };
   std::vector<int32_t> lc(tot, -1), rc(tot, -1), rk(tot, 0);
-  for (int x = 0; x < tot; x++) rk[x] = rank(x);
+  for (int x = 0; x < tot; x++) rk[x] = (int32_t)lab0[x].size();
   for (int32_t j = 0; j < nn; j++) {
     lc[nl + j] = tree[2 * j];
     rc[nl + j] = tree[2 * j + 1];
   }
   std::vector<uint64_t> F(W);
+  bool changed = false;
   // a combined side tensor must never count as big (F <= side < big), so each
   // rotation moves one node down the spine and the loop ends
   const int side = std::min(opt.chain_side, opt.chain_big - 1);
@@ -681,6 +723,7 @@ void reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree,
       int Yp = rk[lc[Y]] >= rk[rc[Y]] ? lc[Y] : rc[Y];
       int Sp = Yp == lc[Y] ? rc[Y] : lc[Y];
       if (rk[Yp] < opt.chain_big || rk[Sp] > side) break;
+      for (int q : {x, Y, S, Yp, Sp}) fill(q);
       int rf = 0, nred = 0, u_ys = 0, u_x = 0, u_f = 0, u_new = 0;
       for (int i = 0; i < W; i++) {
         F[i] = (Lp(Sp)[i] | Lp(S)[i]) & (Lp(Yp)[i] | Lp(x)[i]);
@@ -708,6 +751,7 @@ void reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree,
         break;
       }
       // node Y becomes F = (S', S); x = (Y', F)
+      changed = true;
       lc[Y] = Sp;
       rc[Y] = S;
       std::copy(F.begin(), F.end(), Lp(Y));
@@ -716,6 +760,7 @@ void reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree,
       rc[x] = Y;
     }
   }
+  if (!changed) return false;
   // serialise in post-order again
   std::vector<int32_t> id(tot, -1);
   for (int i = 0; i < nl; i++) id[i] = i;
@@ -739,6 +784,7 @@ void reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree,
     }
   }
   tree.swap(out);
+  return true;
 }
 
 // ---- units: subtrees contracted in LDS (UnitDesc) -----------------------
@@ -748,9 +794,10 @@ void reassociate(int32_t nl, int32_t nv, std::vector<int32_t>& tree,
 // King's-subgraph trees are in one of a slice's 15-40 units.
 struct UnitBuilder {
   const SliceIn& s;
-  const std::vector<std::vector<int32_t>>& lab;
+  const LabelSets& lab;
   const std::vector<int32_t>& uni;
-  const std::vector<int32_t>& prio;  // label -> place in the order of all labels
+  const std::vector<int32_t>& prio;   // label -> place in the order of all labels
+  const std::vector<int32_t>& order;  // ... and its inverse
   SlicePlan& P;
   int32_t nl;
   // log2 of a unit's MACs at most: 4 waves take about 5 us for 2^17
@@ -764,13 +811,30 @@ struct UnitBuilder {
   std::vector<char> small;           // the node's step alone may be in a unit
   std::vector<int32_t> parent, level, node_at, vert, taken;
   std::vector<int32_t> off;          // LDS offset of a unit's tensor
-  std::vector<std::vector<int32_t>> sorted;  // labels of a unit's tensors, by prio
+  // the places of the labels of a unit's tensors, ascending, 16 per tree node
+  std::vector<int32_t> place;
+  // scratch of build()
+  std::vector<int32_t> verts, freeb[kUnitBits + 1];
+  std::vector<UnitItem> wave[kUnitWaves];
 
-  UnitBuilder(const SliceIn& s_, const std::vector<std::vector<int32_t>>& lab_,
-              const std::vector<int32_t>& uni_, const std::vector<int32_t>& prio_, SlicePlan& P_)
-      : s(s_), lab(lab_), uni(uni_), prio(prio_), P(P_), nl(s_.nleaves) {}
+  UnitBuilder(const SliceIn& s_, const LabelSets& lab_, const std::vector<int32_t>& uni_,
+              const std::vector<int32_t>& prio_, const std::vector<int32_t>& order_,
+              SlicePlan& P_)
+      : s(s_), lab(lab_), uni(uni_), prio(prio_), order(order_), P(P_), nl(s_.nleaves) {}
 
-  int rank(int32_t x) const { return (int)lab[x].size(); }
+  int rank(int32_t x) const { return lab.off[x + 1] - lab.off[x]; }
+  int32_t* places(int32_t x) { return &place[16 * (size_t)x]; }
+  // a tensor's places from its labels (at most 14 of them)
+  void set_places(int32_t x) {
+    int32_t* p = places(x);
+    int n = 0;
+    for (int32_t l : lab[x]) {
+      const int32_t v = prio[l];
+      int k = n++;
+      for (; k > 0 && p[k - 1] > v; k--) p[k] = p[k - 1];
+      p[k] = v;
+    }
+  }
 
   // which internal nodes may be inside a unit
   void mark() {
@@ -782,7 +846,10 @@ struct UnitBuilder {
     level.assign(tot, 0);
     off.assign(tot, 0);
     vert.assign(nl, -1);
-    sorted.resize(tot);
+    place.resize(16 * (size_t)tot);
+    P.items.reserve(3 * (size_t)tot);
+    P.unit_steps.reserve(nn);
+    P.unit_w.reserve(nl);
     std::vector<int64_t> peak(tot, 0);
     std::vector<double> macs(tot, 0.0);
     for (int32_t i = 0; i < nl; i++) fit[i] = 1;
@@ -797,7 +864,7 @@ struct UnitBuilder {
       const int64_t first = std::max(peak[x], peak[y]);
       const int64_t second = peak[x] >= peak[y] ? sx + peak[y] : sy + peak[x];
       peak[o] = std::max(std::max(first, second), sx + sy + so);
-      macs[o] = macs[x] + macs[y] + std::ldexp(1.0, uni[j]);
+      macs[o] = macs[x] + macs[y] + (uni[j] < 31 ? (double)(1u << uni[j]) : 1e18);
       small[o] = uni[j] <= kUnitBits && rank(o) <= kUnitRank &&
                  uni[j] - rank(o) <= kUnitReduce && rank(x) <= kUnitOperand &&
                  rank(y) <= kUnitOperand;
@@ -822,11 +889,11 @@ struct UnitBuilder {
     node_at.push_back(root);
     level[root] = 0;
     int depth = 0, nvert = 0;
-    std::vector<int32_t> verts;
+    verts.clear();
     for (size_t k = 0; k < node_at.size(); k++) {
       const int32_t o = node_at[k], j = o - nl;
       if (external(o)) continue;
-      work += std::ldexp(1.0, uni[j]);
+      work += (double)(1u << uni[j]);
       for (int q = 0; q < 2; q++) {
         const int32_t c = s.tree[2 * j + q];
         if (c < nl) {
@@ -853,7 +920,7 @@ struct UnitBuilder {
           top += 1 << rank(o);
           if (top > kUnitLds) return false;
         }
-    std::vector<int32_t> freeb[kUnitBits + 1];
+    for (auto& f : freeb) f.clear();
     size_t dead = node_at.size();  // node_at[dead..]: tensors already released
     for (size_t k = node_at.size(); k-- > 1;) {
       const int32_t o = node_at[k];
@@ -889,16 +956,14 @@ struct UnitBuilder {
       for (int32_t o : node_at)
         if (external(o)) {
           P.ext.push_back({o, (uint32_t)off[o]});
-          sorted[o].assign(lab[o].begin(), lab[o].end());
-          std::sort(sorted[o].begin(), sorted[o].end(),
-                    [&](int32_t p, int32_t q) { return prio[p] < prio[q]; });
+          set_places(o);
           u.next++;
         }
     for (int32_t c : verts) {
       const int32_t v = lab[c][0];
       P.unit_w.push_back(s.wbits ? s.wbits[v] : s.unit_wbits);
     }
-    std::vector<UnitItem> wave[kUnitWaves];
+    for (auto& w : wave) w.clear();
     int next = 0;
     size_t k = node_at.size();
     while (k > 0) {
@@ -908,25 +973,19 @@ struct UnitBuilder {
         if (external(o)) continue;
         const int32_t x = s.tree[2 * j], y = s.tree[2 * j + 1];
         for (int32_t c : {x, y})
-          if (c < nl) {
-            sorted[c] = lab[c];
-            if (sorted[c].size() == 2 && prio[sorted[c][0]] > prio[sorted[c][1]])
-              std::swap(sorted[c][0], sorted[c][1]);
-          }
-        const auto &LX = sorted[x], &LY = sorted[y];
-        auto& LO = sorted[o];
-        LO.clear();
+          if (c < nl) set_places(c);
+        const int32_t *px = places(x), *py = places(y);
+        int32_t* po = places(o);
         UnitItem it{};
+        const int nP = rank(o), rx = rank(x), ry = rank(y);
         int n = 0;
-        for (size_t a = 0, b = 0; a < LX.size() || b < LY.size(); n++) {
-          const int pa = a < LX.size() ? prio[LX[a]] : INT32_MAX;
-          const int pb = b < LY.size() ? prio[LY[b]] : INT32_MAX;
-          LO.push_back(pa <= pb ? LX[a] : LY[b]);
-          if (pa <= pb) it.mA |= (uint16_t)(1u << n), a++;
-          if (pb <= pa) it.mB |= (uint16_t)(1u << n), b++;
+        for (int a = 0, b = 0; a < rx || b < ry; n++) {
+          const int32_t va = a < rx ? px[a] : INT32_MAX, vb = b < ry ? py[b] : INT32_MAX;
+          po[n] = va <= vb ? va : vb;  // (at most 15 labels in a union)
+          if (va <= vb) it.mA |= (uint16_t)(1u << n), a++;
+          if (vb <= va) it.mB |= (uint16_t)(1u << n), b++;
         }
-        const int nP = rank(o), nR = n - nP;
-        LO.resize(nP);
+        const int nR = n - nP;
         auto lds_of = [&](int32_t c) {
           return c >= nl ? off[c] : vert[c] >= 0 && rank(c) == 1 ? 4 + 2 * vert[c] : 0;
         };
@@ -1020,8 +1079,9 @@ struct UnitBuilder {
   // output bit -> position in the layout its consumer reads
   void set_layout(PUnit* u, const std::vector<int32_t>& lay) {
     if (u->rounds == 0) return;  // a leaf: its content is symmetric
-    const auto& L = sorted[u->tensor];
-    for (size_t k = 0; k < L.size(); k++) u->pos |= (uint64_t)(pos_in(lay, L[k]) & 15) << (4 * k);
+    const int32_t* p = places(u->tensor);
+    for (int k = 0; k < rank(u->tensor); k++)
+      u->pos |= (uint64_t)(pos_in(lay, order[p[k]]) & 15) << (4 * k);
   }
 };
 
@@ -1082,12 +1142,6 @@ int verify_units(const SlicePlan& P, std::string* err) {
 
 }  // namespace
 
-int slice_labels(const SliceIn& s, std::vector<std::vector<int32_t>>* labels, std::string* err) {
-  if (validate(s, err)) return -1;
-  compute_labels(s, *labels);
-  return 0;
-}
-
 int slice_complexity(const SliceIn& s, double* tc, double* sc, double* rwc, std::string* err) {
   if (validate(s, err)) return -1;
   if (s.nleaves < 2) {
@@ -1096,13 +1150,13 @@ int slice_complexity(const SliceIn& s, double* tc, double* sc, double* rwc, std:
     *rwc = -INFINITY;
     return 0;
   }
-  std::vector<std::vector<int32_t>> lab;
+  LabelSets lab;
   compute_labels(s, lab);
   double t = 0, rw = 0;
   size_t scm = 0;
   std::vector<char> mark(std::max(1, s.nv), 0);
   for (int32_t j = 0; j + 1 < s.nleaves; j++) {
-    const auto &A = lab[s.tree[2 * j]], &B = lab[s.tree[2 * j + 1]], &C = lab[s.nleaves + j];
+    const Labels A = lab[s.tree[2 * j]], B = lab[s.tree[2 * j + 1]], C = lab[s.nleaves + j];
     int u = 0;
     for (int32_t l : A) mark[l] = 1, u++;
     for (int32_t l : B)
@@ -1126,7 +1180,7 @@ int slice_peak_memory(const SliceIn& s, double* peak, double* all, std::string* 
     *all = -INFINITY;
     return 0;
   }
-  std::vector<std::vector<int32_t>> lab;
+  LabelSets lab;
   compute_labels(s, lab);
   int32_t nl = s.nleaves, nn = nl - 1;
   double cur = 0;
@@ -1163,27 +1217,20 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   SliceIn s = s_in;
   const int32_t nl = s.nleaves, nn = nl - 1;
   P.n_leaves = nl;
-  std::vector<std::vector<int32_t>> lab;
-  std::vector<int32_t> uni;
-  compute_labels(s, lab, &uni);
+  LabelSets lab;
+  std::vector<int32_t> uni, elim;
+  compute_labels(s, lab, &uni, &elim);
   // tree-node contraction count of the given tree (the reference's tc)
   for (int32_t j = 0; j < nn; j++) P.node_macs += std::ldexp(1.0, uni[j]);
   std::vector<int32_t> tree2;
   if (opt.batched && opt.reassociate && nn >= 3 && !std::getenv("TBH_NO_REASSOCIATE")) {
     tree2.assign(s.tree, s.tree + 2 * (size_t)nn);
-    reassociate(nl, s.nv, tree2, lab, opt);
-    s.tree = tree2.data();
-    compute_labels(s, lab, &uni);
+    if (reassociate(nl, s.nv, tree2, lab, opt)) {
+      s.tree = tree2.data();
+      compute_labels(s, lab, &uni, &elim);
+    }
   }
 
-  // elimination step of each label (node index where it disappears)
-  std::vector<int32_t> elim(s.nv, nn);
-  for (int32_t j = 0; j < nn; j++) {
-    const auto &A = lab[s.tree[2 * j]], &B = lab[s.tree[2 * j + 1]], &C = lab[nl + j];
-    for (const auto* X : {&A, &B})
-      for (int32_t l : *X)
-        if (pos_in(C, l) < 0) elim[l] = j;
-  }
   auto sorted_key = [&](std::vector<int32_t> v) {
     std::sort(v.begin(), v.end(), [&](int32_t x, int32_t y) {
       return elim[x] != elim[y] ? elim[x] > elim[y] : x < y;
@@ -1195,31 +1242,42 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   B.posA_.assign(std::max(1, s.nv), -1);
   B.posB_.assign(std::max(1, s.nv), -1);
   B.posC_.assign(std::max(1, s.nv), -1);
-  // a node becomes up to three steps (permutes, split-K reductions)
-  P.ops.reserve(3 * (size_t)nn + 4);
-  P.tensors.reserve(3 * (size_t)(nl + nn) + 4);
-  B.layout.reserve(3 * (size_t)(nl + nn) + 4);
   // batched: the subtrees that run as units; a single leaf, and every leaf
   // and step outside them, as below
-  std::vector<int32_t> prio;
+  std::vector<int32_t> prio, order;
   const bool units = opt.batched && opt.units;
   if (units) {
-    std::vector<int32_t> all(s.nv);
-    std::iota(all.begin(), all.end(), 0);
-    all = sorted_key(all);
+    // every label by sorted_key's rule (elimination nodes are 0 .. nn:
+    // counted, not compared)
+    order.resize(s.nv);
     prio.resize(s.nv);
-    for (int32_t k = 0; k < s.nv; k++) prio[all[k]] = k;
+    std::vector<int32_t> at(nn + 2, 0);
+    for (int32_t l = 0; l < s.nv; l++) at[nn - elim[l] + 1]++;
+    for (int32_t k = 0; k <= nn; k++) at[k + 1] += at[k];
+    for (int32_t l = 0; l < s.nv; l++) {
+      prio[l] = at[nn - elim[l]]++;
+      order[prio[l]] = l;
+    }
   }
-  UnitBuilder U(s, lab, uni, prio, P);
+  UnitBuilder U(s, lab, uni, prio, order, P);
   if (units) U.run();
   auto inside = [&](int32_t x) { return units && U.in_unit[x] == UnitBuilder::kInside; };
+  // the nodes outside units, and their places among them
+  std::vector<int32_t> step_of(nn, -1);
+  int32_t nsteps = 0;
+  for (int32_t j = 0; j < nn; j++)
+    if (!units || !U.in_unit[nl + j]) step_of[j] = nsteps++;
+  // a node becomes up to three steps (permutes, split-K reductions)
+  P.ops.reserve(3 * (size_t)nsteps + P.units.size() + 4);
+  P.tensors.reserve((size_t)(nl + nn) + 3 * (size_t)nsteps + 4);
+  B.layout.reserve((size_t)(nl + nn) + 3 * (size_t)nsteps + 4);
   // leaves are tensors 0..nl-1 (content is symmetric, so any layout works)
   for (int32_t i = 0; i < nl; i++) {
     if (inside(i)) {
       B.add_tensor({});
       continue;
     }
-    B.add_tensor(opt.batched ? sorted_key(lab[i]) : lab[i]);
+    B.add_tensor(opt.batched ? sorted_key(lab[i]) : std::vector<int32_t>(lab[i]));
     if (units) continue;
     PLeaf L;
     L.tensor = i;
@@ -1233,7 +1291,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   }
   // internal node output tensors nl..nl+nn-1 (layouts fixed below)
   for (int32_t j = 0; j < nn; j++)
-    B.add_tensor(inside(nl + j) ? std::vector<int32_t>() : lab[nl + j]);
+    B.add_tensor(inside(nl + j) ? std::vector<int32_t>() : std::vector<int32_t>(lab[nl + j]));
 
   // classify labels of node j
   struct Cls {
@@ -1244,7 +1302,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   auto classify = [&](int32_t j) {
     Cls c;
     int32_t x = s.tree[2 * j], y = s.tree[2 * j + 1];
-    const auto &LX = lab[x], &LY = lab[y], &LC = lab[nl + j];
+    const Labels LX = lab[x], LY = lab[y], LC = lab[nl + j];
     std::vector<int32_t> fx, fy;
     fx.reserve(LC.size());
     fy.reserve(LC.size());
@@ -1290,11 +1348,11 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   if (opt.batched) {
     // top-down layout requests; GEMM-shaped nodes ask their children for
     // (a,k,t) / (k,b,t) and write (a,b,t)
-    std::vector<char> is_gemm(nn, 0), has_req(nl + nn, 0);
+    std::vector<char> is_gemm(nsteps, 0), has_req(nl + nn, 0);
     std::vector<std::vector<int32_t>> req(nl + nn);
-    std::vector<Cls> cls(nn);
-    std::vector<std::vector<int32_t>> gemm_out(nn);
-    std::vector<int> split(nn, 0);
+    std::vector<Cls> cls(nsteps);
+    std::vector<std::vector<int32_t>> gemm_out(nsteps);
+    std::vector<int> split(nsteps, 0);
     for (int32_t j = nn - 1; j >= 0; j--) {
       const int o = nl + j;
       if (inside(o)) continue;
@@ -1304,17 +1362,19 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
           const PUnit& u = P.units[U.unit_of(o)];
           for (int q = 0; q < u.next; q++) {  // in the units' label order
             const int32_t x = P.ext[u.ext0 + q].tensor;
-            req[x] = U.sorted[x];
+            req[x].resize(lab[x].size());
+            for (size_t k = 0; k < req[x].size(); k++) req[x][k] = order[U.places(x)[k]];
             has_req[x] = 1;
           }
         }
         continue;
       }
-      cls[j] = classify(j);
-      Cls& c = cls[j];
+      const int32_t k = step_of[j];
+      cls[k] = classify(j);
+      Cls& c = cls[k];
       int na = (int)c.a.size(), nb = (int)c.b.size(), nk = (int)c.k.size();
       bool g = !c.priv && gemm_shaped(opt, na, nb, nk);
-      is_gemm[j] = g;
+      is_gemm[k] = g;
       if (g) {
         // the order of the M, N and batch labels is free: with a layout
         // request from the consumer, follow it (the output then needs no
@@ -1330,12 +1390,12 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
         // become batch labels between the outputs and t
         const int ks = gemm_split(opt, na, nb, nk, (int)st.size());
         std::vector<int32_t> klo(sk.begin(), sk.end() - ks), khi(sk.end() - ks, sk.end());
-        split[j] = ks;
+        split[k] = ks;
         c.a = sa;
         c.b = sb;
         c.k = sk;
         c.t = st;
-        gemm_out[j] = concat({&sa, &sb, &khi, &st});
+        gemm_out[k] = concat({&sa, &sb, &khi, &st});
         req[c.ca] = concat({&sa, &klo, &khi, &st});
         req[c.cb] = concat({&klo, &sb, &khi, &st});
         has_req[c.ca] = has_req[c.cb] = 1;
@@ -1360,22 +1420,23 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
         P.ops.push_back(op);
         continue;
       }
-      Cls& c = cls[j];
-      if (is_gemm[j]) {
+      const int32_t k = step_of[j];
+      Cls& c = cls[k];
+      if (is_gemm[k]) {
         int dst = o;
         const int na = (int)c.a.size(), nb = (int)c.b.size();
         POp epi;
-        const int scatter = B.layout[o] != gemm_out[j] && split[j] == 0
-                                ? gemm_scatter_mode(opt, B.layout[o], gemm_out[j], na, nb, &epi)
+        const int scatter = B.layout[o] != gemm_out[k] && split[k] == 0
+                                ? gemm_scatter_mode(opt, B.layout[o], gemm_out[k], na, nb, &epi)
                                 : 0;
-        if (B.layout[o] != gemm_out[j] && !scatter) dst = B.add_tensor(gemm_out[j]);
-        B.gemm(c.ca, c.cb, dst, na, nb, (int)c.k.size() - split[j], (int)c.t.size() + split[j]);
+        if (B.layout[o] != gemm_out[k] && !scatter) dst = B.add_tensor(gemm_out[k]);
+        B.gemm(c.ca, c.cb, dst, na, nb, (int)c.k.size() - split[k], (int)c.t.size() + split[k]);
         if (scatter) {
           POp& g = P.ops.back();
           g.scatter = scatter;
           std::fill(std::begin(g.pc), std::end(g.pc), (int8_t)-1);
-          for (size_t q = 0; q < gemm_out[j].size(); q++)
-            g.pc[q] = (int8_t)pos_in(B.layout[o], gemm_out[j][q]);
+          for (size_t q = 0; q < gemm_out[k].size(); q++)
+            g.pc[q] = (int8_t)pos_in(B.layout[o], gemm_out[k][q]);
           std::memcpy(g.ep, epi.ep, sizeof g.ep);
           g.ep_n = epi.ep_n;
           g.ep_split = epi.ep_split;
@@ -1398,7 +1459,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
       c.b.clear();
       c.k.clear();
       c.t.clear();
-      const auto &LX = lab[x], &LY = lab[y], &LC = lab[o];
+      const Labels LX = lab[x], LY = lab[y], LC = lab[o];
       for (int32_t l : LC) {
         bool inx = pos_in(LX, l) >= 0, iny = pos_in(LY, l) >= 0;
         if (inx && iny)
@@ -1422,7 +1483,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
         if (B.ew(y, -1, tb)) return -1;
       }
       int dst = o;
-      if (gout != LC) dst = B.add_tensor(gout);
+      if (gout != std::vector<int32_t>(LC)) dst = B.add_tensor(gout);
       int na = (int)c.a.size(), nb = (int)c.b.size(), nk = (int)c.k.size();
       bool g = gemm_shaped(opt, na, nb, nk);
       if (g)

@@ -146,7 +146,6 @@ struct PlanOptions {
 int plan_slice(const SliceIn& s, const PlanOptions& opt, SlicePlan* out, std::string* err);
 
 // Reference-model helpers (every label of size 2).
-int slice_labels(const SliceIn& s, std::vector<std::vector<int32_t>>* labels, std::string* err);
 int slice_complexity(const SliceIn& s, double* tc, double* sc, double* rwc, std::string* err);
 int slice_peak_memory(const SliceIn& s, double* peak, double* all, std::string* err);
 

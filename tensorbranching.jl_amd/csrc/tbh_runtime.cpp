@@ -454,34 +454,36 @@ int plan_all(tbh_ctx* ctx, const std::vector<const SliceOwned*>& slices, bool ba
 
 PlanStream::PlanStream(const std::vector<const SliceOwned*>& slices, const PlanOptions& opt,
                        WorkerPool& pool, int threads)
-    : slices_(slices), plans_(slices.size()), done_(slices.size(), 0) {
-  auto worker = [this, opt](int) {
-    for (;;) {
-      const size_t i = next_.fetch_add(1);
-      if (i >= slices_.size()) return;
-      {
-        std::lock_guard<std::mutex> g(m_);
-        if (i > bad_) return;
+    : slices_(slices), opt_(opt), plans_(slices.size()), done_(slices.size(), 0) {
+  // the thread that calls get() plans too while it waits: one ticket fewer
+  const int nt = (int)std::min<size_t>(std::max(1, threads), slices.size()) - 1;
+  if (pool.size() > 0 && nt > 0)
+    batch_ = pool.post(nt, [this](int) {
+      while (plan_next()) {
       }
-      std::string err;
-      const int rc = plan_slice(slices_[i]->in, opt, &plans_[i], &err);
-      {
-        std::lock_guard<std::mutex> g(m_);
-        if (rc && i < bad_) {
-          bad_ = i;
-          bad_err_ = "slice " + std::to_string(i) + ": " + err;
-        }
-        done_[i] = 1;
-      }
-      cv_.notify_all();
-    }
-  };
-  const int nt = (int)std::min<size_t>(std::max(1, threads), std::max<size_t>(1, slices.size()));
-  if (pool.size() == 0) {
-    worker(0);  // no pool threads: plan everything now
-  } else {
-    batch_ = pool.post(nt, worker);
+    });
+}
+
+// Plans the next slice nobody has taken; false when there is none left.
+bool PlanStream::plan_next() {
+  const size_t i = next_.fetch_add(1);
+  if (i >= slices_.size()) return false;
+  {
+    std::lock_guard<std::mutex> g(m_);
+    if (i > bad_) return false;
   }
+  std::string err;
+  const int rc = plan_slice(slices_[i]->in, opt_, &plans_[i], &err);
+  {
+    std::lock_guard<std::mutex> g(m_);
+    if (rc && i < bad_) {
+      bad_ = i;
+      bad_err_ = "slice " + std::to_string(i) + ": " + err;
+    }
+    done_[i] = 1;
+  }
+  cv_.notify_all();
+  return true;
 }
 
 PlanStream::~PlanStream() {
@@ -489,10 +491,17 @@ PlanStream::~PlanStream() {
     std::lock_guard<std::mutex> g(m_);
     bad_ = 0;  // stop the workers after their current slice
   }
-  if (batch_) WorkerPool::wait(*batch_);
+  if (batch_) WorkerPool::close_and_wait(*batch_);
 }
 
 const SlicePlan* PlanStream::get(size_t i, std::string* err) {
+  for (;;) {
+    {
+      std::lock_guard<std::mutex> g(m_);
+      if (done_[i] || i >= bad_) break;
+    }
+    if (!plan_next()) break;
+  }
   std::unique_lock<std::mutex> g(m_);
   cv_.wait(g, [&] { return done_[i] || i >= bad_; });
   if (i >= bad_) {
@@ -718,8 +727,6 @@ int BatchRunner::open() {
   }
   arena_base_ = (uint64_t)(ctx_->base + region_off_);
   desc_budget_ = ctx_->pool.largest_free() / 2;
-  for (auto& ev : evs_)
-    if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) ev = nullptr;
   return 0;
 }
 
@@ -733,9 +740,6 @@ void BatchRunner::close() {
     ctx_->pool.free(prev_.doff);
     prev_.on = false;
   }
-  for (auto& ev : evs_)
-    if (ev) (void)hipEventDestroy(ev);
-  evs_[0] = evs_[1] = nullptr;
   if (region_off_ >= 0) ctx_->pool.free(region_off_);
   region_off_ = -1;
   region_ = 0;
@@ -822,7 +826,7 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
         return v < n;
     return false;
   };
-  if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, j.up, 0);
+  if (e == hipSuccess && j.up) e = hipStreamWaitEvent(ctx->stream, j.up, 0);
   hipEvent_t ev = nullptr;
   // the units of level L (0: those that read no tensor from memory)
   auto units = [&](int L) {
@@ -1014,7 +1018,7 @@ void Issuer::reset() {
 
 int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices,
                          const std::vector<const SlicePlan*>& plans, bool add_r, uint32_t* dst,
-                         void* tag, void** done_tag) {
+                         void* tag, void** done_tag, bool only) {
   if (done_tag) *done_tag = nullptr;
   tbh_ctx* ctx = ctx_;
   const size_t nb = plans.size();
@@ -1202,13 +1206,16 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   }
   // the upload goes on the copy stream, beside the batch in flight (its
   // descriptors are a pool block of their own); the issuing thread makes the
-  // compute stream wait for it
+  // compute stream wait for it.  The only batch of a call has nothing to run
+  // beside: it goes up on the compute stream, and the caller issues it.
+  only = only && !prev_.on;
   char* dbase = ctx->base + doff;
-  const hipEvent_t up = ctx->up_events[bidx & 1];
-  hipError_t e = hipMemcpyAsync(dbase, hb, bytes, hipMemcpyHostToDevice, ctx->copy_stream);
-  if (e == hipSuccess) e = hipEventRecord(up, ctx->copy_stream);
+  const hipEvent_t up = only ? nullptr : ctx->up_events[bidx & 1];
+  const hipStream_t upload = only ? ctx->stream : ctx->copy_stream;
+  hipError_t e = hipMemcpyAsync(dbase, hb, bytes, hipMemcpyHostToDevice, upload);
+  if (e == hipSuccess && up) e = hipEventRecord(up, upload);
   if (e != hipSuccess) {
-    (void)hipStreamSynchronize(ctx->copy_stream);
+    (void)hipStreamSynchronize(upload);
     ctx->pool.free(doff);
     set_error(std::string("descriptor upload: ") + hipGetErrorString(e));
     return TBH_EDEVICE;
@@ -1236,7 +1243,7 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   job->dbase = dbase;
   job->hb = hb;
   job->up = up;
-  job->done = evs_[bidx & 1];
+  job->done = ctx->done_events[bidx & 1];
   job->cnt = std::move(cnt);
   job->pfx = std::move(pfx);
   job->o_desc = std::move(o_desc);
@@ -1245,7 +1252,16 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   job->lvl_bytes = std::move(lvl_bytes);
   job->lvl_macs = std::move(lvl_macs);
   job->step_work = std::move(step_work);
-  ctx->issuer.submit(std::move(job));
+  if (only) {
+    if ((e = issue_batch(ctx, *job)) != hipSuccess) {
+      sync_all();
+      ctx->pool.free(doff);
+      set_error(std::string("batched launch: ") + hipGetErrorString(e));
+      return TBH_EDEVICE;
+    }
+  } else {
+    ctx->issuer.submit(std::move(job));
+  }
   // this batch runs while the previous one is waited for
   void* tag_prev = nullptr;
   if ((rc = finish(&tag_prev))) {
@@ -1256,7 +1272,7 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   }
   if (done_tag) *done_tag = early_tag ? early_tag : tag_prev;
   prev_.on = true;
-  prev_.done = evs_[bidx & 1];
+  prev_.done = ctx->done_events[bidx & 1];
   prev_.doff = doff;
   prev_.parity = bidx & 1;
   prev_.nb = nb;
@@ -1315,7 +1331,7 @@ int execute_batched(tbh_ctx* ctx, int dtype, const std::vector<const SliceOwned*
     }
     ctx->stats.host_ms[0] += ms_since(t_plan);
     if (status) break;
-    status = run.enqueue(dtype, sl, plans, add_r, results + i0, nullptr, nullptr);
+    status = run.enqueue(dtype, sl, plans, add_r, results + i0, nullptr, nullptr, i1 == n);
     i0 = i1;
   }
   if (status == 0) status = run.flush(nullptr);
@@ -1568,7 +1584,8 @@ int tbh_create(int device, size_t pool_bytes, tbh_ctx** out) {
     return TBH_ENOMEM;
   }
   auto release = [&] {
-    for (hipEvent_t& x : ctx->up_events)
+    for (hipEvent_t x : {ctx->up_events[0], ctx->up_events[1], ctx->done_events[0],
+                         ctx->done_events[1]})
       if (x) (void)hipEventDestroy(x);
     for (hipStream_t s : {ctx->stream, ctx->stream2, ctx->copy_stream})
       if (s) (void)hipStreamDestroy(s);
@@ -1577,7 +1594,9 @@ int tbh_create(int device, size_t pool_bytes, tbh_ctx** out) {
       hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking) != hipSuccess ||
       hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&ctx->up_events[0], hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->up_events[1], hipEventDisableTiming) != hipSuccess) {
+      hipEventCreateWithFlags(&ctx->up_events[1], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&ctx->done_events[0], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&ctx->done_events[1], hipEventDisableTiming) != hipSuccess) {
     release();
     set_error("stream or event creation failed");
     return TBH_EDEVICE;
@@ -1629,7 +1648,8 @@ int tbh_destroy(tbh_ctx* ctx) {
   if (ctx->base) (void)hipFree(ctx->base);
   for (auto& v : ctx->lvl_events)
     for (hipEvent_t ev : v) (void)hipEventDestroy(ev);
-  for (hipEvent_t ev : ctx->up_events)
+  for (hipEvent_t ev : {ctx->up_events[0], ctx->up_events[1], ctx->done_events[0],
+                        ctx->done_events[1]})
     if (ev) (void)hipEventDestroy(ev);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);

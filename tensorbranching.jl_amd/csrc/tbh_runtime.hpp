@@ -173,6 +173,7 @@ struct tbh_ctx {
   hipStream_t stream2 = nullptr;  // GEMM launches beside the EW launches of a level
   hipStream_t copy_stream = nullptr;   // batched descriptor uploads, beside the batch in flight
   hipEvent_t up_events[2] = {nullptr, nullptr};  // upload done, per batch parity
+  hipEvent_t done_events[2] = {nullptr, nullptr};  // batch done, per batch parity
   std::vector<hipEvent_t> lvl_events[2];  // cross-stream level barriers, per batch parity
   char* base = nullptr;  // device pool
   tbh::Pool pool;
@@ -207,9 +208,9 @@ struct SliceOwned {
 
 int convert_slice(const tbh_slice& s, tbh_dtype dtype, bool copy, SliceOwned* out);
 
-// Plans slices on background host threads in index order; get(i) blocks
-// until slice i is planned and returns nullptr (error in *err) if planning
-// failed at or before i.
+// Plans slices on background host threads in index order, and on the thread
+// that waits for one: get(i) returns slice i's plan, or nullptr (error in
+// *err) if planning failed at or before i.
 class PlanStream {
  public:
   PlanStream(const std::vector<const SliceOwned*>& slices, const PlanOptions& opt,
@@ -218,7 +219,9 @@ class PlanStream {
   const SlicePlan* get(size_t i, std::string* err);
 
  private:
+  bool plan_next();
   const std::vector<const SliceOwned*>& slices_;
+  const PlanOptions opt_;
   std::vector<SlicePlan> plans_;
   std::vector<char> done_;
   std::mutex m_;
@@ -237,7 +240,8 @@ size_t region_bytes(size_t largest);
 // batch in flight behind the one being enqueued.  enqueue() packs a batch
 // (its arenas must fit region() together), launches it, then waits for the
 // batch enqueued before it, whose results it copies to that batch's `dst`
-// and whose `tag` it returns in *done_tag (nullptr: none).  flush() waits
+// and whose `tag` it returns in *done_tag (nullptr: none); only: no batch
+// follows, so with none in flight the caller itself issues it.  flush() waits
 // for the last batch the same way.  After an error the results of the
 // batch being enqueued and of the one in flight are lost; close() (also the
 // destructor) waits for the streams and releases the region.  The caller
@@ -255,7 +259,7 @@ class BatchRunner {
   bool busy() const { return prev_.on; }
   int enqueue(int dtype, const std::vector<const SliceOwned*>& slices,
               const std::vector<const SlicePlan*>& plans, bool add_r, uint32_t* dst, void* tag,
-              void** done_tag);
+              void** done_tag, bool only = false);
   int flush(void** done_tag);
   // waits until every launch of the newest batch is issued (a failed launch
   // is reported by the next enqueue or flush)
@@ -280,7 +284,6 @@ class BatchRunner {
   size_t desc_budget_ = 0;
   uint64_t arena_base_ = 0;
   int bidx_ = 0;
-  hipEvent_t evs_[2] = {nullptr, nullptr};
   Pending prev_;
 };
 
