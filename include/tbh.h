@@ -292,7 +292,8 @@ int tbh_plan_steps(const tbh_slice* slice, tbh_dtype dtype, tbh_mode mode,
  * persistent grid; more: later workgroups start as earlier ones finish,
  * which evens out uneven tiles); gemm_tiles: GEMM tile shapes (0: 128 x 128
  * only; 1: 256 x 64 / 256 x 32 tiles for outputs of M >= 256 rows and N <= 64
- * / 32 columns; 2: 256 x 64 up to N = 128 too); chain_cost > 0: a chain
+ * / 32 columns; 2: 256 x 64 up to N = 128 too; 1 and 2: 64 x 64 for steps of
+ * fewer than 256 such tiles); chain_cost > 0: a chain
  * rotation is taken only when it lowers the estimated cost of the two steps
  * it replaces, bytes moved + MACs * chain_cost / 64, in place of the
  * chain_reduce cap (0: the caps alone).  Results never depend on them. */

@@ -1,6 +1,7 @@
-// tbh_gemm.hip -- K1b tbh_gemm_ksplit_kernel: one max-plus GEMM (the
-// tbh_maxplus_gemm entry point) whose 128 x 128 tiles would not fill the
-// GPU, or whose extents or alignment are odd.
+// tbh_gemm.hip -- K1b: max-plus GEMMs in 64 x 64 tiles, for products whose
+// 128 x 128 tiles would not fill the GPU, or whose extents or alignment are
+// odd.  tbh_gemm_ksplit_kernel runs one product (the tbh_maxplus_gemm entry
+// point), tbh_gemm64_kernel the GEMM steps of a wave (GemmDesc::shape 3).
 //
 // A workgroup of four waves owns one 64 x 64 output tile; every wave holds
 // the whole tile (8 x 8 maxima per lane, the register blocking of K1) and
@@ -17,12 +18,17 @@
 // Bound by the VALU for large products (4096^3 Float32 1742 us = 78.9 T op/s
 // of the 82.1 measured for its instruction mix; 4093 x 4095 x 4091 71.9, 67.2
 // with K1), by too little work in flight and the two launches for small ones
-// (512^3 19 us, 114 with K1's 16 tiles; 64^3 10.5 us, 18.6 with K1, about 6 us
-// of each the events around it).
+// (512^3 19 us, 114 with K1's 16 tiles; 64^3 10 us, 18.6 with K1, about 6 us
+// of each the events around it).  Short K: bound by handing the maxima over,
+// which all four waves share (two waves alone: 4096^2 x 1024 491 us, 479 so;
+// in one round of 48 KB instead of two of 24 KB: 486).  The grouped kernel
+// runs the GEMM steps of 301 n=200 slices at 31 T op/s Int32 (K1: 19 of the
+// 52 measured for the mix).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "tbh_device.hpp"
+#include "tbh_gemm_epi.hpp"
 
 namespace tbh {
 
@@ -46,48 +52,77 @@ __device__ __forceinline__ typename Quad<T>::V shift_quad(typename Quad<T>::V x,
   return x;
 }
 
-}  // namespace
+constexpr int kLdsA = kSlab * kTile, kLdsB = kSlab * kBRow;
+constexpr int kGemmLds = 2 * (kLdsA + kLdsB);  // two slabs
+static_assert(kGemmLds >= 6 * 1024 && kGemmLds >= kTile * kTile, "maxima handed over, the tile");
 
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void
-tbh_gemm_ksplit_kernel(const GemmSplit g) {
+__device__ __forceinline__ int tile_col(int wave, int ty) {
+  return 32 * (wave >> 1) + ty + 2 * (wave & 1);
+}
+
+// One tile over the K range [kb, ke): afterwards quad q of the thread (res[q])
+// is rows 32 (q & 1) + tx .. + 3 of column tile_col(wave, ty) + (q >> 1).  EDGE:
+// any extents >= 4 and alignment; else M and N are multiples of 64 and K is 16
+// or a multiple of 32 (kb = 0, ke = K).
+template <typename T, bool EDGE>
+__device__ __forceinline__ void gemm64_tile(const TBH_GLOBAL T* __restrict__ A,
+                                            const TBH_GLOBAL T* __restrict__ B, int M, int N,
+                                            int K, int64_t lda, int64_t ldb, int kb, int ke,
+                                            int m0, int n0, int tid, T* __restrict__ smem,
+                                            T (&res)[4][4]) {
+  T acc[8][8];
   using V = typename Quad<T>::V;
   using U = typename Quad<T>::U;
-  constexpr int NA = kSlab * kTile, NB = kSlab * kBRow;
-  constexpr int NRED = 2 * 64 * 64;  // two waves' maxima
-  constexpr int NLDS = 2 * (NA + NB) > NRED ? 2 * (NA + NB) : NRED;
-  __shared__ __align__(16) T smem[NLDS];
-  const int tid = threadIdx.x, lane = tid & 63;
+  constexpr int NA = kLdsA, NB = kLdsB;
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  uint32_t b = blockIdx.x;
-  const int tm = b % g.tiles_m;
-  b /= g.tiles_m;
-  const int tn = b % g.tiles_n;
-  b /= g.tiles_n;
-  const int part = b % g.ksplit, t = b / g.ksplit;
-  const int m0 = tm * kTile, n0 = tn * kTile;
-  const int kb = part * g.kpart, ke = g.K < kb + g.kpart ? g.K : kb + g.kpart;
-  const TBH_GLOBAL T* A = reinterpret_cast<const TBH_GLOBAL T*>(g.a) + t * g.sA;
-  const TBH_GLOBAL T* B = reinterpret_cast<const TBH_GLOBAL T*>(g.b) + t * g.sB;
   const T pz = pad_zero<T>();
   // this thread's quads: A rows am..am+3 of slab columns ak and ak + 16, B
   // slab rows bk..bk+3 of columns bn and bn + 32
   const int aq = (tid & 15) * 4, ak = tid >> 4;
   const int bk = (tid & 7) * 4, bn = tid >> 3;
-  // rows past M read earlier ones, shifted so that valid rows stay in place
-  const int am = m0 + aq < g.M - 4 ? m0 + aq : g.M - 4;
-  const int as = m0 + aq - am < 4 ? m0 + aq - am : 0;
-  const bool edge_m = m0 + kTile > g.M;
-  const int bn0 = n0 + bn < g.N ? n0 + bn : g.N - 1;
-  const int bn1 = n0 + bn + 32 < g.N ? n0 + bn + 32 : g.N - 1;
   V ra[2], rb[2];
+  // rows past M read earlier ones, shifted so that valid rows stay in place
+  const int am = !EDGE || m0 + aq < M - 4 ? m0 + aq : M - 4;
+  const int as = m0 + aq - am < 4 ? m0 + aq - am : 0;
+  const bool edge_m = m0 + kTile > M;
+  const int bn0 = !EDGE || n0 + bn < N ? n0 + bn : N - 1;
+  const int bn1 = !EDGE || n0 + bn + 32 < N ? n0 + bn + 32 : N - 1;
+  // !EDGE: wave-uniform bases of the tile and one 32-bit byte offset per lane
+  // and quad (M and K at most 2^24, the planner's rule), which leaves the
+  // registers the maxima need
+  const uint32_t oa = ((uint32_t)ak * (uint32_t)lda + aq) * 4;
+  const uint32_t ob = ((uint32_t)bn * (uint32_t)ldb + bk) * 4;
+  auto at = [](const TBH_GLOBAL T* base, uint32_t byte) {
+    return *reinterpret_cast<const TBH_GLOBAL U*>(
+        reinterpret_cast<const TBH_GLOBAL char*>(base) + byte);
+  };
   auto load = [&](int k0) {
+    if constexpr (!EDGE) {
+      const TBH_GLOBAL T* Ak = A + m0 + (int64_t)k0 * lda;
+      const TBH_GLOBAL T* Bk = B + (int64_t)n0 * ldb + k0;
+      if (k0 + kSlab <= ke) {
+        ra[0] = at(Ak, oa);
+        ra[1] = at(Ak + 16 * lda, oa);
+        rb[0] = at(Bk, ob);
+        rb[1] = at(Bk + 32 * ldb, ob);
+      } else {  // K = 16: half a slab
+        ra[0] = at(Ak, oa);
+        ra[1] = V{pz, pz, pz, pz};
+        rb[0] = rb[1] = V{pz, pz, pz, pz};
+        if (bk < 16) {
+          rb[0] = at(Bk, ob);
+          rb[1] = at(Bk + 32 * ldb, ob);
+        }
+      }
+      return;
+    }
     if (k0 + kSlab <= ke) {
 #pragma unroll
       for (int e = 0; e < 2; e++)
-        ra[e] = *reinterpret_cast<const TBH_GLOBAL U*>(A + (int64_t)(k0 + ak + 16 * e) * g.lda + am);
-      rb[0] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn0 * g.ldb + k0 + bk);
-      rb[1] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn1 * g.ldb + k0 + bk);
+        ra[e] = *reinterpret_cast<const TBH_GLOBAL U*>(A + (int64_t)(k0 + ak + 16 * e) * lda + am);
+      rb[0] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn0 * ldb + k0 + bk);
+      rb[1] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn1 * ldb + k0 + bk);
     } else {
       // the range's last slab: columns of A past it are the tropical zero,
       // and so are B's rows (a range ends at a multiple of 4, or at K)
@@ -95,14 +130,14 @@ tbh_gemm_ksplit_kernel(const GemmSplit g) {
       for (int e = 0; e < 2; e++) {
         const int k = k0 + ak + 16 * e;
         if (k < ke)
-          ra[e] = *reinterpret_cast<const TBH_GLOBAL U*>(A + (int64_t)k * g.lda + am);
+          ra[e] = *reinterpret_cast<const TBH_GLOBAL U*>(A + (int64_t)k * lda + am);
         else
           ra[e] = V{pz, pz, pz, pz};
       }
-      const int k = k0 + bk, kc = k < g.K - 4 ? k : g.K - 4;
+      const int k = k0 + bk, kc = k < K - 4 ? k : K - 4;
       if (k < ke) {
-        rb[0] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn0 * g.ldb + kc);
-        rb[1] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn1 * g.ldb + kc);
+        rb[0] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn0 * ldb + kc);
+        rb[1] = *reinterpret_cast<const TBH_GLOBAL U*>(B + (int64_t)bn1 * ldb + kc);
         rb[0] = shift_quad<T>(rb[0], k - kc, pz);
         rb[1] = shift_quad<T>(rb[1], k - kc, pz);
       } else {
@@ -126,7 +161,6 @@ tbh_gemm_ksplit_kernel(const GemmSplit g) {
     }
   };
   const int tx = (lane & 7) * 4, ty = (lane >> 3) * 4;
-  T acc[8][8];
 #pragma unroll
   for (int i = 0; i < 8; i++)
 #pragma unroll
@@ -165,76 +199,170 @@ tbh_gemm_ksplit_kernel(const GemmSplit g) {
     __syncthreads();
     buf ^= 1;
   }
-  // waves 2 and 3 hand their maxima to waves 0 and 1; then wave 0 takes
-  // columns j < 4 of both and wave 1 the others
-  T* red = smem;
-  auto put = [&](int slot, int j0, int j1) {
+  // wave d ends with columns 2 d and 2 d + 1 of every lane's block: the others
+  // hand it theirs, two waves' columns (24 KB) at a time
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (j >= j0 && j < j1)
+  for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+    for (int i = 0; i < 4; i++) res[q][i] = acc[4 * (q & 1) + i][q >> 1];  // wave 0's
+#pragma unroll
+  for (int half = 0; half < 2; half++) {
+#pragma unroll
+    for (int d = 2 * half; d < 2 * half + 2; d++) {
+      if (wave != d) {
+        T* p = smem + (((d & 1) * 3 + (wave < d ? wave : wave - 1)) * 256 + lane) * 4;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int j = 2 * d + (q >> 1), h = q & 1;
           T x0 = acc[4 * h][j], x1 = acc[4 * h + 1][j], x2 = acc[4 * h + 2][j],
             x3 = acc[4 * h + 3][j];
           asm volatile("" : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3));  // keeps acc in registers
-          *reinterpret_cast<V*>(red + ((slot * 16 + 2 * j + h) * 64 + lane) * 4) = V{x0, x1, x2, x3};
+          *reinterpret_cast<V*>(p + q * 256) = V{x0, x1, x2, x3};
         }
-  };
-  auto take = [&](int slot, int j0, int j1) {
+      } else {
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (j >= j0 && j < j1)
+        for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const V v = *reinterpret_cast<const V*>(red + ((slot * 16 + 2 * j + h) * 64 + lane) * 4);
-          acc[4 * h][j] = Trop<T>::add(acc[4 * h][j], v.x);
-          acc[4 * h + 1][j] = Trop<T>::add(acc[4 * h + 1][j], v.y);
-          acc[4 * h + 2][j] = Trop<T>::add(acc[4 * h + 2][j], v.z);
-          acc[4 * h + 3][j] = Trop<T>::add(acc[4 * h + 3][j], v.w);
+          for (int i = 0; i < 4; i++) res[q][i] = acc[4 * (q & 1) + i][2 * d + (q >> 1)];
+      }
+    }
+    __syncthreads();
+    if ((wave >> 1) == half) {
+#pragma unroll
+      for (int o = 0; o < 3; o++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const V v = *reinterpret_cast<const V*>(
+              smem + ((((wave & 1) * 3 + o) * 4 + q) * 64 + lane) * 4);
+#pragma unroll
+          for (int i = 0; i < 4; i++) res[q][i] = Trop<T>::add(res[q][i], v[i]);
         }
-  };
-  if (wave >= 2) put(wave - 2, 0, 8);
-  __syncthreads();
-  if (wave < 2) take(wave, 0, 8);
-  __syncthreads();
-  if (wave == 0) put(0, 4, 8);
-  if (wave == 1) put(1, 0, 4);
-  __syncthreads();
-  if (wave >= 2) return;
-  if (wave == 0) take(1, 0, 4);
-  if (wave == 1) take(0, 4, 8);
+    }
+    if (half == 0) __syncthreads();
+  }
+}
+
+}  // namespace
+
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void
+tbh_gemm_ksplit_kernel(const GemmSplit g) {
+  using V = typename Quad<T>::V;
+  using U = typename Quad<T>::U;
+  __shared__ __align__(16) T smem[kGemmLds];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tx = (lane & 7) * 4, ty = (lane >> 3) * 4;
+  uint32_t b = blockIdx.x;
+  const int tm = b % g.tiles_m;
+  b /= g.tiles_m;
+  const int tn = b % g.tiles_n;
+  b /= g.tiles_n;
+  const int part = b % g.ksplit, t = b / g.ksplit;
+  const int m0 = tm * kTile, n0 = tn * kTile;
+  const int kb = part * g.kpart, ke = g.K < kb + g.kpart ? g.K : kb + g.kpart;
+  const TBH_GLOBAL T* A = reinterpret_cast<const TBH_GLOBAL T*>(g.a) + t * g.sA;
+  const TBH_GLOBAL T* B = reinterpret_cast<const TBH_GLOBAL T*>(g.b) + t * g.sB;
+  T res[4][4];
+  gemm64_tile<T, true>(A, B, g.M, g.N, g.K, g.lda, g.ldb, kb, ke, m0, n0, threadIdx.x, smem, res);
   // ksplit > 1: raw maxima to the workspace, dense M x N per (batch, part)
   const bool ws = g.ksplit > 1;
   const int64_t ld = ws ? g.M : g.ldc;
   TBH_GLOBAL T* C = ws ? reinterpret_cast<TBH_GLOBAL T*>(g.ws) +
                              ((int64_t)t * g.ksplit + part) * g.M * g.N
                        : reinterpret_cast<TBH_GLOBAL T*>(g.c) + t * g.sC;
-  auto write = [&](int j0) {
 #pragma unroll
-    for (int jj = 0; jj < 4; jj++) {
-      const int j = j0 + jj, n = n0 + (j0 ? 32 : 0) + ty + jj;
-      if (n >= g.N) continue;
+  for (int q = 0; q < 4; q++) {
+    const int n = n0 + tile_col(wave, ty) + (q >> 1), m = m0 + 32 * (q & 1) + tx;
+    if (n >= g.N) continue;
+    V v = V{res[q][0], res[q][1], res[q][2], res[q][3]};
+    if (!ws)
+      v = V{Trop<T>::canon(v.x), Trop<T>::canon(v.y), Trop<T>::canon(v.z), Trop<T>::canon(v.w)};
+    TBH_GLOBAL T* p = C + n * ld + m;
+    if (m + 4 <= g.M) {
+      *reinterpret_cast<TBH_GLOBAL U*>(p) = v;
+    } else {
+      if (m < g.M) p[0] = v.x;
+      if (m + 1 < g.M) p[1] = v.y;
+      if (m + 2 < g.M) p[2] = v.z;
+    }
+  }
+}
+
+// Grouped: prefix[i] is the first tile of GEMM step i; a block walks tiles.
+// Every extent is a power of two, M and N at least 64 (the planner's rule).
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void tbh_gemm64_kernel(
+    const GemmDesc* __restrict__ ops, const int64_t* __restrict__ prefix, int nops,
+    int64_t total) {
+  using V = typename Quad<T>::V;
+  __shared__ __align__(16) T smem[kGemmLds];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int64_t tile = blockIdx.x; tile < total; tile += gridDim.x) {
+    int lo = 0, hi = nops;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (prefix[mid] <= tile)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    const GemmDesc* d = ops + __builtin_amdgcn_readfirstlane(lo);
+    // tiles along M, then N, then the batch, all powers of two
+    uint32_t r = (uint32_t)(tile - prefix[lo]);
+    const int tm = r & (d->tiles_m - 1);
+    r >>= __builtin_ctz(d->tiles_m);
+    const int tn = r & (d->tiles_n - 1);
+    const int64_t t = r >> __builtin_ctz(d->tiles_n);
+    const int m0 = tm * kTile, n0 = tn * kTile;
+    const TBH_GLOBAL T* A = reinterpret_cast<const TBH_GLOBAL T*>(d->a) + t * d->sA;
+    const TBH_GLOBAL T* B = reinterpret_cast<const TBH_GLOBAL T*>(d->b) + t * d->sB;
+    TBH_GLOBAL T* C = reinterpret_cast<TBH_GLOBAL T*>(d->c);
+    // opaque: what a tile derives from the thread index is not held in
+    // registers across tiles
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, tx = (lane & 7) * 4, ty = (lane >> 3) * 4;
+    T res[4][4];
+    gemm64_tile<T, false>(A, B, d->M, d->N, d->K, d->lda, d->ldb, 0, d->K, m0, n0, tid, smem,
+                          res);
+    auto quad = [&](int q) {
+      return V{Trop<T>::canon(res[q][0]), Trop<T>::canon(res[q][1]), Trop<T>::canon(res[q][2]),
+               Trop<T>::canon(res[q][3])};
+    };
+    const int nl = tile_col(wave, ty);
+    if (d->scatter == 0) {
+      C += t * d->sC;
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int m = m0 + 32 * h + tx;
-        V v = V{acc[4 * h][j], acc[4 * h + 1][j], acc[4 * h + 2][j], acc[4 * h + 3][j]};
-        if (!ws)
-          v = V{Trop<T>::canon(v.x), Trop<T>::canon(v.y), Trop<T>::canon(v.z), Trop<T>::canon(v.w)};
-        TBH_GLOBAL T* p = C + n * ld + m;
-        if (m + 4 <= g.M) {
-          *reinterpret_cast<TBH_GLOBAL U*>(p) = v;
-        } else {
-          if (m < g.M) p[0] = v.x;
-          if (m + 1 < g.M) p[1] = v.y;
-          if (m + 2 < g.M) p[2] = v.z;
+      for (int q = 0; q < 4; q++)
+        *reinterpret_cast<TBH_GLOBAL V*>(C + (n0 + nl + (q >> 1)) * d->ldc + m0 + 32 * (q & 1) +
+                                         tx) = quad(q);
+    } else {
+      const int ma = __builtin_ctz((uint32_t)d->M), nb = __builtin_ctz((uint32_t)d->N);
+      C += scatter_bits(d->pc, ma + nb, (uint32_t)t) + scatter_bits(d->pc, 0, m0) +
+           scatter_bits(d->pc, ma, n0);
+      if (d->scatter == 1) {
+        // rows 0 and 1 at C positions 0 and 1: row quads are 16-byte runs
+        const int64_t at = scatter_bits(d->pc, 0, tx) + scatter_bits(d->pc, ma, nl);
+        const int64_t rh = scatter_bits(d->pc, 0, 32), c1 = scatter_bits(d->pc, ma, 1);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          *reinterpret_cast<TBH_GLOBAL V*>(C + at + ((q & 1) ? rh : 0) + ((q >> 1) ? c1 : 0)) =
+              quad(q);
+      } else {
+        // the tile through LDS, read back in ascending C position
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const uint32_t n = nl + (q >> 1), m = 32 * (q & 1) + tx;
+          *reinterpret_cast<V*>(smem + ((m ^ ((n & 15) << 2)) + (n << 6))) = quad(q);
         }
+        __syncthreads();
+        emit_staged<T>(C, smem, d->ep_n, 6, 15, d->pc, ma, d);
       }
     }
-  };
-  if (wave == 0)
-    write(0);
-  else
-    write(4);
+    __syncthreads();
+  }
 }
 
 // C = the maximum over the K ranges' workspaces, one thread per four outputs
@@ -278,6 +406,16 @@ hipError_t launch_gemm_ksplit(int dtype, const GemmSplit& g, hipStream_t s) {
     tbh_gemm_reduce_kernel<float><<<rb, 256, 0, s>>>(g);
   else
     tbh_gemm_reduce_kernel<int32_t><<<rb, 256, 0, s>>>(g);
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm64(int dtype, const GemmDesc* ops, const int64_t* prefix, int nops,
+                         int64_t total, int grid, hipStream_t s) {
+  if (total <= 0) return hipSuccess;
+  if (dtype == 0)
+    tbh_gemm64_kernel<float><<<grid, 256, 0, s>>>(ops, prefix, nops, total);
+  else
+    tbh_gemm64_kernel<int32_t><<<grid, 256, 0, s>>>(ops, prefix, nops, total);
   return hipGetLastError();
 }
 

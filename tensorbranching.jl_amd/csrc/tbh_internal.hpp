@@ -33,8 +33,14 @@ __host__ __device__ inline int gemm_shape(int64_t M, int64_t N, int rule = 1) {
   if (N <= (rule >= 2 ? 128 : 64)) return 1;
   return 0;
 }
-__host__ __device__ inline int gemm_bm(int shape) { return shape ? 256 : 128; }
-__host__ __device__ inline int gemm_bn(int shape) { return shape == 2 ? 32 : shape == 1 ? 64 : 128; }
+// (shape 3: 64 x 64, each K slab split over the workgroup's waves)
+constexpr int kGemm64 = 3, kGemmShapes = 4;
+__host__ __device__ inline int gemm_bm(int shape) {
+  return shape == kGemm64 ? 64 : shape ? 256 : 128;
+}
+__host__ __device__ inline int gemm_bn(int shape) {
+  return shape == 2 ? 32 : shape == 0 ? 128 : 64;
+}
 
 // One EW step C = max over the reduced labels of A + B, tiled through LDS.
 // The output labels split into tile labels (nT bits, ordered by C position)
@@ -81,7 +87,7 @@ struct GemmDesc {
   int64_t lda, ldb, ldc;
   int64_t sA, sB, sC;
   int32_t tiles_m, tiles_n; // tiles per batch entry
-  int32_t shape;            // tile 0: 128 x 128, 1: 256 x 64, 2: 256 x 32
+  int32_t shape;            // tile 0: 128 x 128, 1: 256 x 64, 2: 256 x 32, 3: 64 x 64
   // scatter: 0 C column-major with ldc; otherwise C has its own label order
   // (M, N, batch powers of two): bit q of (m, n, batch) -- m bits first,
   // then n, then batch -- sits at C position pc[q].  1: rows 0..4 sit at

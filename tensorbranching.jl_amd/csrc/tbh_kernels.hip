@@ -23,6 +23,7 @@
 #include <stdint.h>
 
 #include "tbh_device.hpp"
+#include "tbh_gemm_epi.hpp"
 #include "tbh_internal.hpp"
 
 // minimum waves per SIMD the EW kernels are register-limited to
@@ -1016,18 +1017,6 @@ struct GemmShape<2> {
   static constexpr int BM = 256, BN = 32, TN = 4;
 };
 
-// Offset of the output bits x (bit b is GEMM output bit q0 + b) in a C whose
-// bit q sits at position pc[q] (-1: no position; only rows / columns past M /
-// N, which are not written, reach those).
-__device__ __forceinline__ int64_t scatter_bits(const int8_t* __restrict__ pc, int q0, uint32_t x) {
-  int64_t r = 0;
-  for (int b = 0; x != 0 && q0 + b < kGemmScatter; b++, x >>= 1) {
-    const int p = pc[q0 + b];
-    if ((x & 1) && p >= 0) r += (int64_t)1 << p;
-  }
-  return r;
-}
-
 // Output tile of a GEMM whose C has its own label order (scatter 2): the
 // tile goes to LDS, then the threads read it back in ascending C position
 // (enumeration bit k of output e = tid + 256 r is tile bit ep[k]), so that
@@ -1079,62 +1068,7 @@ __device__ __forceinline__ void gemm_epilogue_pass(TBH_GLOBAL T* __restrict__ C,
     }
   }
   __syncthreads();
-  // enumeration bit k as its share of the LDS index (xk: XORed part, ak:
-  // added part; row bit b: xk = 2^b; column bit b: xk = 4 (2^b & s), ak =
-  // 2^(vm+b)) and of the C offset (gk), decoded once (uniform)
-  uint32_t xk[13], ak[13], gk[13];
-#pragma unroll
-  for (int k = 0; k < 13; k++) {
-    xk[k] = ak[k] = gk[k] = 0;
-    if (k < nbits) {
-      const int b = d->ep[k];
-      if (b < 32) {
-        xk[k] = 1u << b;
-        gk[k] = 1u << pc[b];
-      } else {
-        xk[k] = ((1u << (b - 32)) & smask) << 2;
-        ak[k] = (1u << (b - 32)) << vm;
-        gk[k] = 1u << pc[ma + b - 32];
-      }
-    }
-  }
-  // enumeration bits 0 and 1 are C positions 0 and 1 (ep lists the pass's
-  // bits by C position, and C's lowest positions are pass bits): a thread
-  // owns 4 consecutive outputs, one aligned 16-byte store; bits 2..9 are
-  // the thread, bits 10.. the iteration r
-  uint32_t xt = 0, at = 0, gt = 0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const bool on = (tid >> k) & 1;
-    xt ^= on ? xk[2 + k] : 0u;
-    at += on ? ak[2 + k] : 0u;
-    gt += on ? gk[2 + k] : 0u;
-  }
-  uint32_t li[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-    li[i] = ((i & 1) ? xk[0] : 0u) ^ ((i & 2) ? xk[1] : 0u);
-  const uint32_t a1 = ak[0], a2 = ak[1];
-  TBH_GLOBAL T* __restrict__ Ct = C + base;
-  const int R = 1 << (nbits - 10);  // 4 .. 8 per pass
-#pragma unroll
-  for (int r = 0; r < 8; r++) {
-    if (r >= R) break;
-    uint32_t xr = xt, ar = at, gr = gt;
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-      if ((r >> k) & 1) {
-        xr ^= xk[10 + k];
-        ar += ak[10 + k];
-        gr += gk[10 + k];
-      }
-    V q;
-    q.x = st[(xr ^ li[0]) + ar];
-    q.y = st[(xr ^ li[1]) + ar + a1];
-    q.z = st[(xr ^ li[2]) + ar + a2];
-    q.w = st[(xr ^ li[3]) + ar + a1 + a2];
-    *reinterpret_cast<TBH_GLOBAL V*>(Ct + gr) = q;
-  }
+  emit_staged<T>(C + base, st, nbits, vm, smask, pc, ma, d);
   __syncthreads();
 }
 
@@ -1512,6 +1446,9 @@ hipError_t launch_ew_direct(int dtype, const EwDesc* ops, const int64_t* prefix,
   return hipGetLastError();
 }
 
+hipError_t launch_gemm64(int dtype, const GemmDesc* ops, const int64_t* prefix, int nops,
+                         int64_t total, int grid, hipStream_t s);  // tbh_gemm.hip
+
 // The scalar-load kernel (a standalone product of M or K below 4, or of more
 // tiles than K1b indexes) has 128 x 128 tiles only.
 template <typename T>
@@ -1525,12 +1462,14 @@ static void* gemm_kernel(bool vec, int shape) {
 hipError_t launch_gemm(int dtype, bool vec, int shape, const GemmDesc* ops, const int64_t* prefix,
                        int nops, int64_t total, int grid, hipStream_t s) {
   if (total <= 0) return hipSuccess;
+  if (shape == kGemm64) return launch_gemm64(dtype, ops, prefix, nops, total, grid, s);
   void* args[] = {&ops, &prefix, &nops, &total};
   const void* k = dtype == 0 ? gemm_kernel<float>(vec, shape) : gemm_kernel<int32_t>(vec, shape);
   return hipLaunchKernel(k, dim3(grid), dim3(256), args, 0, s);
 }
 
 int gemm_blocks_per_cu(int dtype, bool vec, int shape) {
+  if (shape == kGemm64) return 3;  // 155 VGPRs, 33 KB of LDS
   int n = 0;
   const void* k = dtype == 0 ? gemm_kernel<float>(vec, shape) : gemm_kernel<int32_t>(vec, shape);
   const hipError_t err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 256, 0);

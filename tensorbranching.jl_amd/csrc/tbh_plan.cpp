@@ -151,6 +151,23 @@ struct PosMap {
   }
 };
 
+// The tile shape of a GEMM step of 2^na x 2^nb outputs, 2^nk K, 2^nt batch.  A
+// step of fewer than 2^8 of the large tiles leaves CUs idle, also beside the
+// other steps of its wave, and takes 64 x 64 tiles (301 slices of 3-regular
+// n=200 at sc 20, Int32: GEMM 2.59 -> 1.58 ms; the King's subgraph 1.21 ->
+// 0.66 ms; n=300 at sc 25 unchanged).  Steps of more tiles keep the large ones,
+// whose pass over the maxima costs less at the small K most of them have
+// (lines at 2^7, 2^9, 2^10 tiles: n=300 GEMM 110.5, 111.7, 114.2 ms against
+// 109.3; every step in 64 x 64 tiles: 141 ms).
+int step_shape(const PlanOptions& opt, int na, int nb, int nk, int nt) {
+  const int shape = gemm_shape((int64_t)1 << na, (int64_t)1 << nb, opt.gemm_tiles);
+  // (extents the kernel's 32-bit offsets hold)
+  if (opt.gemm_tiles <= 0 || na < 6 || nb < 6 || nk < 4 || na > 24 || nk > 24) return shape;
+  const int tiles = std::max(0, na - __builtin_ctz(gemm_bm(shape))) +
+                    std::max(0, nb - __builtin_ctz(gemm_bn(shape))) + nt;
+  return tiles < 8 ? kGemm64 : shape;
+}
+
 struct Builder {
   const SliceIn& s;
   const PlanOptions& opt;
@@ -426,7 +443,7 @@ struct Builder {
     op.N = 1 << nb;
     op.K = 1 << nk;
     op.batch = 1 << nt;
-    op.shape = gemm_shape(op.M, op.N, opt.gemm_tiles);
+    op.shape = step_shape(opt, na, nb, nk, nt);
     op.macs = std::ldexp(1.0, na + nb + nk + nt);
     op.bytes = 4.0 * (std::ldexp(1.0, na + nk + nt) + std::ldexp(1.0, nk + nb + nt) +
                       std::ldexp(1.0, na + nb + nt));
@@ -457,11 +474,10 @@ bool gemm_shaped(const PlanOptions& opt, int na, int nb, int nk) {
 // row quads are 16-byte runs of C), else 2 (staged through LDS, ep the
 // pass's tile bits in ascending position of L).
 int gemm_scatter_mode(const PlanOptions& opt, const std::vector<int32_t>& L,
-                      const std::vector<int32_t>& G, int na, int nb, POp* g) {
+                      const std::vector<int32_t>& G, int na, int nb, int shape, POp* g) {
   if (opt.gemm_scatter_bits < 0 || L.size() != G.size() || (int)G.size() > kGemmScatter - 8 ||
       na < 2)
     return 0;
-  const int shape = gemm_shape((int64_t)1 << na, (int64_t)1 << nb, opt.gemm_tiles);
   const int bm = __builtin_ctz(gemm_bm(shape)), bn = __builtin_ctz(gemm_bn(shape));
   const int vm = std::min(na, bm), vn = std::min(nb, bn);
   const int split = vm + vn > 13 ? 1 : 0;  // an LDS pass holds kEpiElems = 2^13 outputs
@@ -625,7 +641,10 @@ int verify_plan(const SlicePlan& P, std::string* err) {
           ec != ((int64_t)1 << rc))
         return bad("GEMM extents");
       if (op.M % 4 || op.K % 4) return bad("GEMM vector alignment");
-      if (op.shape < 0 || op.shape > 2) return bad("GEMM tile shape");
+      if (op.shape < 0 || op.shape >= kGemmShapes ||
+          (op.shape == kGemm64 && (op.M < 64 || op.N < 64 || op.K < 16 || op.M > 1 << 24 ||
+                                   op.K > 1 << 24)))
+        return bad("GEMM tile shape");
       if (op.scatter) {
         // pc: a bijection of the output bits onto C's positions, -1 past
         // them; scatter 1: rows 0 and 1 at positions 0 and 1 (quad stores);
@@ -1427,7 +1446,10 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
         const int na = (int)c.a.size(), nb = (int)c.b.size();
         POp epi;
         const int scatter = B.layout[o] != gemm_out[k] && split[k] == 0
-                                ? gemm_scatter_mode(opt, B.layout[o], gemm_out[k], na, nb, &epi)
+                                ? gemm_scatter_mode(opt, B.layout[o], gemm_out[k], na, nb,
+                                                    step_shape(opt, na, nb, (int)c.k.size(),
+                                                               (int)c.t.size()),
+                                                    &epi)
                                 : 0;
         if (B.layout[o] != gemm_out[k] && !scatter) dst = B.add_tensor(gemm_out[k]);
         B.gemm(c.ca, c.cb, dst, na, nb, (int)c.k.size() - split[k], (int)c.t.size() + split[k]);

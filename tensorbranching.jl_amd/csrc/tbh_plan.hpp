@@ -133,7 +133,8 @@ struct PlanOptions {
   // are direct); steps with reductions run faster LDS-tiled (DMA staging)
   int direct_max_reduce = 0;
   // GEMM tile rule (gemm_shape): 0 128 x 128 only, 1 tall-skinny tiles for
-  // N <= 64, 2 also 256 x 64 up to N = 128
+  // N <= 64, 2 also 256 x 64 up to N = 128; 1 and 2: 64 x 64 tiles for steps
+  // of few such tiles
   int gemm_tiles = 1;
   // subtrees whose tensors fit in LDS run as units (batched only)
   bool units = true;

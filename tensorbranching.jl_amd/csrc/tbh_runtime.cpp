@@ -630,8 +630,8 @@ int ew_chunk(tbh_ctx* ctx, int64_t total) {
 // ------------------------------------------------------ BATCHED ----------
 namespace {
 
-// launch kinds: 0 direct EW, 1 tiled EW, 2 + s GEMM with tile shape s, 5 units
-constexpr int kKinds = 6, kUnitKind = 5;
+// launch kinds: 0 direct EW, 1 tiled EW, 2 + s GEMM with tile shape s, then units
+constexpr int kUnitKind = 2 + kGemmShapes, kKinds = kUnitKind + 1;
 int op_kind(const POp& op) {
   if (op.kind == kUnit) return kUnitKind;
   return op.kind == kGemm ? 2 + op.shape : (op.direct ? 0 : 1);
@@ -1573,7 +1573,7 @@ int tbh_create(int device, size_t pool_bytes, tbh_ctx** out) {
     ctx->ew_occ[t] = ew_blocks_per_cu(t);
     ctx->ew_pf_occ[t] = ew_pf_blocks_per_cu(t);
     for (int v = 0; v < 2; v++)
-      for (int s = 0; s < 3; s++) ctx->gemm_occ[t][v][s] = gemm_blocks_per_cu(t, v != 0, s);
+      for (int s = 0; s < kGemmShapes; s++) ctx->gemm_occ[t][v][s] = gemm_blocks_per_cu(t, v != 0, s);
   }
   size_t fr = 0, tot = 0;
   HIP_TRY(hipMemGetInfo(&fr, &tot));
@@ -1795,10 +1795,10 @@ int tbh_contract_max(tbh_ctx* ctx, tbh_dtype dtype, const tbh_slice* slices, siz
 // Whether a standalone product runs on K1b (64 x 64 tiles), and in how many
 // K ranges.  K1 keeps the aligned products of at least 512 of its tiles and
 // K <= 256: there K1b's pass over the waves' maxima, once per 64 x 64 outputs,
-// costs more than its finer tiles give (4096 x 4096, kernel us K1 / K1b: K = 16
-// 22 / 46, 64 46 / 62, 256 136 / 151, 1024 486 / 491, 4096 1803 / 1742; 512
-// products of 128 x 128 x 64 27 / 34).  With fewer tiles K1 leaves CUs idle
-// (3072 x 2048 x 128 38 / 37; 2048^2 x 64 22 / 20; 1024^3 224 / 47; 512^3
+// costs more than its finer tiles give (4096 x 4096, kernel us K1 / K1b before
+// all four waves shared that pass: K = 16 22 / 46, 64 46 / 62, 256 136 / 151;
+// now 1024 486 / 479, 4096 1803 / 1746).  With fewer tiles K1 leaves CUs idle
+// (3072 x 2048 x 128 38 / 36; 2048^2 x 64 22 / 18; 1024^3 224 / 47; 512^3
 // 114 / 19), and unaligned extents took K1's scalar loads (three 1021 x 515 x
 // 777 Int32 238 / 92).  K1 alone takes M or K below one quad.  Products of
 // fewer than 256 tiles are split over K until 512 workgroups run, in ranges

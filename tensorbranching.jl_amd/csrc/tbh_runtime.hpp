@@ -29,6 +29,8 @@ hipError_t launch_ew_direct(int dtype, const EwDesc* ops, const int64_t* prefix,
                             int64_t total, int grid, int chunk, hipStream_t s);
 hipError_t launch_gemm(int dtype, bool vec, int shape, const GemmDesc* ops, const int64_t* prefix,
                        int nops, int64_t total, int grid, hipStream_t s);
+hipError_t launch_gemm64(int dtype, const GemmDesc* ops, const int64_t* prefix, int nops,
+                         int64_t total, int grid, hipStream_t s);  // tbh_gemm.hip
 hipError_t launch_gemm_ksplit(int dtype, const GemmSplit& g, hipStream_t s);  // tbh_gemm.hip
 hipError_t launch_leaves(int dtype, const LeafDesc* leaves, int64_t n, hipStream_t s);
 hipError_t launch_epilogue(int dtype, const EpiDesc* e, int64_t n, void* out, hipStream_t s);
@@ -167,7 +169,7 @@ struct tbh_ctx {
   int num_cus = 256;
   int ew_occ[2] = {4, 4};     // resident tiled-EW workgroups per CU, per element type
   int ew_pf_occ[2] = {4, 4};  // the same for the prefetching kernel
-  int gemm_occ[2][2][3] = {};  // resident GEMM workgroups per CU [dtype][vec][shape],
+  int gemm_occ[2][2][tbh::kGemmShapes] = {};  // resident GEMM workgroups per CU [dtype][vec][shape],
                                // from the occupancy query in tbh_create
   hipStream_t stream = nullptr;
   hipStream_t stream2 = nullptr;  // GEMM launches beside the EW launches of a level
