@@ -127,36 +127,39 @@ struct EpiDesc {
 
 // A fused part of the tree ("unit"): every step of a maximal connected part
 // whose tensors all fit in LDS, contracted by one workgroup.  Tensors from
-// outside it (ext) are copied to LDS first, only its root goes to memory.  Inside a unit every tensor holds its labels in one global order
-// (elimination time, latest first), so a step's union index -- the output's
-// bits, then the reduced labels' -- maps to an operand's by keeping the
-// operand's bits (mA / mB), and a step is 16 bytes.
-constexpr int kUnitWaves = 4;      // waves of a unit's workgroup
+// outside it (ext) are copied to LDS first, only its root goes to memory.
+// Inside a unit every tensor holds its labels in one global order (elimination
+// time, latest first), so a step's union index is the output's bits, then the
+// reduced labels'.
+constexpr int kUnitWavesLog2 = 3;
+constexpr int kUnitWaves = 1 << kUnitWavesLog2;  // waves of a unit's workgroup
 constexpr int kUnitLds = 8192;     // LDS elements of a unit
 constexpr int kUnitBits = 15;      // union labels of a unit's step
 constexpr int kUnitRank = 14;      // output labels of a unit's step
-constexpr int kUnitOperand = 12;  // labels of a tensor read from memory
+constexpr int kUnitOperand = 12;   // labels of a tensor read from memory
 constexpr int kUnitReduce = 6;     // reduced labels of a unit's step
-// One wave's share of one step: chunks c0 .. c0+nc-1 of 64 outputs.
+// One wave's share of one step: chunks c0 .. c0+nc-1 of 64 outputs (nc a power
+// of two, c0 a multiple), after `levels` more barriers than the wave has passed.
 struct UnitItem {
-  uint16_t mA, mB;      // union bits held by A / B
-  uint16_t oA, oB, oC;  // LDS element offsets
-  uint16_t c0, nc;      // nc = 0: nothing to do
-  uint16_t f;           // output bits | reduced bits << 4 | flags
+  uint16_t mA, mB;  // the union bits of A and B; an operand holds its own in order
+  uint16_t oA, oB;  // LDS element offsets of the operands at chunk c0
+  uint16_t oC, c0;  // ... of the output (chunk 0)
+  uint16_t f;       // output bits | reduced bits << 4 | kItemRoot | log2(nc) << 12
+  uint16_t levels;
 };
-constexpr int kItemBarrier = 1 << 8;  // the last item of a level (in every wave)
-constexpr int kItemRoot = 1 << 9;     // the unit's output: to memory
+constexpr int kItemRoot = 1 << 8;  // the unit's output: to memory
 struct UnitDesc {
   uint64_t c;        // device address of the output, 0: the slice's root scalar
-  uint32_t item0;    // first item; wave w's are item0 + w rounds + 0 .. rounds-1
+  uint64_t pos;      // nibble k: the C position of output bit k
+  uint32_t item0;    // first item; wave w's are item0 + start[w] .. start[w + 1] - 1
   uint32_t w0;       // first vertex weight
-  int32_t rounds;    // items per wave; 0: a leaf tensor (nvert 1: vertex, 0: edge)
-  int32_t nvert;     // vertex leaves, [0, w] at LDS 4 + 2 i (the edge tensor is at 0)
   uint32_t ext0;     // first tensor read from memory
   int32_t next;      // ... and their number
+  int32_t nvert;     // vertex leaves, [0, w] at LDS 4 + 2 i (the edge tensor is at 0)
   int32_t res;       // c == 0: index of the slice's result
   int32_t rbits;     // ... and its r
-  uint64_t pos;      // nibble k: the C position of output bit k
+  // no items at all: a leaf tensor (nvert 1: vertex, 0: edge)
+  uint16_t start[kUnitWaves + 2];
 };
 struct UnitExt {
   uint64_t p;        // device address, labels in the units' order

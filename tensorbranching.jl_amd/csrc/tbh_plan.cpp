@@ -819,7 +819,7 @@ struct UnitBuilder {
   const std::vector<int32_t>& order;  // ... and its inverse
   SlicePlan& P;
   int32_t nl;
-  // log2 of a unit's MACs at most: 4 waves take about 5 us for 2^17
+  // log2 of a unit's MACs at most: 8 waves take about 3 us for 2^17
   static constexpr double kUnitMacs = 131072.0;
   // tree node (leaf or internal): inside a unit, the output of a unit of
   // leaves (or a leaf in memory), or the output of a unit that also reads
@@ -927,7 +927,8 @@ struct UnitBuilder {
         node_at.push_back(c);
       }
     }
-    if (work > kUnitMacs) return false;
+    // (items are indexed by 16 bits: one per node, and one more per 64 MACs)
+    if (work > kUnitMacs || node_at.size() > 0x7fff) return false;
     // breadth first: node_at is in descending level order from the back
     // LDS: the edge tensor, the vertex tensors, then the internal tensors,
     // blocks of a level's dead operands reused one level later
@@ -983,10 +984,12 @@ struct UnitBuilder {
       P.unit_w.push_back(s.wbits ? s.wbits[v] : s.unit_wbits);
     }
     for (auto& w : wave) w.clear();
-    int next = 0;
+    int levels[kUnitWaves] = {};  // barriers since the wave's last item
     size_t k = node_at.size();
     while (k > 0) {
       const int lv = level[node_at[k - 1]];
+      int next = 0;
+      bool any = false;
       for (; k > 0 && level[node_at[k - 1]] == lv; k--) {
         const int32_t o = node_at[k - 1], j = o - nl;
         if (external(o)) continue;
@@ -998,45 +1001,52 @@ struct UnitBuilder {
         UnitItem it{};
         const int nP = rank(o), rx = rank(x), ry = rank(y);
         int n = 0;
+        uint16_t sA[16], sB[16];  // strides of the union's bits
         for (int a = 0, b = 0; a < rx || b < ry; n++) {
           const int32_t va = a < rx ? px[a] : INT32_MAX, vb = b < ry ? py[b] : INT32_MAX;
           po[n] = va <= vb ? va : vb;  // (at most 15 labels in a union)
-          if (va <= vb) it.mA |= (uint16_t)(1u << n), a++;
-          if (vb <= va) it.mB |= (uint16_t)(1u << n), b++;
+          const uint32_t inA = va <= vb, inB = vb <= va;
+          it.mA |= (uint16_t)(inA << n);
+          it.mB |= (uint16_t)(inB << n);
+          sA[n] = (uint16_t)(inA << a);
+          sB[n] = (uint16_t)(inB << b);
+          a += (int)inA;
+          b += (int)inB;
         }
         const int nR = n - nP;
         auto lds_of = [&](int32_t c) {
           return c >= nl ? off[c] : vert[c] >= 0 && rank(c) == 1 ? 4 + 2 * vert[c] : 0;
         };
-        it.oA = (uint16_t)lds_of(x);
-        it.oB = (uint16_t)lds_of(y);
+        const int oA = lds_of(x), oB = lds_of(y);
         it.oC = (uint16_t)(o == root ? 0 : off[o]);
-        it.f = (uint16_t)(nP | nR << 4 | (o == root ? kItemRoot : 0));
         // the step's chunks in up to kUnitWaves equal runs
-        const int chunks = nP > 6 ? 1 << (nP - 6) : 1;
-        const int runs = std::min(chunks, kUnitWaves);
-        for (int q = 0; q < runs; q++) {
-          it.c0 = (uint16_t)(chunks / runs * q);
-          it.nc = (uint16_t)(chunks / runs);
+        const int lp = std::max(nP - 6, 0), lr = std::min(lp, kUnitWavesLog2), lc = lp - lr;
+        it.f = (uint16_t)(nP | nR << 4 | (o == root ? kItemRoot : 0) | lc << 12);
+        for (int q = 0; q < 1 << lr; q++) {
+          it.c0 = (uint16_t)(q << lc);
+          int a = oA, b = oB;
+          for (int h = 0; h < lr; h++)
+            if ((q >> h) & 1) a += sA[6 + lc + h], b += sB[6 + lc + h];
+          it.oA = (uint16_t)a;
+          it.oB = (uint16_t)b;
+          it.levels = (uint16_t)levels[next];
+          levels[next] = 0;
           wave[next].push_back(it);
           next = (next + 1) % kUnitWaves;
+          any = true;
         }
         P.unit_steps.push_back(
             {(int8_t)rank(x), (int8_t)rank(y), (int8_t)nP, (int8_t)nR, (int32_t)P.units.size()});
         u.macs += (double)(1u << n);
         u.bytes += 4.0 * ((1u << rank(x)) + (1u << rank(y)) + (1u << nP));
       }
-      // every wave ends the level in the same round
-      size_t rounds = 0;
-      for (auto& w : wave) rounds = std::max(rounds, w.size());
-      if (rounds == 0) continue;  // a level of tensors from memory only
-      for (auto& w : wave) {
-        w.resize(rounds, UnitItem{});
-        w.back().f |= kItemBarrier;
-      }
+      if (any)  // (a level of tensors from memory only has no barrier)
+        for (int& n : levels) n++;
     }
-    u.rounds = (int)wave[0].size();
-    for (auto& w : wave) P.items.insert(P.items.end(), w.begin(), w.end());
+    for (int w = 0; w < kUnitWaves; w++) {
+      u.start[w + 1] = (uint16_t)(u.start[w] + wave[w].size());
+      P.items.insert(P.items.end(), wave[w].begin(), wave[w].end());
+    }
     P.units.push_back(u);
     P.unit_levels = std::max(P.unit_levels, depth + 1);
     // (root last: external() reads in_unit of the nodes below it)
@@ -1097,7 +1107,7 @@ struct UnitBuilder {
 
   // output bit -> position in the layout its consumer reads
   void set_layout(PUnit* u, const std::vector<int32_t>& lay) {
-    if (u->rounds == 0) return;  // a leaf: its content is symmetric
+    if (u->items() == 0) return;  // a leaf: its content is symmetric
     const int32_t* p = places(u->tensor);
     for (int k = 0; k < rank(u->tensor); k++)
       u->pos |= (uint64_t)(pos_in(lay, order[p[k]]) & 15) << (4 * k);
@@ -1122,11 +1132,11 @@ int verify_units(const SlicePlan& P, std::string* err) {
           x.off + (1u << P.tensors[x.tensor].rank) > (uint32_t)kUnitLds)
         return bad("memory tensor");
     }
-    if (u.rounds == 0) {
+    if (u.items() == 0) {
       if (rank != (u.nvert ? 1 : 2) || u.next) return bad("leaf");
       continue;
     }
-    if (u.item0 + (size_t)u.rounds * kUnitWaves > P.items.size()) return bad("items");
+    if (u.item0 + (size_t)u.items() > P.items.size()) return bad("items");
     uint32_t used = 0;
     for (int k = 0; k < rank; k++) {
       const int p = (int)(u.pos >> (4 * k)) & 15;
@@ -1134,26 +1144,37 @@ int verify_units(const SlicePlan& P, std::string* err) {
       used |= 1u << p;
     }
     int64_t root_chunks = 0;
-    for (int r = 0; r < u.rounds; r++)
-      for (int w = 0; w < kUnitWaves; w++) {
-        const UnitItem& it = P.items[u.item0 + (size_t)w * u.rounds + r];
-        if ((it.f ^ P.items[u.item0 + r].f) & kItemBarrier) return bad("levels");
-        if (r == u.rounds - 1 && !(it.f & kItemBarrier)) return bad("last level");
-        if (!it.nc) continue;
-        const int nP = it.f & 15, nR = (it.f >> 4) & 15, n = nP + nR;
+    for (int w = 0; w < kUnitWaves; w++) {
+      if (u.start[w] > u.start[w + 1]) return bad("waves");
+      for (int i = u.start[w]; i < u.start[w + 1]; i++) {
+        const UnitItem& it = P.items[u.item0 + i];
+        const int nP = it.f & 15, nR = (it.f >> 4) & 15, n = nP + nR, lc = it.f >> 12;
         const int chunks = nP > 6 ? 1 << (nP - 6) : 1;
-        if (n > kUnitBits || nR > kUnitReduce || it.c0 + it.nc > chunks || it.nc > 64 ||
-            (uint32_t)(it.mA | it.mB) != (1u << n) - 1 ||
-            it.oA + (1 << __builtin_popcount(it.mA)) > kUnitLds ||
-            it.oB + (1 << __builtin_popcount(it.mB)) > kUnitLds)
+        if (n > kUnitBits || nR > kUnitReduce || nP > kUnitRank || lc > 6 ||
+            (it.c0 & ((1 << lc) - 1)) || it.c0 + (1 << lc) > chunks ||
+            (it.mA | it.mB) != (1 << n) - 1)
           return bad("step");
+        // the last places that the item reads: all bits of the union set but
+        // those of its chunk number
+        uint32_t eA = 0, eB = 0, a = 1, b = 1;
+        for (int k = 0; k < n; k++) {
+          const bool fixed = k >= 6 + lc && k < nP;
+          const uint32_t inA = (it.mA >> k) & 1, inB = (it.mB >> k) & 1;
+          eA += fixed ? 0 : a * inA;
+          eB += fixed ? 0 : b * inB;
+          a <<= inA;
+          b <<= inB;
+        }
+        if (it.oA + eA >= (uint32_t)kUnitLds || it.oB + eB >= (uint32_t)kUnitLds)
+          return bad("operand");
         if (it.f & kItemRoot) {
           if (nP != rank) return bad("root");
-          root_chunks += it.nc;
+          root_chunks += 1 << lc;
         } else if (it.oC < 4 + 2 * u.nvert || it.oC + (1 << nP) > kUnitLds) {
           return bad("tensor");
         }
       }
+    }
     if (root_chunks != (rank > 6 ? 1 << (rank - 6) : 1)) return bad("root cover");
   }
   return 0;

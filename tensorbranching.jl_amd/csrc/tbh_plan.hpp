@@ -63,7 +63,9 @@ struct PLeaf {
 struct PUnit {
   int tensor = -1;        // output; kind and weight of a leaf as in UnitDesc
   uint32_t item0 = 0, w0 = 0, ext0 = 0;  // into SlicePlan::items / unit_w / ext
-  int rounds = 0, nvert = 0, next = 0;
+  int nvert = 0, next = 0;
+  uint16_t start[kUnitWaves + 2] = {};  // as UnitDesc; all 0: a leaf
+  int items() const { return start[kUnitWaves]; }
   int level = 0;          // wave; 0: before every step (no ext)
   double macs = 0, bytes = 0;  // of its steps, as POp
   uint64_t pos = 0;

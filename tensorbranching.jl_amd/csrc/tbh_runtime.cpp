@@ -1159,7 +1159,7 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
       ud->c = result ? 0 : b + (uint64_t)P.tensors[u.tensor].off;
       ud->item0 = (uint32_t)first[i].item + u.item0;
       ud->w0 = (uint32_t)first[i].w + u.w0;
-      ud->rounds = u.rounds;
+      std::memcpy(ud->start, u.start, sizeof ud->start);
       ud->nvert = u.nvert;
       ud->res = (int32_t)i;
       ud->rbits = (int32_t)rbits;

@@ -81,6 +81,22 @@ def test_star_reduced_at_once(tb, orc, backend, leaves):
         assert np.array_equal(backend.contract_slices([b], dtype), orc.contract_slices([b], dtype))
 
 
+@pytest.mark.parametrize("nv", [32, 33, 34, 64, 66, 200])
+def test_long_chain(tb, orc, backend, nv):
+    """A path contracted from one end: a unit of 2 nv - 2 levels of one step
+    each, all of one wave's, which reads its shares 64 at a time."""
+    g = tb.SimpleGraph(nv, [(i, i + 1) for i in range(nv - 1)])
+    ixs = [[v] for v in range(nv)] + [[int(u), int(v)] for u, v in g.edges]
+    t = 0
+    for i in range(nv - 1):
+        t = tb.ContractionTree(tb.ContractionTree(t, nv + i), i + 1)
+    code = tb.CompressedEinsum(ixs, [], t)
+    w = np.random.default_rng(nv).integers(1, 101, nv)
+    for dtype in (np.float32, np.int32):
+        b = tb.SlicedBranch(tb.MISProblem(g, w.astype(dtype)), code, 3)
+        assert np.array_equal(backend.contract_slices([b], dtype), orc.contract_slices([b], dtype))
+
+
 def test_infinite_weights(tb, backend):
     """A vertex of weight -inf is never taken; one of +inf is."""
     g = tb.random_regular_graph(20, 3, seed=4)
