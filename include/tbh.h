@@ -283,7 +283,8 @@ int tbh_plan_steps(const tbh_slice* slice, tbh_dtype dtype, tbh_mode mode,
  * workgroups per CU in a launch's grid (at most what is resident);
  * direct_max_reduce: EW steps reducing more labels than this run LDS-tiled,
  * not as direct wave tiles (-1: all tiled); concurrent: 1 runs a level's
- * GEMM launches on a second stream beside its EW launches; first_batch:
+ * GEMM launches on a second stream beside its EW launches where both are
+ * long; first_batch:
  * fraction of the arena region the first batch may use; ew_prefetch: 1 runs
  * LDS-tiled EW steps with the next tile's sub-tensors loaded into registers
  * while the current tile computes, 0 stages each tile by DMA after the

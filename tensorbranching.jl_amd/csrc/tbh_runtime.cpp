@@ -845,8 +845,8 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
   if (e == hipSuccess) e = units(0);
   // one launch per kernel kind and level (direct EW, tiled EW, GEMM); in
   // the per-step profiling mode every step alone, tagged with its shape
-  // GEMM launches on a second stream beside a level's EW launches (not
-  // while profiling): a level's steps are independent, so the VALU-bound
+  // GEMM launches on a second stream beside a level's EW launches where both
+  // are long (not while profiling): a level's steps are independent, so the VALU-bound
   // GEMM tiles and the memory-bound EW tiles can share the CUs.  Each
   // stream waits for the other's work of earlier levels (events recorded
   // lazily, only when the other stream launched since the last sync).
@@ -872,6 +872,25 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
     dirty[o] = false;
     return r;
   };
+  hipStream_t gemm_stream = sk[1];
+  // Whether level L's GEMMs go beside its other steps.  The way to the second
+  // stream and back costs two event waits, 5-20 us each with the device idle,
+  // so both sides must have 40 us of work (us by the rates that the steps of
+  // a level reach together: 40 T op/s, 3 TB/s).  Every GEMM on the second
+  // stream / this rule / none: King's subgraph 2.33 / 2.24 / 2.32 ms, a burst
+  // of 24 requests 4.15 / 4.04 / 4.03, 301 slices of n=200 8.46 / 8.33 / 8.99,
+  // n=300 253 / 245 / 267 (10 to 80 us within the spread of runs).
+  auto apart = [&](int L) {
+    double gemm_us = 0, ew_us = 0;
+    for (int k = 0; k < kKinds; k++) {
+      const int w = slot(k, L);
+      if (k >= 2 && k < kUnitKind)
+        gemm_us += 2 * j.lvl_macs[w] / 40e6;
+      else
+        ew_us += j.lvl_bytes[w] / 3e6;
+    }
+    return std::min(gemm_us, ew_us) >= 40;
+  };
   auto launch = [&](int k, const char* descs, const int64_t* prefix, int nops, int64_t total) {
     if (injected()) return hipErrorLaunchFailure;
     if (k == 0)
@@ -884,15 +903,17 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
                        ew_grid(ctx, dtype, total, ew_chunk(ctx, total)), ew_chunk(ctx, total),
                        sk[0]);
     return launch_gemm(dtype, true, k - 2, reinterpret_cast<const GemmDesc*>(descs), prefix, nops,
-                       total, gemm_grid(ctx, total, dtype, true, k - 2), sk[1]);
+                       total, gemm_grid(ctx, total, dtype, true, k - 2), gemm_stream);
   };
   for (int L = 1; L <= H && e == hipSuccess; L++) {
     if (conc) {
       // a stream launching work of this level first waits for the other
       // stream's work of earlier levels (both syncs before any launch)
       bool has[2] = {false, false};
+      const bool two = apart(L);
+      gemm_stream = sk[two];
       for (int k = 0; k < kKinds; k++)
-        if (cnt[slot(k, L)]) has[k >= 2 && k < kUnitKind ? 1 : 0] = true;
+        if (cnt[slot(k, L)]) has[k >= 2 && k < kUnitKind && two ? 1 : 0] = true;
       if (has[0] && e == hipSuccess) e = sync_to(0);
       if (has[1] && e == hipSuccess) e = sync_to(1);
       if (has[0]) dirty[0] = true;
