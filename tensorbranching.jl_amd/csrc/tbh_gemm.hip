@@ -299,55 +299,55 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
   __shared__ __align__(16) T smem[kGemmLds];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   for (int64_t tile = blockIdx.x; tile < total; tile += gridDim.x) {
-    int lo = 0, hi = nops;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (prefix[mid] <= tile)
-        lo = mid;
-      else
-        hi = mid;
-    }
-    const GemmDesc* d = ops + __builtin_amdgcn_readfirstlane(lo);
+    const int step = gemm_step((const TBH_CONST int64_t*)prefix, nops, tile);
+    const KGemm d = (KGemm)(ops + step);
+    const uint32_t w = gemm_lanes(d);
     // tiles along M, then N, then the batch, all powers of two
-    uint32_t r = (uint32_t)(tile - prefix[lo]);
-    const int tm = r & (d->tiles_m - 1);
-    r >>= __builtin_ctz(d->tiles_m);
-    const int tn = r & (d->tiles_n - 1);
-    const int64_t t = r >> __builtin_ctz(d->tiles_n);
+    uint32_t r = (uint32_t)(tile - ((const TBH_CONST int64_t*)prefix)[step]);
+    const int M = d->M, N = d->N, K = d->K;
+    const int tiles_m = d->tiles_m, tiles_n = d->tiles_n;
+    const int tm = r & (tiles_m - 1);
+    r >>= __builtin_ctz(tiles_m);
+    const int tn = r & (tiles_n - 1);
+    const int64_t t = r >> __builtin_ctz(tiles_n);
     const int m0 = tm * kTile, n0 = tn * kTile;
-    const TBH_GLOBAL T* A = reinterpret_cast<const TBH_GLOBAL T*>(d->a) + t * d->sA;
-    const TBH_GLOBAL T* B = reinterpret_cast<const TBH_GLOBAL T*>(d->b) + t * d->sB;
+    const TBH_GLOBAL T* A =
+        reinterpret_cast<const TBH_GLOBAL T*>(d->a) + t * d->sA;
+    const TBH_GLOBAL T* B =
+        reinterpret_cast<const TBH_GLOBAL T*>(d->b) + t * d->sB;
     TBH_GLOBAL T* C = reinterpret_cast<TBH_GLOBAL T*>(d->c);
-    // opaque: what a tile derives from the thread index is not held in
-    // registers across tiles
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
+    const int tid = opaque_tid();
     const int lane = tid & 63, tx = (lane & 7) * 4, ty = (lane >> 3) * 4;
     T res[4][4];
-    gemm64_tile<T, false>(A, B, d->M, d->N, d->K, d->lda, d->ldb, 0, d->K, m0, n0, tid, smem,
-                          res);
+    gemm64_tile<T, false>(A, B, M, N, K, d->lda, d->ldb, 0, K, m0, n0, tid,
+                          smem, res);
     auto quad = [&](int q) {
       return V{Trop<T>::canon(res[q][0]), Trop<T>::canon(res[q][1]), Trop<T>::canon(res[q][2]),
                Trop<T>::canon(res[q][3])};
     };
     const int nl = tile_col(wave, ty);
-    if (d->scatter == 0) {
+    const int scatter = d->scatter;
+    if (scatter == 0) {
       C += t * d->sC;
+      const int64_t ldc = d->ldc;
 #pragma unroll
       for (int q = 0; q < 4; q++)
-        *reinterpret_cast<TBH_GLOBAL V*>(C + (n0 + nl + (q >> 1)) * d->ldc + m0 + 32 * (q & 1) +
-                                         tx) = quad(q);
+        *reinterpret_cast<TBH_GLOBAL V*>(C + (n0 + nl + (q >> 1)) * ldc + m0 + 32 * (q & 1) + tx) =
+            quad(q);
     } else {
-      const int ma = __builtin_ctz((uint32_t)d->M), nb = __builtin_ctz((uint32_t)d->N);
-      C += scatter_bits(d->pc, ma + nb, (uint32_t)t) + scatter_bits(d->pc, 0, m0) +
-           scatter_bits(d->pc, ma, n0);
-      if (d->scatter == 1) {
+      const int ma = __builtin_ctz((uint32_t)M), nb = __builtin_ctz((uint32_t)N);
+      C += gemm_offset(w, (uint32_t)m0 | (uint32_t)n0 << ma | (uint32_t)t << (ma + nb));
+      if (scatter == 1) {
         // rows 0 and 1 at C positions 0 and 1: row quads are 16-byte runs
-        const int64_t at = scatter_bits(d->pc, 0, tx) + scatter_bits(d->pc, ma, nl);
-        const int64_t rh = scatter_bits(d->pc, 0, 32), c1 = scatter_bits(d->pc, ma, 1);
+        uint32_t at = 0;
+#pragma unroll
+        for (int k = 2; k < 5; k++) at |= (((uint32_t)tx >> k) & 1) << gemm_pos(w, k);
+#pragma unroll
+        for (int k = 1; k < 6; k++) at |= (((uint32_t)nl >> k) & 1) << gemm_pos(w, ma + k);
+        const uint32_t rh = 1u << gemm_pos(w, 5), c1 = 1u << gemm_pos(w, ma);
 #pragma unroll
         for (int q = 0; q < 4; q++)
-          *reinterpret_cast<TBH_GLOBAL V*>(C + at + ((q & 1) ? rh : 0) + ((q >> 1) ? c1 : 0)) =
+          *reinterpret_cast<TBH_GLOBAL V*>(C + (at | ((q & 1) ? rh : 0) | ((q >> 1) ? c1 : 0))) =
               quad(q);
       } else {
         // the tile through LDS, read back in ascending C position
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
           *reinterpret_cast<V*>(smem + ((m ^ ((n & 15) << 2)) + (n << 6))) = quad(q);
         }
         __syncthreads();
-        emit_staged<T>(C, smem, d->ep_n, 6, 15, d->pc, ma, d);
+        emit_staged<T>(C, smem, d->ep_n, 6, 15, w);
       }
     }
     __syncthreads();

@@ -1,20 +1,62 @@
 // tbh_gemm_epi.hpp -- output addressing shared by the GEMM kernels: a C in its
 // consumer's label order (GemmDesc::scatter).
 #pragma once
+#include <stddef.h>
+
 #include "tbh_device.hpp"
 
 namespace tbh {
 
-// Offset of the output bits x (bit b is GEMM output bit q0 + b) in a C whose
-// bit q sits at position pc[q] (-1: no position; only rows / columns past M /
-// N, which are not written, reach those).
-__device__ __forceinline__ int64_t scatter_bits(const int8_t* __restrict__ pc, int q0, uint32_t x) {
-  int64_t r = 0;
-  for (int b = 0; x != 0 && q0 + b < kGemmScatter; b++, x >>= 1) {
-    const int p = pc[q0 + b];
-    if ((x & 1) && p >= 0) r += (int64_t)1 << p;
+// A launch's descriptors and prefixes through the constant address space: scalar
+// loads, which do not queue behind the tiles' vector loads.
+#define TBH_CONST __attribute__((address_space(4)))
+using KGemm = const TBH_CONST GemmDesc*;
+
+// The step of tile `tile`: the last i with prefix[i] <= tile.
+__device__ __forceinline__ int gemm_step(const TBH_CONST int64_t* prefix, int nops,
+                                         int64_t tile) {
+  int lo = 0, hi = nops;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (prefix[mid] <= tile)
+      lo = mid;
+    else
+      hi = mid;
   }
-  return r;
+  return lo;
+}
+
+// The thread's index, opaque to the compiler: what a tile derives from it is
+// not held in registers across tiles.
+__device__ __forceinline__ int opaque_tid() {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
+
+// The label positions of a tile's outputs are read from a GemmDesc held a word
+// per lane, by lane reads: read from memory they are a byte each, one after
+// another.
+__device__ __forceinline__ uint32_t gemm_lanes(KGemm d) {
+  const uint32_t lane = opaque_tid() & 63;
+  return ((const uint32_t*)d)[lane < sizeof(GemmDesc) / 4 ? lane : 0];
+}
+
+// C position of output bit q (-1: none; only rows / columns past M / N, which
+// are not written, have none).
+__device__ __forceinline__ int gemm_pos(uint32_t w, uint32_t q) {
+  const uint32_t o = (uint32_t)offsetof(GemmDesc, pc) + q;
+  return (int)(int8_t)((uint32_t)__builtin_amdgcn_readlane((int)w, (int)(o >> 2)) >> (8 * (o & 3)));
+}
+
+// Offset in C of the wave-uniform output index x (m, then n, then batch bits):
+// lane p decides C position p.
+__device__ __forceinline__ int64_t gemm_offset(uint32_t w, uint32_t x) {
+  const uint32_t p = opaque_tid() & 31;
+  const uint32_t word =
+      (uint32_t)__builtin_amdgcn_ds_bpermute((int)(offsetof(GemmDesc, inv) + (p & 28)), (int)w);
+  const uint32_t q = (word >> (8 * (p & 3))) & 0xff;
+  return (int64_t)(uint32_t)__ballot(q < 32 && ((x >> (q & 31)) & 1));
 }
 
 // A pass of 2^nbits staged outputs to C: the threads read LDS in ascending C
@@ -24,27 +66,28 @@ __device__ __forceinline__ int64_t scatter_bits(const int8_t* __restrict__ pc, i
 template <typename T>
 __device__ __forceinline__ void emit_staged(TBH_GLOBAL T* __restrict__ Ct,
                                             const T* __restrict__ st, int nbits, int vm,
-                                            uint32_t smask, const int8_t* __restrict__ pc, int ma,
-                                            const GemmDesc* __restrict__ d) {
+                                            uint32_t smask, uint32_t w) {
   typedef T V __attribute__((ext_vector_type(4)));
-  const int tid = threadIdx.x;
+  const int tid = opaque_tid();
   // enumeration bit k as its share of the LDS index (xk: XORed part, ak:
   // added part; row bit b: xk = 2^b; column bit b: xk = 4 (2^b & s), ak =
   // 2^(vm+b)) and of the C offset (gk), decoded once (uniform)
+  uint32_t e[4], g[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    e[i] = (uint32_t)__builtin_amdgcn_readlane((int)w, (int)(offsetof(GemmDesc, ep) / 4) + i);
+    g[i] = (uint32_t)__builtin_amdgcn_readlane((int)w, (int)(offsetof(GemmDesc, epp) / 4) + i);
+  }
   uint32_t xk[13], ak[13], gk[13];
 #pragma unroll
   for (int k = 0; k < 13; k++) {
     xk[k] = ak[k] = gk[k] = 0;
     if (k < nbits) {
-      const int b = d->ep[k];
-      if (b < 32) {
-        xk[k] = 1u << b;
-        gk[k] = 1u << pc[b];
-      } else {
-        xk[k] = ((1u << (b - 32)) & smask) << 2;
-        ak[k] = (1u << (b - 32)) << vm;
-        gk[k] = 1u << pc[ma + b - 32];
-      }
+      const uint32_t b = (e[k / 4] >> (8 * (k % 4))) & 0xff;
+      const uint32_t bit = 1u << (b & 31);
+      xk[k] = b < 32 ? bit : (bit & smask) << 2;
+      ak[k] = b < 32 ? 0 : bit << vm;
+      gk[k] = 1u << ((g[k / 4] >> (8 * (k % 4))) & 31);
     }
   }
   // enumeration bits 0 and 1 are C positions 0 and 1 (ep lists the pass's

@@ -96,9 +96,12 @@ struct GemmDesc {
   // outputs (two passes split on the top column bit of the tile if ep_split)
   int32_t scatter;
   int8_t pc[kGemmScatter];  // -1 past the rank
+  int8_t inv[32];           // C position -> output bit, -1 past the rank
   int8_t ep[16];            // tile bit b < 32: row bit b; 32 + b: column bit b
+  int8_t epp[16];           // ... and its C position
   int32_t ep_n, ep_split;
 };
+static_assert(sizeof(GemmDesc) % 4 == 0 && sizeof(GemmDesc) <= 256, "a word per lane");
 
 // One max-plus GEMM in 64 x 64 tiles (K1b, passed by value): ksplit K ranges
 // of kpart (a multiple of 32) per tile, their maxima to ws when ksplit > 1

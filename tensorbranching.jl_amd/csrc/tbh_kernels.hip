@@ -983,6 +983,17 @@ tbh_ew_pf_kernel(const EwDesc* __restrict__ ops_g, const int64_t* __restrict__ p
 }
 
 // ---------------------------------------------------------------- K1 -----
+// Bound by the VALU at K >= 256 (planned steps of n=300 slices: 71-78 T op/s
+// of 82.1); at K = 16 .. 64 by a tile's loads, loop and stores coming one after
+// another, which three workgroups per CU overlap in part (3.4-4 TB/s), so that
+// every other access of a tile counts.  The tile's place takes shifts, the
+// descriptor's fields scalar loads (vector loads queue behind the tiles': 54.8
+// for 52.7 us below), the output's label positions lane reads of a descriptor
+// held a word per lane (read from memory, a byte each, one after another),
+// and a whole tile has no bounds to check.  Float32, before / now: M = 32768,
+// N = 64, batch 16, K = 32 61.6 / 52.7 us, K = 64 82.8 / 76.3; N = 32, K = 64
+// 50.1 / 48.5; 2048^3, batch 8, 1795 / 1750; 1024 tiles of 128 x 128 at K = 64
+// (a last wave of a third of the slots) 46.6 / 48.8.
 constexpr int BK = 16, BPAD = 4;
 
 template <typename T>
@@ -1032,13 +1043,12 @@ template <typename T, int SHAPE, int P>
 __device__ __forceinline__ void gemm_epilogue_pass(TBH_GLOBAL T* __restrict__ C,
                                                    const T (&acc)[8][GemmShape<SHAPE>::TN],
                                                    int m0, int n0, int M, int N, int64_t base,
-                                                   const int8_t* __restrict__ pc, int ma,
-                                                   const GemmDesc* __restrict__ d,
+                                                   int ma, KGemm d, uint32_t w,
                                                    T* __restrict__ st) {
   constexpr int BM = GemmShape<SHAPE>::BM, BN = GemmShape<SHAPE>::BN, TN = GemmShape<SHAPE>::TN;
   constexpr int LBM = BM == 256 ? 8 : 7;
   using V = typename Vec4<T>::type;
-  const int tid = threadIdx.x;
+  const int tid = opaque_tid();
   const int tx = tid % (BM / 8), ty = tid / (BM / 8);
   const int vm = ma < LBM ? ma : LBM;
   const bool split = d->ep_split != 0;
@@ -1068,36 +1078,34 @@ __device__ __forceinline__ void gemm_epilogue_pass(TBH_GLOBAL T* __restrict__ C,
     }
   }
   __syncthreads();
-  emit_staged<T>(C + base, st, nbits, vm, smask, pc, ma, d);
+  emit_staged<T>(C + base, st, nbits, vm, smask, w);
   __syncthreads();
 }
 
 template <typename T, int SHAPE>
 __device__ __forceinline__ void gemm_epilogue_lds(TBH_GLOBAL T* __restrict__ C,
                                                   const T (&acc)[8][GemmShape<SHAPE>::TN], int m0,
-                                                  int n0, int M, int N,
-                                                  const int8_t* __restrict__ pc, int ma,
-                                                  const GemmDesc* __restrict__ d,
-                                                  T* __restrict__ st) {
+                                                  int n0, int M, int N, int64_t base, int ma,
+                                                  KGemm d, uint32_t w, T* __restrict__ st) {
   constexpr int BN = GemmShape<SHAPE>::BN;
   constexpr int LBN = BN == 128 ? 7 : BN == 64 ? 6 : 5;
-  const int64_t base = scatter_bits(pc, 0, m0) + scatter_bits(pc, ma, n0);
-  gemm_epilogue_pass<T, SHAPE, 0>(C, acc, m0, n0, M, N, base, pc, ma, d, st);
+  gemm_epilogue_pass<T, SHAPE, 0>(C, acc, m0, n0, M, N, base, ma, d, w, st);
   if (GemmShape<SHAPE>::TN == 8 && d->ep_split)
     gemm_epilogue_pass<T, SHAPE, 1>(C, acc, m0, n0, M, N,
-                                    base + scatter_bits(pc, ma + LBN - 1, 1), pc, ma, d, st);
+                                    base + ((int64_t)1 << gemm_pos(w, ma + LBN - 1)), ma, d, w,
+                                    st);
 }
 
 // One BM x BN tile of one batch entry.  VEC: A, B 16-byte aligned with lda,
-// ldb, M, K multiples of 4.  pc != nullptr: C is written in its own label
-// order (scatter_bits; M a power of two, ma = log2 M), else column-major with
-// ldc.
+// ldb, M, K multiples of 4.  scatter: C is written in its own label order
+// (M and N powers of two; x the batch entry's output bits), else column-major
+// with ldc.
 template <typename T, bool VEC, int SHAPE>
 __device__ __forceinline__ void gemm_tile(
     const TBH_GLOBAL T* __restrict__ A, const TBH_GLOBAL T* __restrict__ B,
     TBH_GLOBAL T* __restrict__ C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-    int m0, int n0, const int8_t* __restrict__ pc, int ma, int nb, const GemmDesc* __restrict__ d,
-    T (*As)[BK][GemmShape<SHAPE>::BM], T (*Bs)[BK][GemmShape<SHAPE>::BN + BPAD],
+    int m0, int n0, int scatter, uint32_t x, KGemm d, uint32_t w0,
+    uint32_t* __restrict__ words, T (*As)[BK][GemmShape<SHAPE>::BM], T (*Bs)[BK][GemmShape<SHAPE>::BN + BPAD],
     T* __restrict__ smem) {
   constexpr int BM = GemmShape<SHAPE>::BM, BN = GemmShape<SHAPE>::BN, TN = GemmShape<SHAPE>::TN;
   constexpr int TX = BM / 8;                    // threads along M
@@ -1107,7 +1115,7 @@ __device__ __forceinline__ void gemm_tile(
   constexpr int NEA = BM * BK / 256;            // scalar loads per thread
   constexpr int NEB = (BN * BK + 255) / 256;
   using V = typename Vec4<T>::type;
-  const int tid = threadIdx.x;
+  const int tid = opaque_tid();
   const int tx = tid % TX, ty = tid / TX;
   T acc[8][TN];
 #pragma unroll
@@ -1116,8 +1124,40 @@ __device__ __forceinline__ void gemm_tile(
     for (int j = 0; j < TN; j++) acc[i][j] = Trop<T>::zero();
   const T pz = pad_zero<T>();
   T ra[VEC ? 4 * NVA : NEA], rb[VEC ? 4 * NVB : NEB];
+  // a whole tile: no bounds to check, and a wave-uniform address per vector
+  // plus one 32-bit byte offset per lane (not for 256 x 32, whose B slab half
+  // the threads load: 54.9 against 48.9 us with K = 64)
+  const bool whole = VEC && SHAPE != 2 && m0 + BM <= M && n0 + BN <= N && (K & (BK - 1)) == 0 &&
+                     lda < 1 << 27 && ldb < 1 << 24;
+  const uint32_t oa = ((uint32_t)(tid / (BM / 4)) * (uint32_t)lda + (tid % (BM / 4)) * 4) * 4;
+  const uint32_t ob = ((uint32_t)(tid >> 2) * (uint32_t)ldb + (tid & 3) * 4) * 4;
   auto load = [&](int k0) {
-    if (VEC) {
+    if (whole) {
+      auto at = [](const TBH_GLOBAL T* base, uint32_t byte) {
+        return *reinterpret_cast<const TBH_GLOBAL V*>(
+            reinterpret_cast<const TBH_GLOBAL char*>(base) + byte);
+      };
+      const TBH_GLOBAL T* Ak = A + m0 + (int64_t)k0 * lda;
+      const TBH_GLOBAL T* Bk = B + (int64_t)n0 * ldb + k0;
+#pragma unroll
+      for (int e = 0; e < NVA; e++) {
+        const V x = at(Ak + (int64_t)e * (1024 / BM) * lda, oa);
+        ra[4 * e + 0] = x.x;
+        ra[4 * e + 1] = x.y;
+        ra[4 * e + 2] = x.z;
+        ra[4 * e + 3] = x.w;
+      }
+#pragma unroll
+      for (int e = 0; e < NVB; e++) {
+        if (NVBT % 256 == 0 || tid + 256 * e < NVBT) {
+          const V x = at(Bk + (int64_t)e * 64 * ldb, ob);
+          rb[4 * e + 0] = x.x;
+          rb[4 * e + 1] = x.y;
+          rb[4 * e + 2] = x.z;
+          rb[4 * e + 3] = x.w;
+        }
+      }
+    } else if (VEC) {
       // A: vector v = tid + 256e covers m = (v % (BM/4))*4 .. +3, k = v / (BM/4)
 #pragma unroll
       for (int e = 0; e < NVA; e++) {
@@ -1193,6 +1233,7 @@ __device__ __forceinline__ void gemm_tile(
   };
   load(0);
   store(0);
+  words[tid & 63] = w0;  // for the epilogue
   __syncthreads();
   int buf = 0;
   for (int k0 = 0; k0 < K; k0 += BK) {
@@ -1229,26 +1270,34 @@ __device__ __forceinline__ void gemm_tile(
     __syncthreads();
     buf ^= 1;
   }
-  if (pc && d->scatter == 2) {
-    gemm_epilogue_lds<T, SHAPE>(C, acc, m0, n0, M, N, pc, ma, d, smem);
+  const uint32_t w = words[tid & 63];
+  const int ma = scatter ? __builtin_ctz((uint32_t)M) : 0;
+  if (scatter) C += gemm_offset(w, x | (uint32_t)m0 | (uint32_t)n0 << ma);
+  if (scatter == 2) {
+    gemm_epilogue_lds<T, SHAPE>(C, acc, m0, n0, M, N, 0, ma, d, w, smem);
     return;
   }
-  if (pc) {
+  if (scatter) {
     // row m0 + h BM/2 + tx 4 + i: its bits are disjoint parts (m0 a multiple
     // of BM, tx 4 < BM/2, i < 4), so its offset is a sum of per-part offsets;
     // the same for columns.  Row bits 0 and 1 sit at C positions 0 and 1 (pc
     // maps them so), every other bit at a position >= 2: the four rows
-    // tx 4 .. +3 are one aligned quad.
-    const int64_t rb = scatter_bits(pc, 0, m0) + scatter_bits(pc, 0, tx * 4);
-    const int64_t rh = scatter_bits(pc, 0, BM / 2);
-    const int64_t cb = scatter_bits(pc, ma, n0) + scatter_bits(pc, ma, ty * 4);
-    const int64_t ch = scatter_bits(pc, ma, BN / 2), c1 = scatter_bits(pc, ma, 1),
-                  c2 = scatter_bits(pc, ma, 2);
+    // tx 4 .. +3 are one aligned quad.  (Bits without a position belong to
+    // rows and columns past M and N: not stored.)
+    constexpr int LTX = BM == 256 ? 5 : 4, LTY = 8 - LTX;
+    auto stride = [&](int q) { return 1u << (gemm_pos(w, q) & 31); };
+    uint32_t rb = 0, cb = 0;
+#pragma unroll
+    for (int k = 0; k < LTX; k++) rb |= (tx >> k) & 1 ? stride(2 + k) : 0u;
+#pragma unroll
+    for (int k = 0; k < LTY; k++) cb |= (ty >> k) & 1 ? stride(ma + 2 + k) : 0u;
+    const uint32_t rh = stride(LTX + 2), ch = TN == 8 ? stride(ma + LTY + 2) : 0u;
+    const uint32_t c1 = stride(ma), c2 = stride(ma + 1);
 #pragma unroll
     for (int j = 0; j < TN; j++) {
       const int n = n0 + (j < 4 ? ty * 4 + j : BN / 2 + ty * 4 + (j - 4));
       if (n >= N) continue;
-      const int64_t co = cb + (j >= 4 ? ch : 0) + ((j & 1) ? c1 : 0) + ((j & 2) ? c2 : 0);
+      const uint32_t co = cb + (j >= 4 ? ch : 0) + ((j & 1) ? c1 : 0) + ((j & 2) ? c2 : 0);
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         const int m = m0 + h * (BM / 2) + tx * 4;
@@ -1296,32 +1345,42 @@ tbh_gemm_kernel(const GemmDesc* __restrict__ ops, const int64_t* __restrict__ pr
   // of a scattered epilogue (up to kEpiElems entries)
   constexpr int NA = 2 * BK * BM, NB = 2 * BK * (BN + BPAD);
   __shared__ __align__(16) T smem[NA + NB > kEpiElems ? NA + NB : kEpiElems];
+  __shared__ uint32_t words[64];  // the tile's GemmDesc
   auto As = reinterpret_cast<T(*)[BK][BM]>(smem);
   auto Bs = reinterpret_cast<T(*)[BK][BN + BPAD]>(smem + NA);
   for (int64_t tile = blockIdx.x; tile < total; tile += gridDim.x) {
-    int lo = 0, hi = nops;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (prefix[mid] <= tile)
-        lo = mid;
-      else
-        hi = mid;
+    const int step = gemm_step((const TBH_CONST int64_t*)prefix, nops, tile);
+    const KGemm d = (KGemm)(ops + step);
+    const uint32_t w = gemm_lanes(d);
+    const int64_t local = (tile - ((const TBH_CONST int64_t*)prefix)[step]);
+    const int M = d->M, N = d->N;
+    const int tiles_m = d->tiles_m, tiles_n = d->tiles_n;
+    int64_t t;
+    int tm, tn;
+    if (((tiles_m & (tiles_m - 1)) | (tiles_n & (tiles_n - 1))) == 0) {  // a planned step's
+      const int lm = __builtin_ctz(tiles_m), ln = __builtin_ctz(tiles_n);
+      tm = (int)(local & (tiles_m - 1));
+      tn = (int)((local >> lm) & (tiles_n - 1));
+      t = local >> (lm + ln);
+    } else {
+      const int64_t per = (int64_t)tiles_m * tiles_n;
+      t = local / per;
+      const int64_t rem = local - t * per;
+      tm = (int)(rem % tiles_m);
+      tn = (int)(rem / tiles_m);
     }
-    const GemmDesc* d = ops + lo;
-    const int64_t local = tile - prefix[lo];
-    const int64_t per = (int64_t)d->tiles_m * d->tiles_n;
-    const int64_t t = local / per;
-    const int64_t rem = local - t * per;
-    const int tm = (int)(rem % d->tiles_m), tn = (int)(rem / d->tiles_m);
-    const TBH_GLOBAL T* A = reinterpret_cast<const TBH_GLOBAL T*>(d->a) + t * d->sA;
-    const TBH_GLOBAL T* B = reinterpret_cast<const TBH_GLOBAL T*>(d->b) + t * d->sB;
-    const int8_t* pc = d->scatter ? d->pc : nullptr;
-    const int ma = pc ? __builtin_ctz((uint32_t)d->M) : 0;
-    const int nb = pc ? __builtin_ctz((uint32_t)d->N) : 0;
+    const TBH_GLOBAL T* A =
+        reinterpret_cast<const TBH_GLOBAL T*>(d->a) + t * d->sA;
+    const TBH_GLOBAL T* B =
+        reinterpret_cast<const TBH_GLOBAL T*>(d->b) + t * d->sB;
+    const int scatter = d->scatter;
+    uint32_t x = 0;  // the batch entry's output bits
+    if (scatter) x = (uint32_t)t << (__builtin_ctz((uint32_t)M) + __builtin_ctz((uint32_t)N));
     TBH_GLOBAL T* C = reinterpret_cast<TBH_GLOBAL T*>(d->c) +
-                      (pc ? scatter_bits(pc, ma + nb, (uint32_t)t) : t * d->sC);
-    gemm_tile<T, VEC, SHAPE>(A, B, C, d->M, d->N, d->K, d->lda, d->ldb, d->ldc, tm * BM, tn * BN,
-                             pc, ma, nb, d, As, Bs, smem);
+                      (scatter ? 0 : t * d->sC);
+    gemm_tile<T, VEC, SHAPE>(A, B, C, M, N, d->K, d->lda, d->ldb,
+                             d->ldc, tm * BM, tn * BN, scatter, x, d, w,
+                             words, As, Bs, smem);
     __syncthreads();
   }
 }

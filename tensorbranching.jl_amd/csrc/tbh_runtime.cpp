@@ -557,6 +557,13 @@ GemmDesc make_gemm(const POp& op, const std::vector<PTensor>& T, uint64_t base) 
   d.scatter = op.scatter;
   std::memcpy(d.pc, op.pc, sizeof d.pc);
   std::memcpy(d.ep, op.ep, sizeof d.ep);
+  if (op.scatter) {
+    std::memset(d.inv, -1, sizeof d.inv);
+    for (int q = 0; q < 32; q++)
+      if (d.pc[q] >= 0) d.inv[d.pc[q]] = (int8_t)q;
+    const int ma = __builtin_ctz((uint32_t)op.M);
+    for (int k = 0; k < op.ep_n; k++) d.epp[k] = d.pc[d.ep[k] < 32 ? d.ep[k] : ma + d.ep[k] - 32];
+  }
   d.ep_n = op.ep_n;
   d.ep_split = op.ep_split;
   d.tiles_m = (op.M + gemm_bm(d.shape) - 1) / gemm_bm(d.shape);
