@@ -19,7 +19,8 @@
 // of the 82.1 measured for its instruction mix; 4093 x 4095 x 4091 71.9, 67.2
 // with K1), by too little work in flight and the two launches for small ones
 // (512^3 19 us, 114 with K1's 16 tiles; 64^3 10 us, 18.6 with K1, about 6 us
-// of each the events around it).  Short K: bound by handing the maxima over,
+// of each the events around it): those whose 32 x 32 tiles fit the chip's LDS
+// with all of K at once run in tbh_gemm32_kernel instead.  Short K: bound by handing the maxima over,
 // which all four waves share (two waves alone: 4096^2 x 1024 491 us, 479 so;
 // in one round of 48 KB instead of two of 24 KB: 486).  The grouped kernel
 // runs the GEMM steps of 301 n=200 slices at 31 T op/s Int32 (K1: 19 of the
@@ -365,6 +366,133 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
   }
 }
 
+// One product in 32 x 32 tiles with the tile's whole operands in LDS (K <=
+// KMAX).  Bound by one pass through memory latency and the launch: every load
+// of a workgroup is in flight at once, by DMA without registers, where a slab
+// loop waits for each slab and a K range per workgroup needs a second launch.
+// Twice the LDS reads per MAC of the 64 x 64 tile, so only for products whose
+// tiles fit the chip at once.  The waves split K (8 of them at K <= 256, 16
+// above: 512^3 21.0 with 8, 20.6 us; 1024 x 512 x 256 20.4, 22.9 with 16; 4 at
+// K <= 64).  Float32 us per call, 64 x 64 tiles / these: 64^3 18.5 / 15.8,
+// 64^2 x 512 25.2 / 19.7, 256^3 25.0 / 17.2, 512^3 27.3 / 20.6, 511 x 512 x
+// 509 30.5 / 22.1.
+template <typename T, int KMAX, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void tbh_gemm32_kernel(const GemmSplit g, bool quads) {
+  using V = typename Quad<T>::V;
+  using U = typename Quad<T>::U;
+  typedef T W __attribute__((ext_vector_type(2)));
+  constexpr int S = KMAX + 4;  // column stride of B in LDS
+  __shared__ __align__(16) T As[32 * KMAX];
+  __shared__ __align__(16) T Bs[32 * S];
+  static_assert(32 * KMAX >= 2 * WAVES * 256, "the waves' maxima meet in A's and B's LDS");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t b = blockIdx.x;
+  const int tm = b % g.tiles_m;
+  b /= g.tiles_m;
+  const int tn = b % g.tiles_n, t = b / g.tiles_n;
+  const int m0 = tm * 32, n0 = tn * 32, M = g.M, N = g.N, K = g.K;
+  const TBH_GLOBAL T* A = reinterpret_cast<const TBH_GLOBAL T*>(g.a) + t * g.sA;
+  const TBH_GLOBAL T* B = reinterpret_cast<const TBH_GLOBAL T*>(g.b) + t * g.sB;
+  // A as [k][32 rows], B as [32 columns][k]; rows and columns past M and N
+  // repeat the last ones (their outputs are not stored)
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass does not know gfx950's 16-byte form
+  if (quads) {
+    const int m = m0 + (lane & 7) * 4, mc = m < M ? m : M - 4;
+    for (int e = wave; e * 8 < K; e += WAVES) {
+      const int k = e * 8 + (lane >> 3);
+      if (k < K)
+        __builtin_amdgcn_global_load_lds(A + k * g.lda + mc, (TBH_LDS T*)As + e * 256, 16, 0, 0);
+    }
+  } else {
+    const int m = m0 + (lane & 31), mc = m < M ? m : M - 1;
+    for (int e = wave; e * 2 < K; e += WAVES) {
+      const int k = e * 2 + (lane >> 5);
+      if (k < K)
+        __builtin_amdgcn_global_load_lds(A + k * g.lda + mc, (TBH_LDS T*)As + e * 64, 4, 0, 0);
+    }
+  }
+  for (int n = wave; n < 32; n += WAVES) {
+    const int nc = n0 + n < N ? n0 + n : N - 1;
+    const TBH_GLOBAL T* Bn = B + nc * g.ldb;
+    if (quads && KMAX >= 256) {
+      for (int k0 = 0; k0 < K; k0 += 256)
+        if (k0 + lane * 4 < K)
+          __builtin_amdgcn_global_load_lds(Bn + k0 + lane * 4, (TBH_LDS T*)Bs + n * S + k0, 16, 0,
+                                           0);
+    } else {
+      for (int k0 = 0; k0 < K; k0 += 64)
+        if (k0 + lane < K)
+          __builtin_amdgcn_global_load_lds(Bn + k0 + lane, (TBH_LDS T*)Bs + n * S + k0, 4, 0, 0);
+    }
+  }
+#endif
+  __builtin_amdgcn_s_waitcnt(0);  // the DMA's writes (a barrier does not wait for them)
+  __syncthreads();
+  // rows tx .. tx + 3, columns ty + 8 j; a quarter of K per wave
+  const int tx = (lane & 7) * 4, ty = lane >> 3;
+  T acc[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[j][i] = Trop<T>::zero();
+  const int per = (K + 2 * WAVES - 1) / (2 * WAVES) * 2;
+  const int kb = wave * per, ke = K < kb + per ? K : kb + per;
+  const T* Ap = As + tx;
+  const T* Bp = Bs + ty * S;
+  int k = kb;
+#pragma unroll 4
+  for (; k + 1 < ke; k += 2) {
+    const V a0 = *reinterpret_cast<const V*>(Ap + k * 32);
+    const V a1 = *reinterpret_cast<const V*>(Ap + k * 32 + 32);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const W w = *reinterpret_cast<const W*>(Bp + 8 * j * S + k);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        acc[j][i] = max3(acc[j][i], Trop<T>::mul(a0[i], w.x), Trop<T>::mul(a1[i], w.y));
+    }
+  }
+  if (k < ke) {
+    const V a0 = *reinterpret_cast<const V*>(Ap + k * 32);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const T w = Bp[8 * j * S + k];
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[j][i] = Trop<T>::add(acc[j][i], Trop<T>::mul(a0[i], w));
+    }
+  }
+  __syncthreads();
+  // the waves' maxima meet: wave w < 4 ends with column ty + 8 w.  Columns 0
+  // and 1 go to A's LDS, 2 and 3 to B's
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    *reinterpret_cast<V*>((j < 2 ? As : Bs) + (((j & 1) * WAVES + wave) * 64 + lane) * 4) =
+        V{acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
+  __syncthreads();
+  if (wave >= 4) return;
+  const T* red = (wave < 2 ? As : Bs) + (wave & 1) * WAVES * 256;
+  V v = *reinterpret_cast<const V*>(red + lane * 4);
+#pragma unroll
+  for (int o = 1; o < WAVES; o++) {
+    const V x = *reinterpret_cast<const V*>(red + (o * 64 + lane) * 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = Trop<T>::add(v[i], x[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = Trop<T>::canon(v[i]);
+  const int n = n0 + ty + 8 * wave, m = m0 + tx;
+  if (n >= N) return;
+  TBH_GLOBAL T* p = reinterpret_cast<TBH_GLOBAL T*>(g.c) + t * g.sC + n * g.ldc + m;
+  if (m + 4 <= M) {
+    *reinterpret_cast<TBH_GLOBAL U*>(p) = v;
+  } else {
+    if (m < M) p[0] = v.x;
+    if (m + 1 < M) p[1] = v.y;
+    if (m + 2 < M) p[2] = v.z;
+  }
+}
+
 // C = the maximum over the K ranges' workspaces, one thread per four outputs
 // of a column.
 template <typename T>
@@ -390,6 +518,29 @@ __global__ __launch_bounds__(256) void tbh_gemm_reduce_kernel(const GemmSplit g)
           Trop<T>::canon(acc.w)};
   *reinterpret_cast<TBH_GLOBAL U*>(reinterpret_cast<TBH_GLOBAL T*>(g.c) + t * g.sC + n * g.ldc +
                                    mc) = acc;
+}
+
+template <typename T>
+static void gemm32(const GemmSplit& g, bool quads, int blocks, hipStream_t s) {
+  if (g.K <= 64)
+    tbh_gemm32_kernel<T, 64, 4><<<blocks, 256, 0, s>>>(g, quads);
+  else if (g.K <= 128)
+    tbh_gemm32_kernel<T, 128, 8><<<blocks, 512, 0, s>>>(g, quads);
+  else if (g.K <= 256)
+    tbh_gemm32_kernel<T, 256, 8><<<blocks, 512, 0, s>>>(g, quads);
+  else
+    tbh_gemm32_kernel<T, 512, 16><<<blocks, 1024, 0, s>>>(g, quads);
+}
+
+// quads: every column of A and B starts at a multiple of 16 bytes and M and K
+// are multiples of 4.
+hipError_t launch_gemm32(int dtype, const GemmSplit& g, bool quads, hipStream_t s) {
+  const int blocks = g.tiles_m * g.tiles_n * g.batch;
+  if (dtype == 0)
+    gemm32<float>(g, quads, blocks, s);
+  else
+    gemm32<int32_t>(g, quads, blocks, s);
+  return hipGetLastError();
 }
 
 hipError_t launch_gemm_ksplit(int dtype, const GemmSplit& g, hipStream_t s) {

@@ -1850,6 +1850,18 @@ static bool split_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec,
   return true;
 }
 
+// Whether a standalone product runs in 32 x 32 tiles with their operands whole
+// in LDS: K up to 512 (132 KB) and every workgroup resident at once, at most
+// 3.2 per CU.  Float32 us per call, 64 x 64 tiles / 32 x 32, with 1 workgroup
+// per CU at K = 512: 512^2 27.3 / 20.6, past it 640^2 29.5 / 37.8; 2 at K =
+// 256: 1024 x 512 27.2 / 20.4, past them 768^2 28.0 / 23.3 but Int32 with odd
+// extents no faster; K = 128: 768 x 1024 23.2 / 19.9, 1024^2 23.3 / 21.3
+// (Int32 equal); K = 64: 512^2 18.9 / 16.2, 1024^2 equal, 1500 x 1000 20.8 /
+// 21.4.
+static bool resident_gemm(const tbh_ctx* ctx, int64_t tiles32, int64_t K) {
+  return K <= 512 && tiles32 * std::max<int64_t>(K, 160) <= (int64_t)ctx->num_cus * 512;
+}
+
 int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_t K, int64_t batch,
                      const void* A, int64_t lda, int64_t strideA, const void* B, int64_t ldb,
                      int64_t strideB, void* C, int64_t ldc, int64_t strideC,
@@ -1946,6 +1958,13 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
     gs.sB = strideB;
     gs.sC = strideC;
     gs.ws = 0;
+    const int64_t tm32 = (M + 31) / 32, tn32 = (N + 31) / 32;
+    if (resident_gemm(ctx, tm32 * tn32 * batch, K)) {
+      gs.tiles_m = (int32_t)tm32;
+      gs.tiles_n = (int32_t)tn32;
+      hipEvent_t ev = ctx->profiling ? ctx->prof.begin(ctx->stream) : nullptr;
+      return finish(launch_gemm32(dtype, gs, vec, ctx->stream), ev);
+    }
     if (gs.ksplit > 1) {
       const int64_t o = ctx->pool.alloc((size_t)4 * gs.ksplit * M * N * batch);
       if (o >= 0) {

@@ -31,6 +31,7 @@ hipError_t launch_gemm(int dtype, bool vec, int shape, const GemmDesc* ops, cons
                        int nops, int64_t total, int grid, hipStream_t s);
 hipError_t launch_gemm64(int dtype, const GemmDesc* ops, const int64_t* prefix, int nops,
                          int64_t total, int grid, hipStream_t s);  // tbh_gemm.hip
+hipError_t launch_gemm32(int dtype, const GemmSplit& g, bool quads, hipStream_t s);
 hipError_t launch_gemm_ksplit(int dtype, const GemmSplit& g, hipStream_t s);  // tbh_gemm.hip
 hipError_t launch_leaves(int dtype, const LeafDesc* leaves, int64_t n, hipStream_t s);
 hipError_t launch_epilogue(int dtype, const EpiDesc* e, int64_t n, void* out, hipStream_t s);
