@@ -1831,14 +1831,31 @@ int tbh_contract_max(tbh_ctx* ctx, tbh_dtype dtype, const tbh_slice* slices, siz
 // 777 Int32 238 / 92).  K1 alone takes M or K below one quad.  Products of
 // fewer than 256 tiles are split over K until 512 workgroups run, in ranges
 // of at least 128 (64^2 outputs of K = 3428: 800 / 25; 256 or 768 workgroups,
-// or ranges of 64, measured within 10% of this).
+// or ranges of 64, measured within 10% of this).  More tiles than CUs that
+// would leave a tenth of the CUs' time idle (384 tiles are 2 on half of the
+// 256 CUs) are split into the fewest ranges, up to four of at least 192, that
+// do not; whole / split, Float32 and Int32 us per call: 1500 x 1000 x 1000
+// 89 / 75, 122 / 95; 1100^2 x 2000 158 / 111, 229 / 149; 1200^2 x 777 74 / 64,
+// 101 / 79; three 1021 x 515 x 777 77 / 76, 100 / 94; 1600 x 1500 x 400 (600
+// tiles) 58 / 58, 76 / 73.  Ranges of 130 lost more to the second launch: five
+// 1000 x 300 x 390 48 / 51, 60 / 58.
 static bool split_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec,
-                       int64_t k1_tiles, GemmSplit* g) {
+                       int64_t k1_tiles, int num_cus, GemmSplit* g) {
   if (M < 4 || K < 4 || (vec && k1_tiles >= 512 && K <= 256)) return false;
   const int64_t tm = (M + 63) / 64, tn = (N + 63) / 64;
   if (tm * tn > (int64_t)1 << 28 || tm * tn * batch > (int64_t)1 << 28) return false;
   const int64_t tiles = tm * tn * batch;
-  const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(K / 128, 512 / tiles));
+  int64_t parts = std::max<int64_t>(1, std::min<int64_t>(K / 128, 512 / tiles));
+  auto even = [&](int64_t p) {
+    const int64_t per_cu = (tiles * p + num_cus - 1) / num_cus;
+    return tiles * p * 10 >= per_cu * num_cus * 9;
+  };
+  if (tiles > num_cus && !even(1))
+    for (int64_t p = 2; p <= 4 && K / p >= 192; p++)
+      if (even(p)) {
+        parts = p;
+        break;
+      }
   g->M = (int32_t)M;
   g->N = (int32_t)N;
   g->K = (int32_t)K;
@@ -1947,7 +1964,7 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
   const int64_t k1_m = (M + gemm_bm(shape) - 1) / gemm_bm(shape),
                 k1_n = (N + gemm_bn(shape) - 1) / gemm_bn(shape);
   GemmSplit gs;
-  if (split_gemm(M, N, K, batch, vec, k1_m * k1_n * batch, &gs)) {
+  if (split_gemm(M, N, K, batch, vec, k1_m * k1_n * batch, ctx->num_cus, &gs)) {
     gs.a = (uint64_t)dA;
     gs.b = (uint64_t)dB;
     gs.c = (uint64_t)dC;

@@ -31,6 +31,20 @@ def test_matches_oracle(backend, orc, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.int32])
+@pytest.mark.parametrize("shape", [(1500, 1000, 384, 1), (1500, 1000, 383, 1),
+                                   (1021, 515, 777, 3), (1600, 1500, 390, 1)])
+def test_uneven_tile_counts(backend, orc, dtype, shape):
+    """More tiles than CUs, split over K where they would not spread evenly
+    over the CUs: at the shortest range, just below it, four ranges, 600
+    tiles."""
+    M, N, K, nb = shape
+    rng = np.random.default_rng(M + K)
+    A = rand_tropical(rng, (M, K, nb), dtype, lo=-1000)
+    B = rand_tropical(rng, (K, N, nb), dtype, lo=-1000, neg_frac=0.3)
+    assert np.array_equal(backend.maxplus_gemm(A, B), orc.maxplus_gemm(A, B))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int32])
 @pytest.mark.parametrize("shape", [(66, 70, 45, 3), (37, 20, 1029, 2), (64, 64, 64, 1)])
 def test_odd_strides(backend, orc, dtype, shape):
     """Leading dimensions and batch strides past the matrices, so that most
