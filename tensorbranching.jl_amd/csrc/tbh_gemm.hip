@@ -102,7 +102,7 @@ __device__ __forceinline__ void gemm64_tile(const TBH_GLOBAL T* __restrict__ A,
     if constexpr (!EDGE) {
       const TBH_GLOBAL T* Ak = A + m0 + (int64_t)k0 * lda;
       const TBH_GLOBAL T* Bk = B + (int64_t)n0 * ldb + k0;
-      if (k0 + kSlab <= ke) {
+      if ((uint32_t)k0 + kSlab <= (uint32_t)ke) {
         ra[0] = at(Ak, oa);
         ra[1] = at(Ak + 16 * lda, oa);
         rb[0] = at(Bk, ob);
@@ -118,7 +118,7 @@ __device__ __forceinline__ void gemm64_tile(const TBH_GLOBAL T* __restrict__ A,
       }
       return;
     }
-    if (k0 + kSlab <= ke) {
+    if ((uint32_t)k0 + kSlab <= (uint32_t)ke) {
 #pragma unroll
       for (int e = 0; e < 2; e++)
         ra[e] = *reinterpret_cast<const TBH_GLOBAL U*>(A + (int64_t)(k0 + ak + 16 * e) * lda + am);
@@ -170,8 +170,8 @@ __device__ __forceinline__ void gemm64_tile(const TBH_GLOBAL T* __restrict__ A,
   if (kb < ke) store(0);
   __syncthreads();
   int buf = 0;
-  for (int k0 = kb; k0 < ke; k0 += kSlab) {
-    const bool more = k0 + kSlab < ke;
+  for (uint32_t k0 = kb; k0 < (uint32_t)ke; k0 += kSlab) {  // (ke + kSlab may pass 2^31)
+    const bool more = k0 + kSlab < (uint32_t)ke;
     if (more) load(k0 + kSlab);
     const T* As = smem + buf * (NA + NB) + wave * 8 * kTile;
     const T* Bs = smem + buf * (NA + NB) + NA + wave * 8 * kBRow;
@@ -261,7 +261,7 @@ tbh_gemm_ksplit_kernel(const GemmSplit g) {
   b /= g.tiles_n;
   const int part = b % g.ksplit, t = b / g.ksplit;
   const int m0 = tm * kTile, n0 = tn * kTile;
-  const int kb = part * g.kpart, ke = g.K < kb + g.kpart ? g.K : kb + g.kpart;
+  const int kb = part * g.kpart, ke = gemm_range_end(g, kb);
   const TBH_GLOBAL T* A = reinterpret_cast<const TBH_GLOBAL T*>(g.a) + t * g.sA;
   const TBH_GLOBAL T* B = reinterpret_cast<const TBH_GLOBAL T*>(g.b) + t * g.sB;
   T res[4][4];

@@ -104,8 +104,8 @@ struct GemmDesc {
 static_assert(sizeof(GemmDesc) % 4 == 0 && sizeof(GemmDesc) <= 256, "a word per lane");
 
 // One max-plus GEMM in 64 x 64 tiles (K1b, passed by value): ksplit K ranges
-// of kpart (a multiple of 32) per tile, their maxima to ws when ksplit > 1
-// (batch x ksplit x N x M).  M >= 4, K >= 4.
+// of kpart (a multiple of 32 when ksplit > 1) per tile, their maxima to ws when
+// ksplit > 1 (batch x ksplit x N x M).  M >= 4, K >= 4.
 struct GemmSplit {
   uint64_t a, b, c, ws;
   int32_t M, N, K, batch;
@@ -113,6 +113,10 @@ struct GemmSplit {
   int64_t sA, sB, sC;
   int32_t tiles_m, tiles_n, ksplit, kpart;
 };
+// The end of the K range that starts at kb (a sum of kb and kpart may pass 2^31).
+__host__ __device__ inline int32_t gemm_range_end(const GemmSplit& g, int32_t kb) {
+  return g.K - kb < g.kpart ? g.K : kb + g.kpart;
+}
 
 // Leaf tensor writes (vertex [0,w] or edge [0,0,0,-inf]).
 struct LeafDesc {

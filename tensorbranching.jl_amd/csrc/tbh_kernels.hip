@@ -1236,8 +1236,8 @@ __device__ __forceinline__ void gemm_tile(
   words[tid & 63] = w0;  // for the epilogue
   __syncthreads();
   int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    const bool more = k0 + BK < K;
+  for (uint32_t k0 = 0; k0 < (uint32_t)K; k0 += BK) {  // (K + BK may pass 2^31)
+    const bool more = k0 + BK < (uint32_t)K;
     if (more) load(k0 + BK);
 #pragma unroll
     for (int kk = 0; kk < BK; kk += 2) {

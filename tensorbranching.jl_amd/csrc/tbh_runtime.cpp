@@ -9,6 +9,7 @@
 //    every step of the batch once, and run one launch per wave and kernel
 //    kind across all slices, then one epilogue launch and one copy back.
 #include "tbh_runtime.hpp"
+#include "tbh_gemm_rule.hpp"
 
 #include <algorithm>
 #include <array>
@@ -1820,65 +1821,6 @@ int tbh_contract_max(tbh_ctx* ctx, tbh_dtype dtype, const tbh_slice* slices, siz
   return 0;
 }
 
-// Whether a standalone product runs on K1b (64 x 64 tiles), and in how many
-// K ranges.  K1 keeps the aligned products of at least 512 of its tiles and
-// K <= 256: there K1b's pass over the waves' maxima, once per 64 x 64 outputs,
-// costs more than its finer tiles give (4096 x 4096, kernel us K1 / K1b before
-// all four waves shared that pass: K = 16 22 / 46, 64 46 / 62, 256 136 / 151;
-// now 1024 486 / 479, 4096 1803 / 1746).  With fewer tiles K1 leaves CUs idle
-// (3072 x 2048 x 128 38 / 36; 2048^2 x 64 22 / 18; 1024^3 224 / 47; 512^3
-// 114 / 19), and unaligned extents took K1's scalar loads (three 1021 x 515 x
-// 777 Int32 238 / 92).  K1 alone takes M or K below one quad.  Products of
-// fewer than 256 tiles are split over K until 512 workgroups run, in ranges
-// of at least 128 (64^2 outputs of K = 3428: 800 / 25; 256 or 768 workgroups,
-// or ranges of 64, measured within 10% of this).  More tiles than CUs that
-// would leave a tenth of the CUs' time idle (384 tiles are 2 on half of the
-// 256 CUs) are split into the fewest ranges, up to four of at least 192, that
-// do not; whole / split, Float32 and Int32 us per call: 1500 x 1000 x 1000
-// 89 / 75, 122 / 95; 1100^2 x 2000 158 / 111, 229 / 149; 1200^2 x 777 74 / 64,
-// 101 / 79; three 1021 x 515 x 777 77 / 76, 100 / 94; 1600 x 1500 x 400 (600
-// tiles) 58 / 58, 76 / 73.  Ranges of 130 lost more to the second launch: five
-// 1000 x 300 x 390 48 / 51, 60 / 58.
-static bool split_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec,
-                       int64_t k1_tiles, int num_cus, GemmSplit* g) {
-  if (M < 4 || K < 4 || (vec && k1_tiles >= 512 && K <= 256)) return false;
-  const int64_t tm = (M + 63) / 64, tn = (N + 63) / 64;
-  if (tm * tn > (int64_t)1 << 28 || tm * tn * batch > (int64_t)1 << 28) return false;
-  const int64_t tiles = tm * tn * batch;
-  int64_t parts = std::max<int64_t>(1, std::min<int64_t>(K / 128, 512 / tiles));
-  auto even = [&](int64_t p) {
-    const int64_t per_cu = (tiles * p + num_cus - 1) / num_cus;
-    return tiles * p * 10 >= per_cu * num_cus * 9;
-  };
-  if (tiles > num_cus && !even(1))
-    for (int64_t p = 2; p <= 4 && K / p >= 192; p++)
-      if (even(p)) {
-        parts = p;
-        break;
-      }
-  g->M = (int32_t)M;
-  g->N = (int32_t)N;
-  g->K = (int32_t)K;
-  g->batch = (int32_t)batch;
-  g->tiles_m = (int32_t)tm;
-  g->tiles_n = (int32_t)tn;
-  g->kpart = (int32_t)std::min<int64_t>(((K + parts - 1) / parts + 31) / 32 * 32, 1 << 30);
-  g->ksplit = (int32_t)((K + g->kpart - 1) / g->kpart);
-  return true;
-}
-
-// Whether a standalone product runs in 32 x 32 tiles with their operands whole
-// in LDS: K up to 512 (132 KB) and every workgroup resident at once, at most
-// 3.2 per CU.  Float32 us per call, 64 x 64 tiles / 32 x 32, with 1 workgroup
-// per CU at K = 512: 512^2 27.3 / 20.6, past it 640^2 29.5 / 37.8; 2 at K =
-// 256: 1024 x 512 27.2 / 20.4, past them 768^2 28.0 / 23.3 but Int32 with odd
-// extents no faster; K = 128: 768 x 1024 23.2 / 19.9, 1024^2 23.3 / 21.3
-// (Int32 equal); K = 64: 512^2 18.9 / 16.2, 1024^2 equal, 1500 x 1000 20.8 /
-// 21.4.
-static bool resident_gemm(const tbh_ctx* ctx, int64_t tiles32, int64_t K) {
-  return K <= 512 && tiles32 * std::max<int64_t>(K, 160) <= (int64_t)ctx->num_cus * 512;
-}
-
 int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_t K, int64_t batch,
                      const void* A, int64_t lda, int64_t strideA, const void* B, int64_t ldb,
                      int64_t strideB, void* C, int64_t ldc, int64_t strideC,
@@ -1976,7 +1918,7 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
     gs.sC = strideC;
     gs.ws = 0;
     const int64_t tm32 = (M + 31) / 32, tn32 = (N + 31) / 32;
-    if (resident_gemm(ctx, tm32 * tn32 * batch, K)) {
+    if (resident_gemm(tm32 * tn32 * batch, K, ctx->num_cus)) {
       gs.tiles_m = (int32_t)tm32;
       gs.tiles_n = (int32_t)tn32;
       hipEvent_t ev = ctx->profiling ? ctx->prof.begin(ctx->stream) : nullptr;
@@ -1988,8 +1930,7 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
         offs.push_back(o);
         gs.ws = (uint64_t)(ctx->base + o);
       } else {
-        gs.ksplit = 1;  // no room for partial maxima
-        gs.kpart = (int32_t)std::min<int64_t>(((int64_t)gs.K + 31) / 32 * 32, INT32_MAX / 32 * 32);
+        whole_k(&gs);  // no room for partial maxima
       }
     }
     hipEvent_t ev = ctx->profiling ? ctx->prof.begin(ctx->stream) : nullptr;
