@@ -8,30 +8,34 @@
 
 namespace tbh {
 
-// Whether a standalone product runs on K1b (64 x 64 tiles), and in how many
-// K ranges.  K1 keeps the aligned products of at least 512 of its tiles and
-// K <= 256: there K1b's pass over the waves' maxima, once per 64 x 64 outputs,
-// costs more than its finer tiles give (4096 x 4096, kernel us K1 / K1b before
-// all four waves shared that pass: K = 16 22 / 46, 64 46 / 62, 256 136 / 151;
-// now 1024 486 / 479, 4096 1803 / 1746).  With fewer tiles K1 leaves CUs idle
-// (3072 x 2048 x 128 38 / 36; 2048^2 x 64 22 / 18; 1024^3 224 / 47; 512^3
-// 114 / 19), and unaligned extents took K1's scalar loads (three 1021 x 515 x
-// 777 Int32 238 / 92).  K1 alone takes M or K below one quad.  Products of
-// fewer than 256 tiles are split over K until 512 workgroups run, in ranges
-// of at least 128 (64^2 outputs of K = 3428: 800 / 25; 256 or 768 workgroups,
-// or ranges of 64, measured within 10% of this).  More tiles than CUs that
-// would leave a tenth of the CUs' time idle (384 tiles are 2 on half of the
-// 256 CUs) are split into the fewest ranges, up to four of at least 192, that
-// do not; whole / split, Float32 and Int32 us per call: 1500 x 1000 x 1000
-// 89 / 75, 122 / 95; 1100^2 x 2000 158 / 111, 229 / 149; 1200^2 x 777 74 / 64,
-// 101 / 79; three 1021 x 515 x 777 77 / 76, 100 / 94; 1600 x 1500 x 400 (600
-// tiles) 58 / 58, 76 / 73.  Ranges of 130 lost more to the second launch: five
-// 1000 x 300 x 390 48 / 51, 60 / 58.
+// Workgroups of 256 in one launch: it holds at most 2^32 - 1 work-items.
+constexpr int64_t kGemmMaxBlocks = ((int64_t)1 << 24) - 1;
+
+// Whether a standalone product runs on K1b (64 x 64 tiles), and in how many K
+// ranges.  K1 keeps the aligned products of at least 512 of its tiles and K <=
+// 256: there K1b's pass over the waves' maxima, once per 64 x 64 outputs, costs
+// more than its finer tiles give (4096 x 4096, kernel us K1 / K1b before all
+// four waves shared that pass: K = 16 22 / 46, 64 46 / 62, 256 136 / 151; now
+// 1024 486 / 479, 4096 1803 / 1746).  With fewer tiles K1 leaves CUs idle (3072
+// x 2048 x 128 38 / 36; 2048^2 x 64 22 / 18; 1024^3 224 / 47; 512^3 114 / 19),
+// and unaligned extents took K1's scalar loads (three 1021 x 515 x 777 Int32
+// 238 / 92).  K1 alone takes M or K below one quad, and more tiles than K1b has
+// workgroups in a launch (K1 walks its tiles).  Products of fewer than 256
+// tiles are split over K until 512 workgroups run, in ranges of at least 128
+// (64^2 outputs of K = 3428: 800 / 25; 256 or 768 workgroups, or ranges of 64,
+// measured within 10% of this).  More tiles than CUs that would leave a tenth
+// of the CUs' time idle (384 tiles are 2 on half of the 256 CUs) are split into
+// the fewest ranges, up to four of at least 192, that do not; whole / split,
+// Float32 and Int32 us per call: 1500 x 1000 x 1000 89 / 75, 122 / 95; 1100^2 x
+// 2000 158 / 111, 229 / 149; 1200^2 x 777 74 / 64, 101 / 79; three 1021 x 515 x
+// 777 77 / 76, 100 / 94; 1600 x 1500 x 400 (600 tiles) 58 / 58, 76 / 73.
+// Ranges of 130 lost more to the second launch: five 1000 x 300 x 390 48 / 51,
+// 60 / 58.
 inline bool split_gemm(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec,
                        int64_t k1_tiles, int num_cus, GemmSplit* g) {
   if (M < 4 || K < 4 || (vec && k1_tiles >= 512 && K <= 256)) return false;
   const int64_t tm = (M + 63) / 64, tn = (N + 63) / 64;
-  if (tm * tn > (int64_t)1 << 28 || tm * tn * batch > (int64_t)1 << 28) return false;
+  if (tm * tn > kGemmMaxBlocks || tm * tn * batch > kGemmMaxBlocks) return false;
   const int64_t tiles = tm * tn * batch;
   int64_t parts = std::max<int64_t>(1, std::min<int64_t>(K / 128, 512 / tiles));
   auto even = [&](int64_t p) {

@@ -1509,7 +1509,7 @@ hipError_t launch_gemm64(int dtype, const GemmDesc* ops, const int64_t* prefix, 
                          int64_t total, int grid, hipStream_t s);  // tbh_gemm.hip
 
 // The scalar-load kernel (a standalone product of M or K below 4, or of more
-// tiles than K1b indexes) has 128 x 128 tiles only.
+// tiles than K1b has workgroups in a launch) has 128 x 128 tiles only.
 template <typename T>
 static void* gemm_kernel(bool vec, int shape) {
   if (!vec) return (void*)tbh_gemm_kernel<T, false, 0>;

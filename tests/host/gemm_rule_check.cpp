@@ -2,7 +2,8 @@
 // built by tests/test_gemm_rule.py with UndefinedBehaviorSanitizer (g++, host
 // code only): over extents up to 2^31 - 1 the K ranges of a split product
 // follow one another from 0 to K, all but the last a multiple of a slab, and
-// so does the one range of a product without a workspace.
+// so does the one range of a product without a workspace; no launch passes
+// 2^32 - 1 work-items.
 #include <cstdio>
 
 #include "tbh_gemm_rule.hpp"
@@ -57,7 +58,9 @@ int main() {
                         max - 30,
                         max - 1,
                         max};
-  const int64_t batches[] = {1, 2, 3, 7, 129, 257, 512, 1000};
+  const int64_t batches[] = {1,   2,    3,         7,             129,
+                             257, 512,  1000,      (1 << 24) - 1, 1 << 24,
+                             1 << 25, 1 << 28, (1 << 28) + 1, max};
   long n = 0;
   for (int64_t M : ext)
     for (int64_t N : {(int64_t)1, (int64_t)3, (int64_t)64, (int64_t)515, (int64_t)4096})
@@ -71,6 +74,11 @@ int main() {
           if (g.M != M || g.N != N || g.K != K || g.batch != batch)
             return bad("extents", M, N, K, batch);
           if (!covers(g)) return bad("K ranges", M, N, K, batch);
+          const int64_t blocks = (int64_t)g.tiles_m * g.tiles_n * g.ksplit * g.batch;
+          const int64_t quads = (M + 3) / 4 * N * batch;
+          if (blocks * 256 >= 1ll << 32 ||
+              (g.ksplit > 1 && (quads + 255) / 256 * 256 >= 1ll << 32))
+            return bad("launch", M, N, K, batch);
           whole_k(&g);
           if (g.ksplit != 1 || !covers(g)) return bad("one range", M, N, K, batch);
         }

@@ -66,3 +66,21 @@ def test_k_up_to_2_31(backend):
             dev.put(B + 4 * k, 0)
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int32])
+def test_2_24_products(backend, dtype):
+    """A batch of 2^24 products of 4 x 1 x 5 (one A, overlapping windows as
+    B): more workgroups of a tile each than one launch holds."""
+    from tensorbranching_jl_amd import _lib
+    M, K, batch = 4, 5, 1 << 24
+    rng = np.random.default_rng(24)
+    A = np.asfortranarray(rng.integers(-99, 100, (M, K)).astype(dtype))
+    B = rng.integers(-999, 1000, batch + K - 1).astype(dtype)
+    out = np.empty((batch, M), dtype)
+    _lib.check(_lib.tbh().tbh_maxplus_gemm(
+        backend.handle, 0 if dtype == np.float32 else 1, M, 1, K, batch, A.ctypes.data, M, 0,
+        B.ctypes.data, K, 1, out.ctypes.data, M, M, _lib.TBH_HOST))
+    for m in range(M):
+        want = np.max([A[m, k] + B[k:k + batch] for k in range(K)], axis=0)
+        assert np.array_equal(out[:, m], want), m
