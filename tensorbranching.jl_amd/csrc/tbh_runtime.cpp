@@ -1906,7 +1906,7 @@ int tbh_maxplus_gemm(tbh_ctx* ctx, tbh_dtype dtype, int64_t M, int64_t N, int64_
   const int64_t k1_m = (M + gemm_bm(shape) - 1) / gemm_bm(shape),
                 k1_n = (N + gemm_bn(shape) - 1) / gemm_bn(shape);
   GemmSplit gs;
-  if (split_gemm(M, N, K, batch, vec, k1_m * k1_n * batch, ctx->num_cus, &gs)) {
+  if (split_gemm(dtype, M, N, K, batch, vec, k1_m * k1_n * batch, ctx->num_cus, &gs)) {
     gs.a = (uint64_t)dA;
     gs.b = (uint64_t)dB;
     gs.c = (uint64_t)dC;

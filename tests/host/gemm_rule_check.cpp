@@ -3,7 +3,8 @@
 // code only): over extents up to 2^31 - 1 the K ranges of a split product
 // follow one another from 0 to K, all but the last a multiple of a slab, and
 // so does the one range of a product without a workspace; no launch passes
-// 2^32 - 1 work-items.
+// 2^32 - 1 work-items.  And at the lines between the two kernels, each product
+// runs on the one that measured faster.
 #include <cstdio>
 
 #include "tbh_gemm_rule.hpp"
@@ -27,7 +28,43 @@ static bool covers(const GemmSplit& g) {
   return at == g.K;
 }
 
+struct Line {
+  int dtype;  // 0 Float32, 1 Int32
+  int64_t M, N, K, batch;
+  bool k1;
+};
+// (extents in multiples of 4 are aligned products)
+static const Line kLines[] = {
+    // narrow outputs in 256 x 32 tiles: 224 of them Float32, 192 at K <= 16,
+    // 160 Int32
+    {0, 256 * 224, 8, 64, 1, true}, {0, 256 * 223, 8, 64, 1, false},
+    {0, 256 * 192, 8, 16, 1, true}, {0, 256 * 191, 8, 16, 1, false},
+    {1, 256 * 160, 8, 64, 1, true}, {1, 256 * 159, 8, 64, 1, false},
+    {0, 102400, 20, 1024, 1, true}, {1, 102400, 20, 1024, 1, true},
+    {0, 768, 5, 452, 160, true},    {1, 600, 5, 64, 100, false},
+    {1, 324, 3, 260, 1256, true},
+    // K > 256: K1's tiles spread evenly, or not
+    {0, 4096, 4096, 260, 1, true},  {1, 4096, 4096, 260, 1, true},
+    {0, 2048, 4096, 512, 1, true},  {1, 2048, 4096, 512, 1, false},
+    {0, 8192, 8192, 1024, 1, true}, {0, 3072, 3072, 1024, 1, false},
+    {0, 6144, 6144, 4096, 1, true}, {0, 4096, 4096, 4096, 1, false},
+    {0, 8, 12, 712, 1024, false},
+    // unaligned, short K
+    {0, 71, 68, 15, 1493, true},    {1, 200001, 65, 5, 1, true},
+    {0, 85, 477, 6, 3097, true},    {0, 191, 4039, 5, 16, false},
+    {0, 200001, 65, 17, 1, false},  {0, 50, 3133, 7, 586, false},
+};
+
 int main() {
+  for (const Line& l : kLines) {
+    const bool vec = l.M % 4 == 0 && l.K % 4 == 0;
+    const int shape = vec ? gemm_shape(l.M, l.N) : 0;
+    const int64_t tm = (l.M + gemm_bm(shape) - 1) / gemm_bm(shape),
+                  tn = (l.N + gemm_bn(shape) - 1) / gemm_bn(shape);
+    GemmSplit g{};
+    if (split_gemm(l.dtype, l.M, l.N, l.K, l.batch, vec, tm * tn * l.batch, 256, &g) == l.k1)
+      return bad("line", l.M, l.N, l.K, l.batch);
+  }
   const int64_t max = INT32_MAX;
   const int64_t ext[] = {4,    5,    63,   64,   65,    100,           513,           1021,
                          4096, 1500, 9999, 1024, 65536, (1ll << 20) + 1};
@@ -67,7 +104,7 @@ int main() {
       for (int64_t K : ks)
         for (int64_t batch : batches) {
           GemmSplit g{};
-          if (!split_gemm(M, N, K, batch, false, ((M + 127) / 128) * ((N + 127) / 128) * batch,
+          if (!split_gemm(0, M, N, K, batch, false, ((M + 127) / 128) * ((N + 127) / 128) * batch,
                           256, &g))
             continue;
           n++;
