@@ -162,7 +162,7 @@ struct PosMap {
 int step_shape(const PlanOptions& opt, int na, int nb, int nk, int nt) {
   const int shape = gemm_shape((int64_t)1 << na, (int64_t)1 << nb, opt.gemm_tiles);
   // (extents the kernel's 32-bit offsets hold)
-  if (opt.gemm_tiles <= 0 || na < 6 || nb < 6 || nk < 4 || na > 24 || nk > 24) return shape;
+  if (opt.lean || opt.gemm_tiles <= 0 || na < 6 || nb < 6 || nk < 4 || na > 24 || nk > 24) return shape;
   const int tiles = std::max(0, na - __builtin_ctz(gemm_bm(shape))) +
                     std::max(0, nb - __builtin_ctz(gemm_bn(shape))) + nt;
   return tiles < 8 ? kGemm64 : shape;
@@ -214,8 +214,8 @@ struct Builder {
     // n=200 at sc 20: tiled EW 3.33 ms when only R > 8 splits, 1.99 from 7,
     // 1.92 from 6, 1.85 from 5; n=300 at sc 25 the same within 1%.  Below
     // 2^18 configurations a second launch costs more than the loop.)
-    if ((R.size() >= 7 && op.nP < 20 && (op.nP + R.size() >= 18 || R.size() > 8)) ||
-        R.size() > (size_t)kMaxReduce) {
+    const bool seven = !opt.lean && R.size() >= 7 && op.nP + R.size() >= 18;
+    if (((R.size() > 8 || seven) && op.nP < 20) || R.size() > (size_t)kMaxReduce) {
       // split-K: keep the last s reduced labels in a temporary (more
       // outputs, shorter loops), then reduce them in a second step
       const int s_keep = R.size() > (size_t)kMaxReduce && op.nP >= 20
@@ -1285,7 +1285,7 @@ int plan_slice(const SliceIn& s_in, const PlanOptions& opt_in, SlicePlan* out, s
   // batched: the subtrees that run as units; a single leaf, and every leaf
   // and step outside them, as below
   std::vector<int32_t> prio, order;
-  const bool units = opt.batched && opt.units;
+  const bool units = opt.batched && opt.units && !opt.lean;
   if (units) {
     // every label by sorted_key's rule (elimination nodes are 0 .. nn:
     // counted, not compared)

@@ -140,6 +140,11 @@ struct PlanOptions {
   int gemm_tiles = 1;
   // subtrees whose tensors fit in LDS run as units (batched only)
   bool units = true;
+  // the plan of less memory, for a slice whose default plan does not fit the
+  // pool: no units (their outputs live from the first wave on), no temporary
+  // for steps of 7 or 8 reduced labels, no 64 x 64 GEMM tiles (some of whose
+  // outputs need a permuting step)
+  bool lean = false;
   // tiled EW steps: outer labels absent from the larger sub-tensor first,
   // so that consecutive tiles reuse it from LDS; false: C's label order
   bool reuse_order = true;

@@ -668,13 +668,34 @@ size_t desc_bytes(const SlicePlan& P) {
   // a step: its descriptor, its prefix entry and (per-step profiling) its
   // one-step prefix pair
   return P.ops.size() * (std::max(sizeof(EwDesc), sizeof(GemmDesc)) + 3 * sizeof(int64_t)) +
-         P.units.size() * sizeof(UnitDesc) + P.items.size() * sizeof(UnitItem) +
+         P.leaves.size() * sizeof(LeafDesc) + P.units.size() * sizeof(UnitDesc) + P.items.size() * sizeof(UnitItem) +
          P.unit_w.size() * sizeof(uint32_t) + P.ext.size() * sizeof(UnitExt) + sizeof(EpiDesc) + 4;
 }
 
-size_t desc_batch_overhead(int levels) {
-  const size_t slots = (size_t)kKinds * (size_t)(levels + 1);
+static size_t slots_overhead(size_t slots) {
   return 256 * (6 + 3 * slots) + sizeof(int64_t) * slots;
+}
+size_t desc_batch_overhead(int levels) {
+  return slots_overhead((size_t)kKinds * (size_t)(levels + 1));
+}
+
+bool slice_fits(const SlicePlan& P, size_t region, size_t desc_budget) {
+  if (!P.empty && (size_t)P.arena_bytes > region) return false;
+  const size_t d = desc_bytes(P);
+  if (d + desc_batch_overhead(P.nlevels) <= desc_budget) return true;
+  // closer: the launches that the slice has
+  std::vector<char> used((size_t)kKinds * (P.nlevels + 1), 0);
+  for (const PUnit& u : P.units) used[(size_t)kUnitKind * (P.nlevels + 1) + u.level] = 1;
+  for (const POp& op : P.ops) used[(size_t)op_kind(op) * (P.nlevels + 1) + op.level] = 1;
+  const size_t slots = (size_t)std::count(used.begin(), used.end(), 1);
+  return d + slots_overhead(slots) <= desc_budget;
+}
+
+int plan_lean(const tbh_ctx* ctx, const SliceOwned& slice, bool batched, SlicePlan* out,
+              std::string* err) {
+  PlanOptions opt = plan_options(ctx, batched);
+  opt.lean = true;
+  return plan_slice(slice.in, opt, out, err);
 }
 
 namespace {
@@ -800,9 +821,9 @@ struct IssueJob {
   bool prof = false, per_step = false;
   int bidx = 0, H = 0;
   size_t nb = 0;
-  int64_t nepi = 0;
+  int64_t nleaves = 0, nepi = 0;
   int unit_levels = 0;   // deepest unit
-  size_t o_items = 0, o_w = 0, o_ext = 0, o_epi = 0, o_res = 0;
+  size_t o_leaves = 0, o_items = 0, o_w = 0, o_ext = 0, o_epi = 0, o_res = 0;
   char* dbase = nullptr;     // the batch's descriptors on the device
   const char* hb = nullptr;  // ... and in the pinned staging buffer (step tags)
   hipEvent_t up = nullptr, done = nullptr;
@@ -850,6 +871,12 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
     ctx->stats.launches++;
     return r;
   };
+  if (e == hipSuccess && j.nleaves) {  // of slices without units
+    e = injected() ? hipErrorLaunchFailure
+                   : launch_leaves(dtype, (const LeafDesc*)(dbase + j.o_leaves), j.nleaves,
+                                   ctx->stream);
+    ctx->stats.launches++;
+  }
   if (e == hipSuccess) e = units(0);
   // one launch per kernel kind and level (direct EW, tiled EW, GEMM); in
   // the per-step profiling mode every step alone, tagged with its shape
@@ -1083,9 +1110,9 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   std::vector<std::vector<int64_t>> pfx(W, std::vector<int64_t>(1, 0));
   std::vector<double> lvl_bytes(W, 0.0), lvl_macs(W, 0.0);
   std::vector<std::vector<std::pair<double, double>>> step_work(per_step ? W : 0);
-  // per slice: its first item, vertex weight, memory tensor and epilogue entry
+  // per slice: its first leaf, item, vertex weight, memory tensor and epilogue entry
   struct Start {
-    int64_t item = 0, w = 0, ext = 0, epi = 0;
+    int64_t leaf = 0, item = 0, w = 0, ext = 0, epi = 0;
   };
   std::vector<Start> first(nb + 1);
   int unit_levels = 0;
@@ -1095,6 +1122,7 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
     first[i + 1] = first[i];
     first[i + 1].epi += P.empty || !P.unit_root;
     if (P.empty) continue;
+    first[i + 1].leaf += (int64_t)P.leaves.size();
     first[i + 1].ext += (int64_t)P.ext.size();
     first[i + 1].item += (int64_t)P.items.size();
     first[i + 1].w += (int64_t)P.unit_w.size();
@@ -1133,6 +1161,7 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
     off = o + bytes;
     return o;
   };
+  const size_t o_leaves = take((size_t)first[nb].leaf * sizeof(LeafDesc));
   const size_t o_items = take((size_t)first[nb].item * sizeof(UnitItem));
   const size_t o_w = take((size_t)first[nb].w * sizeof(uint32_t));
   const size_t o_ext = take((size_t)first[nb].ext * sizeof(UnitExt));
@@ -1178,6 +1207,13 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
       std::memcpy(hb + o_epi + (size_t)first[i].epi * sizeof(EpiDesc), &e, sizeof e);
     }
     if (P.empty) return;
+    LeafDesc* ld = reinterpret_cast<LeafDesc*>(hb + o_leaves) + first[i].leaf;
+    for (const PLeaf& L : P.leaves) {
+      ld->p = b + (uint64_t)P.tensors[L.tensor].off;
+      ld->kind = L.kind;
+      ld->wbits = (int32_t)L.wbits;
+      ld++;
+    }
     std::vector<int32_t>& loc = local[t];
     std::fill(loc.begin(), loc.end(), 0);
     const int32_t* st = &start[i * W];
@@ -1262,8 +1298,10 @@ int BatchRunner::enqueue(int dtype, const std::vector<const SliceOwned*>& slices
   job->bidx = bidx;
   job->H = H;
   job->nb = nb;
+  job->nleaves = first[nb].leaf;
   job->nepi = first[nb].epi;
   job->unit_levels = unit_levels;
+  job->o_leaves = o_leaves;
   job->o_ext = o_ext;
   job->o_items = o_items;
   job->o_w = o_w;
@@ -1323,6 +1361,7 @@ int execute_batched(tbh_ctx* ctx, int dtype, const std::vector<const SliceOwned*
   // starts while the later slices are still being planned
   const double first_frac = std::min(1.0, std::max(0.01, ctx->tune.first_batch));
   size_t i0 = 0;
+  SlicePlan lean;  // of a batch's first slice (packed before the next batch)
   for (int bidx = 0; i0 < n && status == 0; bidx++) {
     auto t_plan = std::chrono::steady_clock::now();
     // admit slices while their arenas fit the region (waiting for plans)
@@ -1338,13 +1377,25 @@ int execute_batched(tbh_ctx* ctx, int dtype, const std::vector<const SliceOwned*
         status = TBH_EINVAL;
         break;
       }
-      const size_t a = P->empty ? 0 : (size_t)P->arena_bytes, d = desc_bytes(*P);
-      const int lv = std::max(levels, P->nlevels);
+      size_t a = P->empty ? 0 : (size_t)P->arena_bytes, d = desc_bytes(*P);
+      int lv = std::max(levels, P->nlevels);
       // a batch is bounded by its arenas and by its descriptors
       if (i1 > i0 &&
           (arena + a > cap || desc + d + desc_batch_overhead(lv) > dbudget))
         break;
-      if (a > region || d + desc_batch_overhead(lv) > dbudget) {
+      if (i1 == i0 && !slice_fits(*P, region, dbudget)) {
+        // too large as planned: a plan of less memory may fit
+        if (plan_lean(ctx, *slices[i1], true, &lean, &err)) {
+          set_error("slice " + std::to_string(i1) + ": " + err);
+          status = TBH_EINVAL;
+          break;
+        }
+        P = &lean;
+        a = P->empty ? 0 : (size_t)P->arena_bytes;
+        d = desc_bytes(*P);
+        lv = P->nlevels;
+      }
+      if (i1 == i0 && P == &lean && !slice_fits(*P, region, dbudget)) {
         set_error(a > region ? "slice arena (" + std::to_string(a) + " bytes) does not fit the pool"
                              : "slice descriptors (" + std::to_string(d) +
                                    " bytes) do not fit the pool");
@@ -1724,6 +1775,9 @@ static int contract_impl(tbh_ctx* ctx, tbh_dtype dtype, const tbh_slice* slices,
   if (rc) return rc;
   for (size_t i = 0; i < n; i++) {
     rc = execute_plain(ctx, dtype, owned[i], plans[i], add_r, out + i);
+    std::string err;
+    if (rc == TBH_ENOMEM && plan_lean(ctx, owned[i], false, &plans[i], &err) == 0)
+      rc = execute_plain(ctx, dtype, owned[i], plans[i], add_r, out + i);
     if (rc) return rc;
   }
   return 0;
@@ -1773,7 +1827,11 @@ int tbh_contract_slices_noalloc(tbh_ctx* ctx, tbh_dtype dtype, const tbh_slice* 
   int rc = plan_all(ctx, ptrs, false, &plans);
   if (rc) return rc;
   for (size_t i = 0; i < n; i++) {
-    const size_t need = plain_device_bytes(owned[i], plans[i]);
+    size_t need = plain_device_bytes(owned[i], plans[i]);
+    std::string err;
+    if (need > (size_t)TBH_NOALLOC_SCRATCH_BYTES &&
+        plan_lean(ctx, owned[i], false, &plans[i], &err) == 0)
+      need = plain_device_bytes(owned[i], plans[i]);
     if (need > (size_t)TBH_NOALLOC_SCRATCH_BYTES) {
       set_error("slice " + std::to_string(i) + " needs " + std::to_string(need) +
                 " bytes of device memory; tbh_contract_slices_noalloc holds at most " +

@@ -295,6 +295,12 @@ class BatchRunner {
 // (the 256-byte alignment of every (kernel kind, level) array).
 size_t desc_bytes(const SlicePlan& P);
 size_t desc_batch_overhead(int levels);
+// Whether a slice fits a batch of its own: its arena a region, its descriptors
+// their share of the pool.
+bool slice_fits(const SlicePlan& P, size_t region, size_t desc_budget);
+// Plans a slice again for less memory (PlanOptions::lean).
+int plan_lean(const tbh_ctx* ctx, const SliceOwned& slice, bool batched, SlicePlan* out,
+              std::string* err);
 
 // Executes the plans of `slices` (plan_of(i) may block until slice i is
 // planned, nullptr = planning failed); results[i] (dtype bits) = root + r

@@ -122,18 +122,24 @@ struct ServeState {
       std::string err = rc ? std::string(tbh_last_error()) : std::string();
       // admission by footprint: every slice's arena must fit the region an
       // idle pool gives a round, or the request is refused alone
-      for (size_t i = 0; !rc && i < plans.size(); i++)
-        if (arena_of(plans[i]) > region_cap) {
+      for (size_t i = 0; !rc && i < plans.size(); i++) {
+        if (slice_fits(plans[i], region_cap, desc_cap)) continue;
+        if (plan_lean(ctx, *ptrs[i], true, &plans[i], &err)) {
+          rc = TBH_EINVAL;
+        } else if (slice_fits(plans[i], region_cap, desc_cap)) {
+          continue;
+        } else if (arena_of(plans[i]) > region_cap) {
           rc = TBH_ENOMEM;
           err = "slice " + std::to_string(i) + ": arena of " +
                 std::to_string(arena_of(plans[i])) + " bytes exceeds the serving region (" +
                 std::to_string(region_cap) + " bytes of the pool)";
-        } else if (desc_bytes(plans[i]) + desc_batch_overhead(plans[i].nlevels) > desc_cap) {
+        } else {
           rc = TBH_ENOMEM;
           err = "slice " + std::to_string(i) + ": descriptors of " +
                 std::to_string(desc_bytes(plans[i])) + " bytes exceed the pool's share for them (" +
                 std::to_string(desc_cap) + " bytes)";
         }
+      }
       {
         std::lock_guard<std::mutex> g(m);
         if (r->status == TBH_FAILED) continue;  // cancelled while planning
