@@ -821,6 +821,8 @@ struct UnitBuilder {
   int32_t nl;
   // log2 of a unit's MACs at most: 8 waves take about 3 us for 2^17
   static constexpr double kUnitMacs = 131072.0;
+  // (items are indexed by 16 bits: one per node, and one more per 64 MACs)
+  static constexpr int32_t kUnitNodes = 0x7fff;
   // tree node (leaf or internal): inside a unit, the output of a unit of
   // leaves (or a leaf in memory), or the output of a unit that also reads
   // tensors from memory
@@ -829,6 +831,19 @@ struct UnitBuilder {
   std::vector<char> fit;             // the node's whole subtree may be one unit
   std::vector<char> small;           // the node's step alone may be in a unit
   std::vector<int32_t> parent, level, node_at, vert, taken;
+  // what a unit of an internal node would hold at least (mark(): its whole
+  // subtree; mark_mixed(): down to units, steps and what is not small): build()
+  // refuses more, and visiting the nodes to find that out at every node of a
+  // long chain takes planning time quadratic in its length
+  struct Need {
+    double macs;
+    int32_t nodes, verts;
+    int64_t lds;  // tensors from memory
+  };
+  std::vector<Need> need;
+  int64_t wasted = 0;                // nodes visited by builds that failed
+  std::vector<int32_t> most;         // the nodes that a unit below may have (empty: any)
+  size_t mixed0 = 0, mixed1 = 0;     // P.units that read tensors from memory, by falling node
   std::vector<int32_t> off;          // LDS offset of a unit's tensor
   // the places of the labels of a unit's tensors, ascending, 16 per tree node
   std::vector<int32_t> place;
@@ -865,12 +880,12 @@ struct UnitBuilder {
     level.assign(tot, 0);
     off.assign(tot, 0);
     vert.assign(nl, -1);
+    need.reserve(nn);
     place.resize(16 * (size_t)tot);
     P.items.reserve(3 * (size_t)tot);
     P.unit_steps.reserve(nn);
     P.unit_w.reserve(nl);
     std::vector<int64_t> peak(tot, 0);
-    std::vector<double> macs(tot, 0.0);
     for (int32_t i = 0; i < nl; i++) fit[i] = 1;
     for (int32_t j = 0; j < nn; j++) {
       const int32_t o = nl + j, x = s.tree[2 * j], y = s.tree[2 * j + 1];
@@ -883,12 +898,38 @@ struct UnitBuilder {
       const int64_t first = std::max(peak[x], peak[y]);
       const int64_t second = peak[x] >= peak[y] ? sx + peak[y] : sy + peak[x];
       peak[o] = std::max(std::max(first, second), sx + sy + so);
-      macs[o] = macs[x] + macs[y] + (uni[j] < 31 ? (double)(1u << uni[j]) : 1e18);
+      need.push_back(joined(o, need_of(x, true), need_of(y, true)));
       small[o] = uni[j] <= kUnitBits && rank(o) <= kUnitRank &&
                  uni[j] - rank(o) <= kUnitReduce && rank(x) <= kUnitOperand &&
                  rank(y) <= kUnitOperand;
-      fit[o] = fit[x] && fit[y] && small[o] && macs[o] <= kUnitMacs &&
+      fit[o] = fit[x] && fit[y] && small[o] && may_hold(need[j]) &&
                std::max(first, second) <= kUnitLds;
+    }
+  }
+
+  // inner: the node is part of the unit, else it is read from memory
+  Need need_of(int32_t x, bool inner) const {
+    if (x < nl) return {0, 0, rank(x) == 1, 0};
+    if (inner) return need[x - nl];
+    return {0, 1, 0, (int64_t)1 << rank(x)};
+  }
+  Need joined(int32_t o, const Need& a, const Need& b) const {
+    const int u = uni[o - nl];
+    return {a.macs + b.macs + (u < 31 ? (double)(1u << u) : 1e18), a.nodes + b.nodes + 1,
+            a.verts + b.verts, a.lds + b.lds};
+  }
+  static bool may_hold(const Need& n) {
+    return n.macs <= kUnitMacs && n.nodes <= kUnitNodes && 4 + 2 * n.verts + n.lds <= kUnitLds;
+  }
+
+  // need[] of the units that also read tensors from memory, once the units of
+  // leaves are built
+  void mark_mixed() {
+    auto inner = [&](int32_t x) { return small[x] && in_unit[x] == kOutside; };
+    for (int32_t j = 0; j + 1 < nl; j++) {
+      if (!inner(nl + j)) continue;
+      const int32_t x = s.tree[2 * j], y = s.tree[2 * j + 1];
+      need[j] = joined(nl + j, need_of(x, inner(x)), need_of(y, inner(y)));
     }
   }
 
@@ -927,8 +968,7 @@ struct UnitBuilder {
         node_at.push_back(c);
       }
     }
-    // (items are indexed by 16 bits: one per node, and one more per 64 MACs)
-    if (work > kUnitMacs || node_at.size() > 0x7fff) return false;
+    if (work > kUnitMacs || node_at.size() > (size_t)kUnitNodes) return false;
     // breadth first: node_at is in descending level order from the back
     // LDS: the edge tensor, the vertex tensors, then the internal tensors,
     // blocks of a level's dead operands reused one level later
@@ -1071,20 +1111,42 @@ struct UnitBuilder {
   void run() {
     const int32_t nn = nl - 1;
     mark();
+    // Below a node whose tensors do not fit every node is tried, until that has
+    // visited kPatience nodes per node of the tree; from then on only those of
+    // half its size or less (trees of MIS networks visit less than one).
+    constexpr int64_t kPatience = 8;
+    const int64_t patience = kPatience * (nl + nn);
+    auto attempt = [&](int32_t o, bool mixed) {
+      const int32_t size = need[o - nl].nodes;
+      int32_t below = most.empty() ? INT32_MAX : most[o];
+      if (wasted <= patience || size <= below) {
+        if (build(o, mixed)) return true;
+        wasted += (int64_t)node_at.size();
+        below = size / 2;
+      }
+      if (most.empty()) most.assign(nl + nn, INT32_MAX);
+      for (int q = 0; q < 2; q++) most[s.tree[2 * (o - nl) + q]] = below;
+      return false;
+    };
     std::vector<int32_t> roots;
     for (int32_t o = nl + nn - 1; o >= nl; o--)
       if (fit[o] && (parent[o] < 0 || !fit[parent[o]])) roots.push_back(o);
     while (!roots.empty()) {
       const int32_t o = roots.back();
       roots.pop_back();
-      if (build(o, false)) continue;
+      if (attempt(o, false)) continue;
       for (int q = 0; q < 2; q++) {
         const int32_t c = s.tree[2 * (o - nl) + q];
         if (c >= nl) roots.push_back(c);
       }
     }
+    mark_mixed();
+    most.clear();
+    mixed0 = P.units.size();
     for (int32_t o = nl + nn - 1; o >= nl; o--)
-      if (small[o] && in_unit[o] == kOutside && !build(o, true)) small[o] = 0;
+      if (small[o] && in_unit[o] == kOutside && (!may_hold(need[o - nl]) || !attempt(o, true)))
+        small[o] = 0;
+    mixed1 = P.units.size();
     for (int32_t i = 0; i < nl; i++) {
       if (in_unit[i]) continue;
       PUnit u;
@@ -1098,11 +1160,11 @@ struct UnitBuilder {
     }
   }
 
-  // index of the unit whose output is o
+  // index of the unit that reads tensors from memory and whose output is o
   int unit_of(int32_t o) const {
-    for (size_t k = P.units.size(); k-- > 0;)
-      if (P.units[k].tensor == o) return (int)k;
-    return -1;
+    auto it = std::lower_bound(P.units.begin() + mixed0, P.units.begin() + mixed1, o,
+                               [](const PUnit& u, int32_t x) { return u.tensor > x; });
+    return (int)(it - P.units.begin());
   }
 
   // output bit -> position in the layout its consumer reads
