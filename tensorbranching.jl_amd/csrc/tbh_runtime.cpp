@@ -846,13 +846,15 @@ hipError_t issue_batch(tbh_ctx* ctx, IssueJob& j) {
   const auto& pfx = j.pfx;
   char* dbase = j.dbase;
   // a launch failure forced from the host (error-path tests), checked
-  // before every launch of the batch; nothing is launched in its place
-  // (the units' launch counts as many as the levels it runs)
-  auto injected = [ctx](int64_t n = 1) {
+  // before every launch of the batch; nothing is launched in its place.
+  // Counted in waves of steps (stats.launches counts launches): the launch of
+  // the units that read no tensor from memory runs as many as its deepest
+  // unit has levels, every other launch one
+  auto injected = [ctx](int64_t waves = 1) {
     int64_t v = ctx->inject_launch_failure.load();
     while (v >= 0)
-      if (ctx->inject_launch_failure.compare_exchange_weak(v, std::max<int64_t>(-1, v - n)))
-        return v < n;
+      if (ctx->inject_launch_failure.compare_exchange_weak(v, std::max<int64_t>(-1, v - waves)))
+        return v < waves;
     return false;
   };
   if (e == hipSuccess && j.up) e = hipStreamWaitEvent(ctx->stream, j.up, 0);

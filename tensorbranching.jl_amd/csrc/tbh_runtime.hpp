@@ -189,9 +189,9 @@ struct tbh_ctx {
   tbh_tuning tune{};   // planner / launch parameters (tbh_set_tuning, tbh_autotune)
   bool profiling = false;
   tbh::Profiler prof;
-  // error-path tests: after this many batched launches the next one reports
-  // a launch failure instead of launching, once (-1: never;
-  // TBH_INJECT_LAUNCH_FAILURE at tbh_create)
+  // error-path tests: the batched launch that holds the wave of steps after
+  // this many (issue_batch) reports a launch failure instead of launching,
+  // once (-1: never; TBH_INJECT_LAUNCH_FAILURE at tbh_create)
   std::atomic<int64_t> inject_launch_failure{-1};
   tbh::Issuer issuer;  // batched launch sequences
   std::mutex serve_mu;   // guards `serve` (never held across an execution)
