@@ -61,12 +61,18 @@ inline bool k1_better(int dtype, int64_t M, int64_t N, int64_t K, int64_t batch,
 // at least 128 (64^2 outputs of K = 3428: 800 / 25; 256 or 768 workgroups, or
 // ranges of 64, measured within 10% of this).  More tiles than CUs that would
 // leave a tenth of the CUs' time idle (384 tiles are 2 on half of the 256 CUs)
-// are split into the fewest ranges, up to four of at least 192, that do not;
-// whole / split, Float32 and Int32 us per call: 1500 x 1000 x 1000 89 / 75, 122
-// / 95; 1100^2 x 2000 158 / 111, 229 / 149; 1200^2 x 777 74 / 64, 101 / 79;
-// three 1021 x 515 x 777 77 / 76, 100 / 94; 1600 x 1500 x 400 (600 tiles) 58 /
-// 58, 76 / 73. Ranges of 130 lost more to the second launch: five 1000 x 300 x
-// 390 48 / 51, 60 / 58.
+// are split into the fewest ranges, up to four, that do not, while K / p >= 192
+// (ranges are rounded up to slabs; what is left of K for the last, which starts
+// last, may be shorter: K = 777 in four is 224, 224, 224 and 105). Whole /
+// split, Float32 and Int32 us per call: 1500 x 1000 x 1000 89 / 75, 122 / 95;
+// 1100^2 x 2000 158 / 111, 229 / 149; 1200^2 x 777 74 / 64, 101 / 79; three
+// 1021 x 515 x 777 77 / 76, 100 / 94; 1600 x 1500 x 400 (600 tiles) 58 / 58, 76
+// / 73. The second launch is made up for from K / p of (Float32 / Int32) 130 /
+// 100 at 1100^2 in three ranges, 160 / 150 at 1200^2 and 190 / 150 at 1500 x
+// 1000 in two, 150 / 120 at five 1000 x 300 in three, 210 / 165 at 1600 x 1500
+// in two, 190 / 145 at three 1021 x 515 in four (97 there loses 12% / 5%): from
+// 192 on all gain or are equal. Ranges that differ by at most a slab are equal
+// or up to 8% slower: the short last one fills the end of the launch.
 inline bool split_gemm(int dtype, int64_t M, int64_t N, int64_t K, int64_t batch, bool vec,
                        int64_t k1_tiles, int num_cus, GemmSplit* g) {
   if (M < 4 || K < 4) return false;
@@ -98,13 +104,18 @@ inline bool split_gemm(int dtype, int64_t M, int64_t N, int64_t K, int64_t batch
 }
 
 // Whether a standalone product runs in 32 x 32 tiles with their operands whole
-// in LDS: K up to 512 (132 KB) and every workgroup resident at once, at most
-// 3.2 per CU.  Float32 us per call, 64 x 64 tiles / 32 x 32, with 1 workgroup
-// per CU at K = 512: 512^2 27.3 / 20.6, past it 640^2 29.5 / 37.8; 2 at K =
-// 256: 1024 x 512 27.2 / 20.4, past them 768^2 28.0 / 23.3 but Int32 with odd
-// extents no faster; K = 128: 768 x 1024 23.2 / 19.9, 1024^2 23.3 / 21.3
-// (Int32 equal); K = 64: 512^2 18.9 / 16.2, 1024^2 equal, 1500 x 1000 20.8 /
-// 21.4.
+// in LDS: K up to 512 (132 KB), on at most 3.2 workgroups per CU, fewer as K
+// grows past 160 (2 at 256, 1 at 512). A CU holds one workgroup at K > 256, two
+// at K > 128 and at least four below, so between those sizes up to two rounds
+// run; they are faster than 64 x 64 tiles all the same. Float32 and Int32 us
+// per call, 64 x 64 tiles / 32 x 32: 512^2 x 512 (1 per CU) 27.3 / 20.6, past
+// the line 640^2 x 512 29.5 / 37.8; 640^2 x 260 (1.6 per CU, one resident) 28.8
+// / 24.3, 28.7 / 25.2; batches of 32^2, K = 260, 504 of them 41.6 / 25.1, 50.6
+// / 26.2; 300 of K = 384 46.6 / 26.1, 59.1 / 27.4; 800 x 1000 x 160 (3.1 per
+// CU, two resident) 26.2 / 23.9, 26.3 / 25.7; 1024 x 512 x 256 27.2 / 20.4,
+// past it 768^2 28.0 / 23.3 but Int32 with odd extents no faster; K = 128: 768
+// x 1024 23.2 / 19.9, 1024^2 23.3 / 21.3 (Int32 equal); K = 64: 512^2 18.9 /
+// 16.2, 1024^2 equal, 1500 x 1000 20.8 / 21.4.
 inline bool resident_gemm(int64_t tiles32, int64_t K, int num_cus) {
   return K <= 512 && tiles32 * std::max<int64_t>(K, 160) <= (int64_t)num_cus * 512;
 }
