@@ -163,9 +163,9 @@ int step_shape(const PlanOptions& opt, int na, int nb, int nk, int nt) {
   const int shape = gemm_shape((int64_t)1 << na, (int64_t)1 << nb, opt.gemm_tiles);
   // (extents the kernel's 32-bit offsets hold)
   if (opt.lean || opt.gemm_tiles <= 0 || na < 6 || nb < 6 || nk < 4 || na > 24 || nk > 24) return shape;
-  const int tiles = std::max(0, na - __builtin_ctz(gemm_bm(shape))) +
-                    std::max(0, nb - __builtin_ctz(gemm_bn(shape))) + nt;
-  return tiles < 8 ? kGemm64 : shape;
+  const int log2_tiles = std::max(0, na - __builtin_ctz(gemm_bm(shape))) +
+                         std::max(0, nb - __builtin_ctz(gemm_bn(shape))) + nt;
+  return log2_tiles < 8 ? kGemm64 : shape;
 }
 
 struct Builder {
@@ -819,7 +819,7 @@ struct UnitBuilder {
   const std::vector<int32_t>& order;  // ... and its inverse
   SlicePlan& P;
   int32_t nl;
-  // log2 of a unit's MACs at most: 8 waves take about 3 us for 2^17
+  // a unit's MACs at most: 8 waves take about 3 us for 2^17
   static constexpr double kUnitMacs = 131072.0;
   // (items are indexed by 16 bits: one per node, and one more per 64 MACs)
   static constexpr int32_t kUnitNodes = 0x7fff;
@@ -1176,8 +1176,9 @@ struct UnitBuilder {
   }
 };
 
-// Every LDS and memory address a unit forms is in range, and its items cover
-// every output of every step.
+// Every LDS and memory address a unit forms is in range, and its items cover its
+// output.  (That steps read what earlier levels wrote, and write where nothing
+// of their level is read, is replayed by tests/host/unit_replay.cpp.)
 int verify_units(const SlicePlan& P, std::string* err) {
   auto bad = [&](const std::string& m) { return fail(err, "plan check: unit " + m); };
   for (const PUnit& u : P.units) {
