@@ -219,15 +219,21 @@ __global__ __launch_bounds__(64 * kUnitWaves) void tbh_unit_kernel(
 hipError_t launch_units(int dtype, const UnitDesc* units, const UnitItem* items,
                         const uint32_t* weights, const UnitExt* ext, int64_t n, void* results,
                         hipStream_t s) {
-  if (n <= 0) return hipSuccess;
   const uint4* it = reinterpret_cast<const uint4*>(items);
-  if (dtype == 0)
-    tbh_unit_kernel<float><<<(int)n, 64 * kUnitWaves, 0, s>>>(units, it, weights, ext,
-                                                              static_cast<float*>(results));
-  else
-    tbh_unit_kernel<int32_t><<<(int)n, 64 * kUnitWaves, 0, s>>>(units, it, weights, ext,
-                                                                static_cast<int32_t*>(results));
-  return hipGetLastError();
+  // a launch holds at most 2^32 - 1 work-items
+  constexpr int64_t kMost = ((int64_t)1 << 32) / (64 * kUnitWaves) - 1;
+  for (int64_t i = 0; i < n; i += kMost) {
+    const int blocks = (int)(n - i < kMost ? n - i : kMost);
+    if (dtype == 0)
+      tbh_unit_kernel<float><<<blocks, 64 * kUnitWaves, 0, s>>>(units + i, it, weights, ext,
+                                                                static_cast<float*>(results));
+    else
+      tbh_unit_kernel<int32_t><<<blocks, 64 * kUnitWaves, 0, s>>>(
+          units + i, it, weights, ext, static_cast<int32_t*>(results));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace tbh
