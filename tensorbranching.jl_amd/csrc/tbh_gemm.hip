@@ -570,4 +570,12 @@ hipError_t launch_gemm64(int dtype, const GemmDesc* ops, const int64_t* prefix, 
   return hipGetLastError();
 }
 
+int gemm64_blocks_per_cu(int dtype) {
+  int n = 0;
+  const void* k = dtype == 0 ? (const void*)tbh_gemm64_kernel<float>
+                             : (const void*)tbh_gemm64_kernel<int32_t>;
+  const hipError_t err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 256, 0);
+  return err == hipSuccess && n > 0 ? n : 2;
+}
+
 }  // namespace tbh

@@ -1507,6 +1507,7 @@ hipError_t launch_ew_direct(int dtype, const EwDesc* ops, const int64_t* prefix,
 
 hipError_t launch_gemm64(int dtype, const GemmDesc* ops, const int64_t* prefix, int nops,
                          int64_t total, int grid, hipStream_t s);  // tbh_gemm.hip
+int gemm64_blocks_per_cu(int dtype);                               // tbh_gemm.hip
 
 // The scalar-load kernel (a standalone product of M or K below 4, or of more
 // tiles than K1b has workgroups in a launch) has 128 x 128 tiles only.
@@ -1528,7 +1529,7 @@ hipError_t launch_gemm(int dtype, bool vec, int shape, const GemmDesc* ops, cons
 }
 
 int gemm_blocks_per_cu(int dtype, bool vec, int shape) {
-  if (shape == kGemm64) return 3;  // 155 VGPRs, 33 KB of LDS
+  if (shape == kGemm64) return gemm64_blocks_per_cu(dtype);
   int n = 0;
   const void* k = dtype == 0 ? gemm_kernel<float>(vec, shape) : gemm_kernel<int32_t>(vec, shape);
   const hipError_t err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 256, 0);
