@@ -105,9 +105,10 @@ __device__ __forceinline__ float of_key<float>(int32_t k) {
 constexpr int kAlphaLdsBits = 12;    // boundary bits kept in LDS
 constexpr int kAlphaRun = 1 << 12;   // configurations of one workgroup
 
-__global__ __launch_bounds__(256) void tbh_alpha_fill_kernel(int32_t* __restrict__ keys,
+__global__ __launch_bounds__(256) void tbh_alpha_fill_kernel(int64_t block0,
+                                                              int32_t* __restrict__ keys,
                                                               int64_t total) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t g = (block0 + blockIdx.x) * blockDim.x + threadIdx.x;
   if (g < total) keys[g] = kNoKey;
 }
 
@@ -115,12 +116,14 @@ __global__ __launch_bounds__(256) void tbh_alpha_fill_kernel(int32_t* __restrict
 // region), in ascending vertex order of their weights' sum, as in
 // tbh_configs_kernel.
 template <typename T>
-__global__ __launch_bounds__(256) void tbh_alpha_kernel(const RegionDesc* __restrict__ R,
+__global__ __launch_bounds__(256) void tbh_alpha_kernel(int64_t block0,
+                                                        const RegionDesc* __restrict__ R,
                                                         const int64_t* __restrict__ bprefix,
                                                         int n, int32_t* __restrict__ keys) {
   __shared__ int32_t best[1 << kAlphaLdsBits];
   __shared__ uint32_t adj[kRegionMaxNv], wb[kRegionMaxNv];
-  const int r = find_region(bprefix, n, blockIdx.x);
+  const int64_t block = block0 + blockIdx.x;
+  const int r = find_region(bprefix, n, block);
   const RegionDesc& d = R[r];
   const int tid = threadIdx.x;
   const uint32_t open = d.open, entries = 1u << d.nopen;
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(256) void tbh_alpha_kernel(const RegionDesc* __rest
     for (uint32_t k = tid; k < entries; k += 256) best[k] = kNoKey;
   __syncthreads();
   const uint32_t total = 1u << d.nv;
-  const uint32_t x0 = (uint32_t)(blockIdx.x - bprefix[r]) * kAlphaRun;
+  const uint32_t x0 = (uint32_t)(block - bprefix[r]) * kAlphaRun;
   const uint32_t x1 = x0 + kAlphaRun < total ? x0 + kAlphaRun : total;
   for (uint32_t x = x0 + tid; x < x1; x += 256) {
     T w = (T)0;
@@ -158,21 +161,23 @@ __global__ __launch_bounds__(256) void tbh_alpha_kernel(const RegionDesc* __rest
 
 // the keys as values, in place; no configuration: the tropical zero
 template <typename T>
-__global__ __launch_bounds__(256) void tbh_alpha_value_kernel(int32_t* __restrict__ keys,
+__global__ __launch_bounds__(256) void tbh_alpha_value_kernel(int64_t block0,
+                                                              int32_t* __restrict__ keys,
                                                               int64_t total) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t g = (block0 + blockIdx.x) * blockDim.x + threadIdx.x;
   if (g >= total) return;
   const int32_t k = keys[g];
   reinterpret_cast<T*>(keys)[g] = k == kNoKey ? tzero<T>() : of_key<T>(k);
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void tbh_compactify_kernel(const RegionDesc* __restrict__ R,
+__global__ __launch_bounds__(256) void tbh_compactify_kernel(int64_t block0,
+                                                              const RegionDesc* __restrict__ R,
                                                               const int64_t* __restrict__ aprefix,
                                                               int n, int64_t total,
                                                               const T* __restrict__ in,
                                                               T* __restrict__ out) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t g = (block0 + blockIdx.x) * blockDim.x + threadIdx.x;
   if (g >= total) return;
   const int r = find_region(aprefix, n, g);
   const int64_t base = aprefix[r];
@@ -193,14 +198,15 @@ __global__ __launch_bounds__(256) void tbh_compactify_kernel(const RegionDesc* _
 // PASS 0: counts[alpha entry] += 1 per matching configuration; PASS 1: writes
 // x at slot[entry]++ within the entry's group (group offsets in `offs`).
 template <typename T, int PASS>
-__global__ __launch_bounds__(256) void tbh_configs_kernel(const RegionDesc* __restrict__ R,
+__global__ __launch_bounds__(256) void tbh_configs_kernel(int64_t block0,
+                                                           const RegionDesc* __restrict__ R,
                                                            const int64_t* __restrict__ xprefix,
                                                            int n, int64_t total,
                                                            const T* __restrict__ alpha,
                                                            uint32_t* __restrict__ counts,
                                                            const int64_t* __restrict__ offs,
                                                            uint32_t* __restrict__ configs) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t g = (block0 + blockIdx.x) * blockDim.x + threadIdx.x;
   if (g >= total) return;
   const int r = find_region(xprefix, n, g);
   const RegionDesc& d = R[r];
@@ -222,6 +228,55 @@ __global__ __launch_bounds__(256) void tbh_configs_kernel(const RegionDesc* __re
     const uint32_t slot = atomicAdd(&counts[e], 1u);
     configs[offs[e] + slot] = x;
   }
+}
+
+// launch(block0, blocks) for runs of workgroups of 256 that a launch can hold:
+// from 2^32 work-items on their number wraps, without an error.
+template <class F>
+hipError_t in_runs(int64_t blocks, F launch) {
+  constexpr int64_t kMost = ((int64_t)1 << 24) - 1;
+  for (int64_t b = 0; b < blocks; b += kMost) {
+    launch(b, (int)std::min(blocks - b, kMost));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+template <typename T>
+hipError_t launch_alpha(const RegionDesc* R, const int64_t* bprefix, int n, int64_t blocks,
+                        int32_t* keys, int64_t total, hipStream_t s) {
+  const int64_t ga = (total + 255) / 256;
+  hipError_t e = in_runs(ga, [&](int64_t b, int grid) {
+    tbh_alpha_fill_kernel<<<grid, 256, 0, s>>>(b, keys, total);
+  });
+  if (e == hipSuccess)
+    e = in_runs(blocks, [&](int64_t b, int grid) {
+      tbh_alpha_kernel<T><<<grid, 256, 0, s>>>(b, R, bprefix, n, keys);
+    });
+  if (e == hipSuccess)
+    e = in_runs(ga, [&](int64_t b, int grid) {
+      tbh_alpha_value_kernel<T><<<grid, 256, 0, s>>>(b, keys, total);
+    });
+  return e;
+}
+
+template <typename T>
+hipError_t launch_compactify(const RegionDesc* R, const int64_t* aprefix, int n, int64_t total,
+                             const void* in, void* out, hipStream_t s) {
+  return in_runs((total + 255) / 256, [&](int64_t b, int grid) {
+    tbh_compactify_kernel<T><<<grid, 256, 0, s>>>(b, R, aprefix, n, total, (const T*)in, (T*)out);
+  });
+}
+
+template <typename T, int PASS>
+hipError_t launch_configs(const RegionDesc* R, const int64_t* xprefix, int n, int64_t total,
+                          const void* alpha, uint32_t* counts, const int64_t* offs,
+                          uint32_t* configs, hipStream_t s) {
+  return in_runs((total + 255) / 256, [&](int64_t b, int grid) {
+    tbh_configs_kernel<T, PASS><<<grid, 256, 0, s>>>(b, R, xprefix, n, total, (const T*)alpha,
+                                                     counts, offs, configs);
+  });
 }
 
 }  // namespace
@@ -367,7 +422,6 @@ extern "C" int tbh_region_alpha(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region*
   char* dev = ctx->base + doff;
   int32_t* keys = (int32_t*)(dev + o_key);
   hipStream_t s = ctx->stream;
-  const int ga = (int)((A + 255) / 256);
   const RegionDesc* dR = (const RegionDesc*)dev;
   const int64_t* dbp = (const int64_t*)(dev + o_bp);
   hipError_t e = hipSetDevice(ctx->device);
@@ -375,17 +429,9 @@ extern "C" int tbh_region_alpha(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region*
     e = hipMemcpyAsync(dev, desc.data(), n * sizeof(RegionDesc), hipMemcpyHostToDevice, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(dev + o_bp, bprefix.data(), (n + 1) * 8, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) {
-    tbh_alpha_fill_kernel<<<ga, 256, 0, s>>>(keys, A);
-    if (dtype == TBH_F32) {
-      tbh_alpha_kernel<float><<<(int)bprefix[n], 256, 0, s>>>(dR, dbp, (int)n, keys);
-      tbh_alpha_value_kernel<float><<<ga, 256, 0, s>>>(keys, A);
-    } else {
-      tbh_alpha_kernel<int32_t><<<(int)bprefix[n], 256, 0, s>>>(dR, dbp, (int)n, keys);
-      tbh_alpha_value_kernel<int32_t><<<ga, 256, 0, s>>>(keys, A);
-    }
-    e = hipGetLastError();
-  }
+  if (e == hipSuccess)
+    e = dtype == TBH_F32 ? launch_alpha<float>(dR, dbp, (int)n, bprefix[n], keys, A, s)
+                         : launch_alpha<int32_t>(dR, dbp, (int)n, bprefix[n], keys, A, s);
   if (e == hipSuccess) e = hipMemcpyAsync(alpha, keys, 4 * A, hipMemcpyDeviceToHost, s);
   const hipError_t es = hipStreamSynchronize(s);
   ctx->pool.free(doff);
@@ -465,30 +511,18 @@ extern "C" int tbh_region_tables(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region
   const int64_t* dap = (const int64_t*)(dev + o_ap);
   uint32_t* dcnt = (uint32_t*)(dev + o_cnt);
   const int64_t* doffs = (const int64_t*)(dev + o_offs);
-  const int ga = (int)((A + G - 1) / G);
-  const int64_t gx64 = (X + G - 1) / G;
-  if (gx64 > INT32_MAX) {
+  if ((X + G - 1) / G > INT32_MAX) {
     set_error("region tables: too many configurations in one call");
     return done(TBH_EINVAL);
   }
-  const int gx = (int)gx64;
-  if (dtype == TBH_F32) {
-    tbh_compactify_kernel<float><<<ga, G, 0, s>>>(dR, dap, (int)n, A, (const float*)(dev + o_in),
-                                                  (float*)(dev + o_out));
-    if ((e = hipGetLastError()) != hipSuccess) return fail(e, "compactify");
-    tbh_configs_kernel<float, 0><<<gx, G, 0, s>>>(dR, dxp, (int)n, X,
-                                                  (const float*)(dev + o_out), dcnt, doffs,
-                                                  nullptr);
-  } else {
-    tbh_compactify_kernel<int32_t><<<ga, G, 0, s>>>(dR, dap, (int)n, A,
-                                                    (const int32_t*)(dev + o_in),
-                                                    (int32_t*)(dev + o_out));
-    if ((e = hipGetLastError()) != hipSuccess) return fail(e, "compactify");
-    tbh_configs_kernel<int32_t, 0><<<gx, G, 0, s>>>(dR, dxp, (int)n, X,
-                                                    (const int32_t*)(dev + o_out), dcnt, doffs,
-                                                    nullptr);
-  }
-  if ((e = hipGetLastError()) != hipSuccess) return fail(e, "count");
+  const char* dalpha = dev + o_out;
+  e = dtype == TBH_F32 ? launch_compactify<float>(dR, dap, (int)n, A, dev + o_in, dev + o_out, s)
+                       : launch_compactify<int32_t>(dR, dap, (int)n, A, dev + o_in, dev + o_out, s);
+  if (e != hipSuccess) return fail(e, "compactify");
+  e = dtype == TBH_F32
+          ? launch_configs<float, 0>(dR, dxp, (int)n, X, dalpha, dcnt, doffs, nullptr, s)
+          : launch_configs<int32_t, 0>(dR, dxp, (int)n, X, dalpha, dcnt, doffs, nullptr, s);
+  if (e != hipSuccess) return fail(e, "count");
   if ((e = hipMemcpyAsync(alpha, dev + o_out, 4 * A, hipMemcpyDeviceToHost, s)) != hipSuccess ||
       (e = hipMemcpyAsync(cnt.data(), dcnt, 4 * A, hipMemcpyDeviceToHost, s)) != hipSuccess ||
       (e = hipStreamSynchronize(s)) != hipSuccess)
@@ -516,15 +550,10 @@ extern "C" int tbh_region_tables(tbh_ctx* ctx, tbh_dtype dtype, const tbh_region
             hipSuccess ||
         (e = hipMemsetAsync(dcnt, 0, 4 * A, s)) != hipSuccess)
       return fail(e, "offsets");
-    if (dtype == TBH_F32)
-      tbh_configs_kernel<float, 1><<<gx, G, 0, s>>>(dR, dxp, (int)n, X,
-                                                    (const float*)(dev + o_out), dcnt, doffs,
-                                                    dcfg);
-    else
-      tbh_configs_kernel<int32_t, 1><<<gx, G, 0, s>>>(dR, dxp, (int)n, X,
-                                                      (const int32_t*)(dev + o_out), dcnt, doffs,
-                                                      dcfg);
-    if ((e = hipGetLastError()) != hipSuccess) return fail(e, "write");
+    e = dtype == TBH_F32
+            ? launch_configs<float, 1>(dR, dxp, (int)n, X, dalpha, dcnt, doffs, dcfg, s)
+            : launch_configs<int32_t, 1>(dR, dxp, (int)n, X, dalpha, dcnt, doffs, dcfg, s);
+    if (e != hipSuccess) return fail(e, "write");
     if ((e = hipMemcpyAsync(configs, dcfg, (size_t)T * 4, hipMemcpyDeviceToHost, s)) !=
             hipSuccess ||
         (e = hipStreamSynchronize(s)) != hipSuccess)
