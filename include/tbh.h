@@ -99,8 +99,8 @@ int tbh_contract_slices(tbh_ctx* ctx, tbh_dtype dtype, const tbh_slice* slices,
  * nothing: each slice's arena and step descriptors live in a static device
  * array of TBH_NOALLOC_SCRATCH_BYTES (64 MiB) that every GPU the library runs
  * on holds until the process ends; the context's pool is not touched.  A
- * slice needing more than the array fails the call with TBH_ENOMEM before
- * any work.  All calls on one GPU share its array, so the
+ * slice needing more than the array, also when planned for less memory, fails
+ * the call with TBH_ENOMEM before any work.  All calls on one GPU share its array, so the
  * library runs them one at a time (a per-GPU lock; unserialized they would
  * race on it); results equal tbh_contract_slices(..., TBH_PLAIN) bit for
  * bit. */
@@ -143,7 +143,8 @@ int tbh_peak_memory(const tbh_slice* slice, double* log2_elems);
 int tbh_all_memory(const tbh_slice* slice, double* log2_elems);
 
 /* Device bytes the BATCHED executor reserves for this slice (its arena, the
- * admission footprint used by the pool and the serving scheduler). */
+ * admission footprint used by the pool and the serving scheduler).  A slice
+ * whose arena does not fit is planned again for less memory. */
 int tbh_slice_footprint(const tbh_slice* slice, tbh_dtype dtype,
                         size_t* bytes);
 
@@ -167,9 +168,9 @@ typedef enum {
 } tbh_status;
 
 /* Start the planner and scheduler threads.  A request is refused alone
- * (FAILED) when one of its slices' arenas (tbh_slice_footprint) exceeds the
- * region an idle pool gives a batched run, or its descriptors the pool's
- * share for them.  The scheduler runs rounds: a round admits slices --
+ * (FAILED) when one of its slices' arenas exceeds the region an idle pool
+ * gives a batched run, or its descriptors the pool's share for them, as
+ * planned by default (tbh_slice_footprint) and for less memory.  The scheduler runs rounds: a round admits slices --
  * latency-lane requests first, then arrival order -- while their summed
  * arenas fit that region, their descriptors that share, their summed
  * estimated work (the MACs of the slices' trees) stays within
@@ -278,8 +279,9 @@ int tbh_plan_steps(const tbh_slice* slice, tbh_dtype dtype, tbh_mode mode,
  * tiles per node, K parts >= 2^split_min_k_bits); ew_chunk / direct_chunk:
  * tiles per claim of the tiled / direct EW kernels, at most (a tiled claim
  * above 4 is halved, down to 4, on launches with too few tiles to give every
- * workgroup of the grid such a claim, and either claim is shortened further
- * until every resident workgroup has one); ew_per_cu: tiled EW
+ * workgroup of the grid such a claim; both are shortened further, a tiled one
+ * until every resident workgroup has two, a direct one until each of 16 waves
+ * per CU has one); ew_per_cu: tiled EW
  * workgroups per CU in a launch's grid (at most what is resident);
  * direct_max_reduce: EW steps reducing more labels than this run LDS-tiled,
  * not as direct wave tiles (-1: all tiled); concurrent: 1 runs a level's

@@ -370,8 +370,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
 // KMAX).  Bound by one pass through memory latency and the launch: every load
 // of a workgroup is in flight at once, by DMA without registers, where a slab
 // loop waits for each slab and a K range per workgroup needs a second launch.
-// Twice the LDS reads per MAC of the 64 x 64 tile, so only for products whose
-// tiles fit the chip at once.  The waves split K (8 of them at K <= 256, 16
+// Twice the LDS reads per MAC of the 64 x 64 tile, so only for products of few
+// tiles per CU (resident_gemm).  The waves split K (8 of them at K <= 256, 16
 // above: 512^3 21.0 with 8, 20.6 us; 1024 x 512 x 256 20.4, 22.9 with 16; 4 at
 // K <= 64).  Float32 us per call, 64 x 64 tiles / these: 64^3 18.5 / 15.8,
 // 64^2 x 512 25.2 / 19.7, 256^3 25.0 / 17.2, 512^3 27.3 / 20.6, 511 x 512 x
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(64 * WAVES) void tbh_gemm32_kernel(const GemmSplit 
 #endif
   __builtin_amdgcn_s_waitcnt(0);  // the DMA's writes (a barrier does not wait for them)
   __syncthreads();
-  // rows tx .. tx + 3, columns ty + 8 j; a quarter of K per wave
+  // rows tx .. tx + 3, columns ty + 8 j; an equal part of K per wave
   const int tx = (lane & 7) * 4, ty = lane >> 3;
   T acc[4][4];
 #pragma unroll

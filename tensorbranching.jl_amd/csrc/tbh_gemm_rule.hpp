@@ -8,7 +8,8 @@
 
 namespace tbh {
 
-// Workgroups of 256 in one launch: it holds at most 2^32 - 1 work-items.
+// Workgroups of 256 in one launch: it holds at most 2^32 - 1 work-items (more
+// wrap without an error).
 constexpr int64_t kGemmMaxBlocks = ((int64_t)1 << 24) - 1;
 
 // Whether K1 (128 x 128, 256 x 64 or 256 x 32 tiles; slabs of 16) takes a

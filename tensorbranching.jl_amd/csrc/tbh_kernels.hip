@@ -992,8 +992,10 @@ tbh_ew_pf_kernel(const EwDesc* __restrict__ ops_g, const int64_t* __restrict__ p
 // held a word per lane (read from memory, a byte each, one after another),
 // and a whole tile has no bounds to check.  Float32, before / now: M = 32768,
 // N = 64, batch 16, K = 32 61.6 / 52.7 us, K = 64 82.8 / 76.3; N = 32, K = 64
-// 50.1 / 48.5; 2048^3, batch 8, 1795 / 1750; 1024 tiles of 128 x 128 at K = 64
-// (a last wave of a third of the slots) 46.6 / 48.8.
+// 50.1 / 48.5; 2048^3, batch 8, 1795 / 1750.  Whole calls, Float32 and Int32,
+// before / now: 1024 tiles of 128 x 128 at K = 64 57.9 / 57.7, 71.4 / 69.7, at K
+// = 256 138 / 135, 203 / 201; 4000^2 x 100 (cut tiles) 75.7 / 76.4, 103.3 /
+// 104.3; 18 shapes of M, N 2048 .. 8192 0.99 in the geometric mean.
 constexpr int BK = 16, BPAD = 4;
 
 template <typename T>

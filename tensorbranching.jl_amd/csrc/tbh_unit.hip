@@ -220,7 +220,7 @@ hipError_t launch_units(int dtype, const UnitDesc* units, const UnitItem* items,
                         const uint32_t* weights, const UnitExt* ext, int64_t n, void* results,
                         hipStream_t s) {
   const uint4* it = reinterpret_cast<const uint4*>(items);
-  // a launch holds at most 2^32 - 1 work-items
+  // a launch holds at most 2^32 - 1 work-items (more wrap without an error)
   constexpr int64_t kMost = ((int64_t)1 << 32) / (64 * kUnitWaves) - 1;
   for (int64_t i = 0; i < n; i += kMost) {
     const int blocks = (int)(n - i < kMost ? n - i : kMost);
